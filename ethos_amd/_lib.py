@@ -50,6 +50,8 @@ SIGNATURES = {
     "ethos_expert_backward_workspace_bytes": (_sz, [_i64, _i32, _i32, _i32]),
     "ethos_expert_backward": (ctypes.c_int, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i32, _i32, _i32, _i32, _vp,
                                              _sz, _vp, _vp, _vp, _vp, _vp]),
+    "ethos_expert_grads_workspace_bytes": (_sz, [_i64, _i32, _i32, _i64, _i32, _i32, _i32]),
+    "ethos_expert_grads": (ctypes.c_int, [_vp] * 9 + [_i64] + [_vp] * 4 + [_i64] + [_i32] * 6 + [_vp, _sz] + [_vp] * 6),
     "ethos_expert_forward_workspace_bytes": (_sz, [_i64, _i32, _i32, _i64, _i32, _i32, _i32, _i32]),
     "ethos_expert_forward": (ctypes.c_int, [_vp, _vp, _i64, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _vp, _vp, _vp,
                                             _vp, _i64, _i32, _i32, _i32, _i32, _i32, _i32, _i32, _vp, _sz, _vp, _vp,

@@ -568,4 +568,47 @@ int ethos_expert_backward(const void* h, const float* xp, const float* dyb, cons
     return hip_status(rc, "ethos_expert_backward");
 }
 
+size_t ethos_expert_grads_workspace_bytes(int64_t n_tok, int32_t n_heads, int32_t top_k, int64_t max_unique,
+                                          int32_t d_latent, int32_t d_hidden, int32_t d_model) {
+    if (n_tok <= 0 || n_heads <= 0 || top_k <= 0 || max_unique <= 0 || d_latent <= 0 || d_hidden <= 0 || d_model <= 0) return 256;
+    return ethos::expert_grads_workspace_bytes(n_tok, n_heads, top_k, max_unique, d_latent, d_hidden, d_model, num_cus());
+}
+
+int ethos_expert_grads(const void* x, const void* dy, const void* h, const void* latents, const void* w1, const void* w2,
+                       const int32_t* uniq_ids, const int32_t* seg_off, const int32_t* n_unique, int64_t max_unique,
+                       const int32_t* perm, const int32_t* sorted_slot, const int32_t* pair_slot, const void* scores,
+                       int64_t n_tok, int32_t n_heads, int32_t top_k, int32_t d_latent, int32_t d_hidden, int32_t d_model,
+                       int32_t dtype, void* workspace, size_t workspace_bytes, void* dx, float* dscores, void* dlatents,
+                       void* dw1, void* dw2, void* stream) {
+    g_err[0] = 0;
+    if (!dtype_ok(dtype)) return fail(ETHOS_EDTYPE, "ethos_expert_grads: unknown dtype %d", dtype);
+    if (n_tok < 0 || n_heads <= 0 || top_k <= 0 || max_unique < 0 || d_latent <= 0 || d_hidden <= 0 || d_model <= 0)
+        return fail(ETHOS_ESIZE, "ethos_expert_grads: bad sizes");
+    const int vec = dtype == ETHOS_BF16 ? 8 : 4;
+    if (d_latent % 8 || d_hidden % 8 || d_model % 8 || ethos::apply_chunks(d_hidden, dtype) > 8)
+        return fail(ETHOS_EUNSUPPORTED,
+                    "ethos_expert_grads: d_latent=%d, d_hidden=%d and d_model=%d must be multiples of 8, d_hidden <= %d",
+                    d_latent, d_hidden, d_model, 8 * 64 * vec);
+    if (n_tok > INT32_MAX || n_tok * n_heads * top_k > INT32_MAX || max_unique > INT32_MAX)
+        return fail(ETHOS_ESIZE, "ethos_expert_grads: too many pairs");
+    if (n_tok == 0) return 0;
+    if (max_unique < 1) return fail(ETHOS_ESIZE, "ethos_expert_grads: max_unique must be >= 1 for a nonempty batch");
+    if (!x || !dy || !h || !latents || !w1 || !w2 || !uniq_ids || !seg_off || !n_unique || !perm || !sorted_slot || !pair_slot ||
+        !scores || !workspace || !dx || !dscores || !dlatents || !dw1 || !dw2)
+        return fail(ETHOS_ENULL, "ethos_expert_grads: null pointer");
+    const size_t need = ethos::expert_grads_workspace_bytes(n_tok, n_heads, top_k, max_unique, d_latent, d_hidden, d_model,
+                                                            num_cus());
+    if (workspace_bytes < need)
+        return fail(ETHOS_EWORKSPACE, "ethos_expert_grads: workspace of %zu bytes, %zu needed", workspace_bytes, need);
+    if (!aligned16(x) || !aligned16(dy) || !aligned16(h) || !aligned16(latents) || !aligned16(w1) || !aligned16(w2) ||
+        !aligned16(workspace))
+        return fail(ETHOS_EALIGN, "ethos_expert_grads: x, dy, h, latents, w1, w2 and workspace must be 16-byte aligned");
+    const int rc = ethos::launch_expert_grads(x, dy, h, latents, w1, w2, uniq_ids, seg_off, n_unique, max_unique, perm,
+                                              sorted_slot, pair_slot, scores, n_tok, n_heads, top_k, d_latent, d_hidden,
+                                              d_model, dtype, workspace, dx, dscores, dlatents, dw1, dw2, num_cus(),
+                                              (hipStream_t)stream);
+    if (rc < 0) return fail(ETHOS_EUNSUPPORTED, "ethos_expert_grads: d_hidden=%d not supported", d_hidden);
+    return hip_status(rc, "ethos_expert_grads");
+}
+
 }  // extern "C"

@@ -13,29 +13,28 @@
 //   dh_s  += a_p dYB_t + dc_p xp_t                                          (expert sums)
 //
 // Three kernels, all deterministic (every sum has a fixed order, no atomics):
-//  1. expert_bwd_pairs_kernel: one wave per token walks its H k pairs (kBwdUnroll hidden
+//  1. expert_bwd_pairs_kernel: one wave per token walks its H k pairs (bwd_unroll hidden
 //     rows in flight), keeps xp_t, dYB_t and the token sums in registers, and stores each
 //     pair's scalars (a_p, dc_p);
 //  2. expert_bwd_sums_kernel: the expert sums over the sorted pairs (ethos_sort_segment's
-//     permutation, each expert's pairs consecutive and in pair order), one wave per block
-//     of kBwdBlock sorted positions, summing each segment's terms in sorted order: a
+//     permutation, each expert's pairs consecutive and in pair order), a quarter wave per
+//     block of kBwdBlock sorted positions and 64 columns, summing each segment's terms in sorted order: a
 //     segment that lies in one block is written to dh; a segment crossing blocks leaves
 //     its part in its first block (tail) and in each later block (head) as partial rows;
 //  3. expert_bwd_join_kernel: each crossing segment's dh = its first block's tail part plus
 //     the later blocks' head parts, in block order.
-// The weight, input and latent gradients that follow are GEMMs.
+// launch_expert_grads runs the whole node: xp and dYB first, then these kernels, then the
+// weight, input and latent gradients as float32 matrix products (gemm.hip).
 #include "ethos_common.hpp"
+#include "ethos_gelu.hpp"
+#include "ethos_gemm.hpp"
 #include "ethos_launch.hpp"
 #include "ethos_rows.hpp"
 
 namespace ethos {
 
-constexpr int kBwdUnroll = 8;
-
-__device__ __forceinline__ float gelu_erf_grad(float x) {
-    // Phi(x) + x phi(x)
-    return 0.5f * erfcf(-x * 0.70710678118654752f) + x * expf(-0.5f * x * x) * 0.39894228040143268f;
-}
+// Hidden rows in flight per wave: fewer for rows of many registers.
+constexpr int bwd_unroll(int ch) { return ch <= 2 ? 8 : ch == 4 ? 4 : 2; }
 
 constexpr int kBwdBlock = 64;  // sorted positions per block of the expert-sum pass
 
@@ -48,6 +47,7 @@ __global__ __launch_bounds__(256) void expert_bwd_pairs_kernel(const T* __restri
                                                                float* __restrict__ hacc, float* __restrict__ dxp,
                                                                float2* __restrict__ ac) {
     constexpr int N = Vec16<T>::kN;
+    constexpr int kBwdUnroll = bwd_unroll(CH);
     typedef typename Vec16<T>::raw Raw;
     const int lane = threadIdx.x & 63;
     const int64_t wave_id = (int64_t)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -76,9 +76,14 @@ __global__ __launch_bounds__(256) void expert_bwd_pairs_kernel(const T* __restri
             for (int q = 0; q < kBwdUnroll; ++q) sq[q] = pair_slot[pbase + (j0 + q < hk ? j0 + q : hk - 1)];
 #pragma unroll
             for (int q = 0; q < kBwdUnroll; ++q) load_raw_buf<T, CH>(hid + (int64_t)sq[q] * dh, dh, lane, hr[q]);
+            // lane q's pair: its gate, then its two dot products, so that the GELU and its derivative
+            // are evaluated once for the group (for every pair by every lane they took 100 us at
+            // 524,288 pairs)
+            const int mine = j0 + lane < hk ? j0 + lane : hk - 1;
+            const float g = Elem<T>::to_f32(gates[pbase + mine]);
+            float my_c = 0.0f, my_d = 0.0f;
 #pragma unroll
             for (int q = 0; q < kBwdUnroll; ++q) {
-                if (j0 + q >= hk) continue;
                 float hf[CH * N];
                 float cp = 0.0f, dp = 0.0f;
 #pragma unroll
@@ -90,19 +95,26 @@ __global__ __launch_bounds__(256) void expert_bwd_pairs_kernel(const T* __restri
                         dp = __builtin_fmaf(hf[c * N + v], yr[c * N + v], dp);
                     }
                 }
-                const float cdot = wave_sum(cp);
-                const float da = wave_sum(dp);
-                const int64_t p = pbase + j0 + q;
-                const float g = Elem<T>::to_f32(gates[p]);
-                const float act = gelu_erf(cdot);
-                const float a = act * g;
-                const float dc = g * gelu_erf_grad(cdot) * da;
-                if (lane == 0) {
-                    dg[p] = act * da;
-                    ac[p] = make_float2(a, dc);
-                }
+                const float cdot = wave_sum(cp), da = wave_sum(dp);
+                my_c = lane == q ? cdot : my_c;
+                my_d = lane == q ? da : my_d;
+            }
+            const float act = gelu_erf(my_c);
+            const float my_a = act * g;
+            const float my_dc = g * gelu_erf_grad(my_c) * my_d;
+            if (lane < kBwdUnroll && j0 + lane < hk) {
+                dg[pbase + mine] = act * my_d;
+                ac[pbase + mine] = make_float2(my_a, my_dc);
+            }
+#pragma unroll
+            for (int q = 0; q < kBwdUnroll; ++q) {
+                if (j0 + q >= hk) continue;
+                const float a = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(my_a), q));
+                const float dc = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(my_dc), q));
+                float hf[CH * N];
 #pragma unroll
                 for (int c = 0; c < CH; ++c) {
+                    Vec16<T>::unpack(hr[q][c], hf + c * N);
 #pragma unroll
                     for (int v = 0; v < N; ++v) {
                         ha[c * N + v] = __builtin_fmaf(a, hf[c * N + v], ha[c * N + v]);
@@ -125,14 +137,73 @@ __global__ __launch_bounds__(256) void expert_bwd_pairs_kernel(const T* __restri
     }
 }
 
-// Expert sums, one wave per block of kBwdBlock sorted positions: lane l holds columns
-// 64 j + l (j < NB) of the running sum of the segment being walked, the positions are
-// taken one at a time in sorted order (their pair, token and scalars loaded a lane each
-// and broadcast), and a segment's sum is stored when the walk leaves it: to dh when the
-// segment lies in the block, else as the block's head part (the segment that began
-// before the block) or tail part (the segment that begins in the block and continues
-// past it).
-template <int NB>
+// Expert sums.  A quarter wave (16 lanes, 4 columns each) takes one block of kBwdBlock sorted
+// positions for one slice of 64 columns, one position at a time in sorted order; 16 positions'
+// pairs, tokens and scalars are loaded a lane each and broadcast over the quarter (DPP), and
+// kSumUnroll positions' row pieces are requested together.  A segment's sum is stored when the
+// walk leaves it: to dh when the segment lies in the block, else as the block's head part (the
+// segment that began before the block) or tail part (the segment that begins in the block and
+// continues past it).
+// What bounds it is the row gathers, two of 4 d_hidden bytes per pair: 2.1 GB for 524,288 pairs
+// at d_hidden 512, out of two tables of 8 MB.  Workgroup b works on slice b % (slices), and runs
+// on XCD b % 8, so at 512 columns each XCD's gathers stay in 2 MB of the tables, inside its L2:
+// 278 us (one wave per block over all columns, 7.5 TB/s out of the memory-side cache) -> 173 us.
+// 16,000 pairs (500 tokens): 113 -> 18 us, a wave's 64 positions no longer one load after another.
+constexpr int kSumUnroll = 8;
+constexpr int kSumSlice = 64;
+
+// Lane i of each row of 16 to the whole row.
+template <int I>
+__device__ __forceinline__ int row_bcast(int v) {
+    return __builtin_amdgcn_update_dpp(0, v, 0x150 + I, 0xf, 0xf, false);
+}
+
+struct SumPos {  // a lane's position
+    int t, s, to;   // token, slot, and after this position: 0 go on, 1 store to dh, 2 to head, 3 to tail
+    float a, dc;
+};
+
+template <int I>
+struct SumStep {
+    // positions I .. I + kSumUnroll - 1 of the 16
+    __device__ __forceinline__ static void run(const SumPos& me, const float* __restrict__ xp, const float* __restrict__ dyb,
+                                               int dh, int col, bool in, float4& acc, float* __restrict__ dhs,
+                                               float* head, float* tail) {
+        float4 x[kSumUnroll], y[kSumUnroll];
+        load<0>(me, xp, dyb, dh, col, x, y);
+        add<0>(me, dh, col, in, acc, x, y, dhs, head, tail);
+    }
+    template <int U>
+    __device__ __forceinline__ static void load(const SumPos& me, const float* xp, const float* dyb, int dh, int col, float4* x,
+                                                float4* y) {
+        if constexpr (U < kSumUnroll) {
+            const int64_t at = (int64_t)row_bcast<I + U>(me.t) * dh + col;
+            y[U] = *reinterpret_cast<const float4*>(dyb + at);
+            x[U] = *reinterpret_cast<const float4*>(xp + at);
+            load<U + 1>(me, xp, dyb, dh, col, x, y);
+        }
+    }
+    template <int U>
+    __device__ __forceinline__ static void add(const SumPos& me, int dh, int col, bool in, float4& acc, const float4* x,
+                                               const float4* y, float* dhs, float* head, float* tail) {
+        if constexpr (U < kSumUnroll) {
+            const float a = __int_as_float(row_bcast<I + U>(__float_as_int(me.a)));
+            const float dc = __int_as_float(row_bcast<I + U>(__float_as_int(me.dc)));
+            const int to = row_bcast<I + U>(me.to), s = row_bcast<I + U>(me.s);
+            acc.x = __builtin_fmaf(dc, x[U].x, __builtin_fmaf(a, y[U].x, acc.x));
+            acc.y = __builtin_fmaf(dc, x[U].y, __builtin_fmaf(a, y[U].y, acc.y));
+            acc.z = __builtin_fmaf(dc, x[U].z, __builtin_fmaf(a, y[U].z, acc.z));
+            acc.w = __builtin_fmaf(dc, x[U].w, __builtin_fmaf(a, y[U].w, acc.w));
+            if (to != 0) {
+                float* dst = (to == 1 ? dhs + (int64_t)s * dh : to == 2 ? head : tail) + col;
+                if (in) *reinterpret_cast<float4*>(dst) = acc;
+                acc = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            }
+            add<U + 1>(me, dh, col, in, acc, x, y, dhs, head, tail);
+        }
+    }
+};
+
 __global__ __launch_bounds__(256) void expert_bwd_sums_kernel(const float* __restrict__ xp,
                                                               const float* __restrict__ dyb,
                                                               const int32_t* __restrict__ perm,
@@ -143,51 +214,33 @@ __global__ __launch_bounds__(256) void expert_bwd_sums_kernel(const float* __res
                                                               float* __restrict__ head, float* __restrict__ tail) {
     const int lane = threadIdx.x & 63;
     const int64_t n_blocks = (n_pairs + kBwdBlock - 1) / kBwdBlock;
-    const int64_t wave_id = (int64_t)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int64_t n_waves = (int64_t)gridDim.x * 4;
-    for (int64_t blk = wave_id; blk < n_blocks; blk += n_waves) {
-        const int64_t b0 = blk * kBwdBlock;
-        const int cnt = (int)min((int64_t)kBwdBlock, n_pairs - b0);
-        // this lane's position: pair, token, scalars, slot and segment bounds
-        int my_t = 0, my_s = 0;
-        float my_a = 0.0f, my_dc = 0.0f;
-        int64_t my_beg = 0, my_end = 0;
-        if (lane < cnt) {
-            const int p = perm[b0 + lane];
-            my_t = p / hk;
+    const int slices = (dh + kSumSlice - 1) / kSumSlice;
+    const int slice = blockIdx.x % slices;
+    const int col0 = slice * kSumSlice + 4 * (lane & 15);
+    const bool in = col0 < dh;
+    const int col = in ? col0 : 0;  // past the row: column 0, not stored
+    // this quarter wave's block of positions; quarters past the last one idle with no positions
+    const int64_t blk = ((int64_t)(blockIdx.x / slices) * 4 + (threadIdx.x >> 6)) * 4 + (lane >> 4);
+    const int64_t b0 = blk * kBwdBlock;
+    const int cnt = blk < n_blocks ? (int)min((int64_t)kBwdBlock, n_pairs - b0) : 0;
+    float4 acc = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    for (int c = 0; c < kBwdBlock; c += 16) {
+        // 16 positions, a lane each; past the block's end nothing is added or stored
+        const int i = c + (lane & 15);
+        SumPos me{0, 0, 0, 0.0f, 0.0f};
+        if (i < cnt) {
+            const int p = perm[b0 + i];
+            me.s = sorted_slot[b0 + i];
+            const int after = i + 1 < cnt ? sorted_slot[b0 + i + 1] : -1;
             const float2 v = ac[p];
-            my_a = v.x;
-            my_dc = v.y;
-            my_s = sorted_slot[b0 + lane];
-            my_beg = seg_off[my_s];
-            my_end = seg_off[my_s + 1];
+            me.t = p / hk;
+            me.a = v.x;
+            me.dc = v.y;
+            if (after != me.s)
+                me.to = seg_off[me.s] < b0 ? 2 : seg_off[me.s + 1] > b0 + kBwdBlock ? 3 : 1;
         }
-        float acc[NB];
-#pragma unroll
-        for (int j = 0; j < NB; ++j) acc[j] = 0.0f;
-        for (int i = 0; i < cnt; ++i) {
-            const int t = __shfl(my_t, i, 64);
-            const float a = __shfl(my_a, i, 64), dc = __shfl(my_dc, i, 64);
-            const float* yr = dyb + (int64_t)t * dh;
-            const float* xr = xp + (int64_t)t * dh;
-#pragma unroll
-            for (int j = 0; j < NB; ++j) {
-                const int e = 64 * j + lane;
-                if (e < dh) acc[j] = __builtin_fmaf(dc, xr[e], __builtin_fmaf(a, yr[e], acc[j]));
-            }
-            const int s = __shfl(my_s, i, 64);
-            const bool last = i + 1 == cnt || __shfl(my_s, i + 1, 64) != s;
-            if (last) {
-                const int64_t beg = (int64_t)__shfl((int)my_beg, i, 64), end = (int64_t)__shfl((int)my_end, i, 64);
-                float* dst = beg < b0 ? head + blk * dh : end > b0 + kBwdBlock ? tail + blk * dh : dhs + (int64_t)s * dh;
-#pragma unroll
-                for (int j = 0; j < NB; ++j) {
-                    const int e = 64 * j + lane;
-                    if (e < dh) dst[e] = acc[j];
-                    acc[j] = 0.0f;
-                }
-            }
-        }
+        SumStep<0>::run(me, xp, dyb, dh, col, in, acc, dhs, head + blk * dh, tail + blk * dh);
+        SumStep<8>::run(me, xp, dyb, dh, col, in, acc, dhs, head + blk * dh, tail + blk * dh);
     }
 }
 
@@ -249,17 +302,14 @@ static void launch_bwd_t(const void* hid, const float* xp, const float* dyb, con
 }
 
 template <int NB>
-static void launch_sums_t(const float* xp, const float* dyb, const int32_t* perm, const int32_t* sorted_slot,
-                          const int32_t* seg_off, const float2* ac, int64_t n_pairs, int hk, int dh, float* dhs,
-                          float* head, float* tail, int num_cus, hipStream_t stream) {
+static void launch_join_t(const int32_t* sorted_slot, const int32_t* seg_off, int64_t n_pairs, int dh, const float* head,
+                          const float* tail, float* dhs, int num_cus, hipStream_t stream) {
     const int64_t n_blocks = (n_pairs + kBwdBlock - 1) / kBwdBlock;
     int64_t g = (n_blocks + 3) / 4;
     const int64_t cap = (int64_t)num_cus * 16;
     g = g > cap ? cap : (g < 1 ? 1 : g);
-    hipLaunchKernelGGL((expert_bwd_sums_kernel<NB>), dim3((unsigned)g), dim3(256), 0, stream, xp, dyb, perm,
-                       sorted_slot, seg_off, ac, n_pairs, hk, dh, dhs, head, tail);
     hipLaunchKernelGGL((expert_bwd_join_kernel<NB>), dim3((unsigned)g), dim3(256), 0, stream, sorted_slot, seg_off,
-                       n_pairs, dh, (const float*)head, (const float*)tail, dhs);
+                       n_pairs, dh, head, tail, dhs);
 }
 
 int launch_expert_backward(const void* hid, const float* xp, const float* dyb, const int32_t* pair_slot,
@@ -291,17 +341,114 @@ int launch_expert_backward(const void* hid, const float* xp, const float* dyb, c
     }
 #undef ETHOS_BWD_CASE
     if (!done) return -1;
+    const int slices = (dh + kSumSlice - 1) / kSumSlice;
+    hipLaunchKernelGGL(expert_bwd_sums_kernel, dim3((unsigned)((n_blocks + 15) / 16 * slices)), dim3(256), 0, stream, xp, dyb,
+                       perm, sorted_slot, seg_off, (const float2*)ac, n_pairs, H * k, dh, dhs, head, tail);
     const int nb = (dh + 63) / 64;
 #define ETHOS_SUMS_CASE(NBC)                                                                                      \
     if (nb <= NBC) {                                                                                              \
-        launch_sums_t<NBC>(xp, dyb, perm, sorted_slot, seg_off, ac, n_pairs, H * k, dh, dhs, head, tail, num_cus, \
-                           stream);                                                                               \
+        launch_join_t<NBC>(sorted_slot, seg_off, n_pairs, dh, head, tail, dhs, num_cus, stream);                  \
         return (int)hipGetLastError();                                                                            \
     }
     ETHOS_SUMS_CASE(1) ETHOS_SUMS_CASE(2) ETHOS_SUMS_CASE(4) ETHOS_SUMS_CASE(8) ETHOS_SUMS_CASE(16)
     ETHOS_SUMS_CASE(32) ETHOS_SUMS_CASE(64)
 #undef ETHOS_SUMS_CASE
     return -1;
+}
+
+namespace {
+
+size_t pad256(size_t n) { return (n + 255) & ~(size_t)255; }
+
+// Offsets in expert_grads' workspace.
+struct GradsLayout {
+    size_t xp, dyb, hacc, dxp, dhs, pairs, part, total;
+    int split_w2, split_w1;
+};
+
+GradsLayout grads_layout(int64_t n_tok, int H, int k, int64_t max_u, int dl, int dh, int d, int num_cus) {
+    GradsLayout l{};
+    const size_t tok = pad256((size_t)n_tok * dh * sizeof(float));
+    l.xp = 0;
+    l.dyb = tok;
+    l.hacc = 2 * tok;
+    l.dxp = 3 * tok;
+    l.dhs = 4 * tok;
+    l.pairs = l.dhs + pad256((size_t)max_u * dh * sizeof(float));
+    l.part = l.pairs + pad256(expert_backward_workspace_bytes(n_tok * H * k, dh));
+    l.split_w2 = gemm_split(dh, d, n_tok, num_cus);
+    l.split_w1 = gemm_split(dh, dl, max_u, num_cus);
+    const size_t p2 = l.split_w2 > 1 ? (size_t)l.split_w2 * dh * d : 0, p1 = l.split_w1 > 1 ? (size_t)l.split_w1 * dh * dl : 0;
+    l.total = l.part + pad256((p1 > p2 ? p1 : p2) * sizeof(float));
+    return l;
+}
+
+}  // namespace
+
+size_t expert_grads_workspace_bytes(int64_t n_tok, int H, int k, int64_t max_u, int dl, int dh, int d, int num_cus) {
+    return grads_layout(n_tok, H, k, max_u, dl, dh, d, num_cus).total;
+}
+
+// The expert stages' backward.  Every matrix product keeps float32 sums and no less than
+// float32 operands (gemm.hip), and the number of unique experts stays on the device: the
+// products over the experts' rows read it there, so the host does not wait for the routing.
+// 4,096 tokens, 200,070 experts, bf16: about 4.0 ms as library float32 GEMMs with the GELU
+// derivative as a chain of elementwise passes over [U, d_hidden], 0.99 ms as here (dpre 200 us,
+// expert sums 173, d latents 158, d W1 130, pairs 95, d W2 83, the token products 105).
+int launch_expert_grads(const void* x, const void* dy, const void* hid, const void* latents, const void* w1, const void* w2,
+                        const int32_t* uniq, const int32_t* seg_off, const int32_t* n_unique, int64_t max_u,
+                        const int32_t* perm, const int32_t* sorted_slot, const int32_t* pair_slot, const void* gates,
+                        int64_t n_tok, int H, int k, int dl, int dh, int d, int dtype, void* ws, void* dx, float* dg,
+                        void* dlat, void* dw1, void* dw2, int num_cus, hipStream_t stream) {
+    const bool bf = dtype == kBF16;
+    const size_t size = bf ? 2 : 4;
+    const GradsLayout l = grads_layout(n_tok, H, k, max_u, dl, dh, d, num_cus);
+    unsigned char* w = static_cast<unsigned char*>(ws);
+    float *xp = (float*)(w + l.xp), *dyb = (float*)(w + l.dyb), *hacc = (float*)(w + l.hacc), *dxp = (float*)(w + l.dxp);
+    float *dhs = (float*)(w + l.dhs), *part = (float*)(w + l.part);
+    const void* w2v = (const unsigned char*)w2 + (size_t)d * dh * size;  // W_v^T
+    const float inv_h = 1.0f / (float)H;
+    int rc;
+
+    Gemm g;  // xp = x W_u
+    g.a = x, g.lda = d, g.b = w2, g.ldb = dh, g.c = xp, g.ldc = dh;
+    g.m = n_tok, g.n = dh, g.k = d;
+    if ((rc = launch_gemm(bf ? kGemmBK_BR : kGemmFK_FR, g, num_cus, stream))) return rc;
+    g.a = dy, g.b = w2v, g.c = dyb, g.alpha = inv_h;  // dYB = (dy / H) W_v^T
+    if ((rc = launch_gemm(bf ? kGemmBK_BR : kGemmFK_FR, g, num_cus, stream))) return rc;
+
+    rc = launch_expert_backward(hid, xp, dyb, pair_slot, perm, sorted_slot, seg_off, gates, n_tok, H, k, dh, dtype,
+                                w + l.pairs, dg, hacc, dxp, dhs, num_cus, stream);
+    if (rc) return rc;
+
+    g = Gemm{};  // d W_u^T = x^T dxp and d W_v^T = (dy / H)^T hacc, stored [d][d_hidden]
+    g.a = dxp, g.lda = dh, g.b = x, g.ldb = d, g.c = dw2, g.ldc = dh;
+    g.m = dh, g.n = d, g.k = n_tok;
+    g.transposed = true, g.out_bf16 = bf, g.split = l.split_w2, g.part = part;
+    if ((rc = launch_gemm(bf ? kGemmFR_BR : kGemmFR_FR, g, num_cus, stream))) return rc;
+    g.a = hacc, g.b = dy, g.c = (unsigned char*)dw2 + (size_t)d * dh * size, g.alpha = inv_h;
+    if ((rc = launch_gemm(bf ? kGemmFR_BR : kGemmFR_FR, g, num_cus, stream))) return rc;
+
+    g = Gemm{};  // dx = dxp W_u^T
+    g.a = dxp, g.lda = dh, g.b = w2, g.ldb = dh, g.c = dx, g.ldc = d;
+    g.m = n_tok, g.n = d, g.k = dh, g.out_bf16 = bf;
+    if ((rc = launch_gemm(bf ? kGemmFK_BK : kGemmFK_FK, g, num_cus, stream))) return rc;
+
+    g = Gemm{};  // dpre = gelu'(z W1) dh, in place of dh
+    g.a = latents, g.lda = dl, g.a_rows = uniq, g.b = w1, g.ldb = dl, g.c = dhs, g.ldc = dh;
+    g.m = max_u, g.n = dh, g.k = dl, g.dyn = n_unique, g.gelu_grad = true;
+    if ((rc = launch_gemm(bf ? kGemmBK_BK : kGemmFK_FK, g, num_cus, stream))) return rc;
+
+    g = Gemm{};  // d latents: dpre W1^T into the unique experts' rows
+    g.a = dhs, g.lda = dh, g.b = w1, g.ldb = dl, g.c = dlat, g.ldc = dl, g.c_rows = uniq;
+    g.m = max_u, g.n = dl, g.k = dh, g.dyn = n_unique, g.out_bf16 = bf;
+    if ((rc = launch_gemm(bf ? kGemmFK_BR : kGemmFK_FR, g, num_cus, stream))) return rc;
+
+    g = Gemm{};  // d W1 = dpre^T z
+    g.a = dhs, g.lda = dh, g.b = latents, g.ldb = dl, g.b_rows = uniq, g.c = dw1, g.ldc = dl;
+    g.m = dh, g.n = dl, g.k = max_u, g.dyn = n_unique, g.dyn_k = true, g.out_bf16 = bf;
+    g.split = l.split_w1, g.part = part;
+    return launch_gemm(bf ? kGemmFR_BR : kGemmFR_FR, g, num_cus, stream);
 }
 
 }  // namespace ethos

@@ -1,0 +1,51 @@
+// Matrix products of the training path with float32 results (gemm.hip).
+#pragma once
+
+#include <hip/hip_runtime.h>
+#include <stddef.h>
+#include <stdint.h>
+
+namespace ethos {
+
+// C[m][n] = alpha * sum_k A[m][k] B[k][n] (+ bias[n]), accumulated in float32.  Each operand
+// is float32 or bf16 and stored either with k contiguous ([m][k] / [n][k], "K") or with k as
+// the row ([k][m] / [k][n], "R").  Sizes: k-contiguous operands need k % 8 == 0 and 16-byte
+// aligned rows; row-wise bf16 operands an even column count and 4-byte aligned rows.
+struct Gemm {
+    const void* a = nullptr;
+    const void* b = nullptr;
+    void* c = nullptr;
+    const float* bias = nullptr;       // float32 [n] (not with split > 1)
+    const int32_t* a_rows = nullptr;   // K-stored A: row m of A is row a_rows[m] of `a`
+    const int32_t* b_rows = nullptr;   // R-stored B: row k of B is row b_rows[k] of `b`
+    const int32_t* c_rows = nullptr;   // row m of C is row c_rows[m] of `c`
+    const int32_t* dyn = nullptr;      // device count: m (or, dyn_k, k) is min(m, *dyn)
+    int64_t m = 0, k = 0;
+    int n = 0;
+    int64_t lda = 0, ldb = 0, ldc = 0;
+    float alpha = 1.0f;
+    bool dyn_k = false;
+    bool out_bf16 = false;             // C is bf16 (rounded to nearest even), else float32
+    bool transposed = false;           // C is stored [n][m], ldc its row length
+    bool gelu_grad = false;            // C[m][n] = gelu'(sum) * C[m][n] (float32, in place)
+    int split = 1;                     // reduction split over this many workgroups per tile:
+    float* part = nullptr;             // [split][m][n] (or [n][m]) float32 partial sums
+};
+
+enum GemmForm {
+    kGemmBK_BK,  // A bf16 K, B bf16 K
+    kGemmBK_BR,  // A bf16 K, B bf16 R
+    kGemmFK_BK,  // A float32 K, B bf16 K
+    kGemmFK_BR,  // A float32 K, B bf16 R
+    kGemmFR_BR,  // A float32 R, B bf16 R
+    kGemmFK_FK,  // float32 both
+    kGemmFK_FR,
+    kGemmFR_FR,
+};
+
+// Splits of a product of m x n outputs over k so that the chip has about two workgroups per
+// CU, each with at least 256 of the reduction.
+int gemm_split(int64_t m, int n, int64_t k, int num_cus);
+int launch_gemm(GemmForm form, const Gemm& g, int num_cus, hipStream_t stream);
+
+}  // namespace ethos

@@ -90,6 +90,13 @@ int launch_expert_backward(const void* hid, const float* xp, const float* dyb, c
                            const int32_t* perm, const int32_t* sorted_slot, const int32_t* seg_off, const void* gates,
                            int64_t n_tok, int H, int k, int dh, int dtype, void* ws, float* dg, float* hacc,
                            float* dxp, float* dhs, int num_cus, hipStream_t stream);
+// The whole expert node's backward (see backward.hip); dlat holds zeros on entry.
+size_t expert_grads_workspace_bytes(int64_t n_tok, int H, int k, int64_t max_u, int dl, int dh, int d, int num_cus);
+int launch_expert_grads(const void* x, const void* dy, const void* hid, const void* latents, const void* w1, const void* w2,
+                        const int32_t* uniq, const int32_t* seg_off, const int32_t* n_unique, int64_t max_u,
+                        const int32_t* perm, const int32_t* sorted_slot, const int32_t* pair_slot, const void* gates,
+                        int64_t n_tok, int H, int k, int dl, int dh, int d, int dtype, void* ws, void* dx, float* dg,
+                        void* dlat, void* dw1, void* dw2, int num_cus, hipStream_t stream);
 size_t apply_hidden_workspace_bytes(int64_t n_tok, int H, int k, int d, int dh, int dtype);
 int launch_apply_hidden(const void* x, const void* w2, const void* hid, const int32_t* perm,
                         const int32_t* sorted_slot, const int32_t* pair_slot, const void* gates, int64_t n_tok, int H,

@@ -398,3 +398,50 @@ def expert_backward(h: torch.Tensor, xp: torch.Tensor, dyb: torch.Tensor, seg: d
                                       _stream())
     check(rc, "ethos_expert_backward")
     return dg, hacc, dxp, dhs[:U]
+
+
+def expert_grads_supported(x: torch.Tensor, dy: torch.Tensor, h: torch.Tensor, latents: torch.Tensor, w1: torch.Tensor,
+                           w2: torch.Tensor) -> bool:
+    """Whether expert_grads takes these operands: one dtype, contiguous, 16-byte aligned, sizes
+    that are multiples of 8, d_hidden within the per-pair kernel's limit."""
+    ts = (x, dy, h, latents, w1, w2)
+    if any(t.dtype != x.dtype or not t.is_cuda or not t.is_contiguous() or t.data_ptr() % 16 for t in ts):
+        return False
+    d, dl, dh = x.shape[1], w1.shape[1], w1.shape[0]
+    return d % 8 == 0 and dl % 8 == 0 and dh % 8 == 0 and dh <= (4096 if x.dtype == torch.bfloat16 else 2048)
+
+
+def expert_grads(x: torch.Tensor, dy: torch.Tensor, h: torch.Tensor, latents: torch.Tensor, w1: torch.Tensor,
+                 w2: torch.Tensor, seg: dict, gates: torch.Tensor, n_heads: int, top_k: int):
+    """The expert stages' backward: (dx, dgates float32 [n, H, k], dlatents, dw1, dw2) from the
+    forward's hidden rows h and sorted segments `seg` (with uniq and n_unique, the count staying
+    on the device); deterministic."""
+    _need(x, "x", dim=2)
+    for name, t in (("dy", dy), ("h", h), ("latents", latents), ("w1", w1), ("w2", w2)):
+        _need(t, name, x.dtype, 2)
+    _need(gates, "gates", x.dtype)
+    for name in ("uniq", "n_unique", "pair_slot", "perm", "sorted_slot", "seg_off"):
+        _need(seg[name], name, torch.int32)
+    n, d = x.shape
+    dh, dl = w1.shape
+    max_u = seg["uniq"].numel()
+    if (dy.shape != x.shape or latents.shape[1] != dl or w2.shape != (2 * d, dh) or h.shape != (max_u, dh)
+            or gates.numel() != n * n_heads * top_k or seg["perm"].numel() != gates.numel()
+            or seg["pair_slot"].numel() != gates.numel() or seg["sorted_slot"].numel() != gates.numel()
+            or seg["seg_off"].numel() != max_u + 1):
+        raise RuntimeError("expert_grads: inconsistent shapes")
+    dev = x.device
+    dx = torch.empty_like(x)
+    dg = torch.empty(gates.shape, dtype=torch.float32, device=dev)
+    dlat = torch.zeros_like(latents)
+    dw1 = torch.empty_like(w1)
+    dw2 = torch.empty_like(w2)
+    ws, ws_bytes = workspace(load().ethos_expert_grads_workspace_bytes(n, n_heads, top_k, max_u, dl, dh, d), dev)
+    rc = load().ethos_expert_grads(x.data_ptr(), dy.data_ptr(), h.data_ptr(), latents.data_ptr(), w1.data_ptr(), w2.data_ptr(),
+                                   seg["uniq"].data_ptr(), seg["seg_off"].data_ptr(), seg["n_unique"].data_ptr(), max_u,
+                                   seg["perm"].data_ptr(), seg["sorted_slot"].data_ptr(), seg["pair_slot"].data_ptr(),
+                                   gates.data_ptr(), n, n_heads, top_k, dl, dh, d, dtype_code(x.dtype), ws.data_ptr(),
+                                   ws_bytes, dx.data_ptr(), dg.data_ptr(), dlat.data_ptr(), dw1.data_ptr(),
+                                   dw2.data_ptr(), _stream())
+    check(rc, "ethos_expert_grads")
+    return dx, dg, dlat, dw1, dw2

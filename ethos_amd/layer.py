@@ -78,11 +78,12 @@ class _ExpertStages(torch.autograd.Function):
     dc_p = g_p gelu'(c_p) da_p;  dxp_t = Σ_p dc_p h_s;  dh_s = Σ_p (dc_p xp_t + a_p dY_t B);
     dA = x^T dxp,  dB = dY^T hacc with hacc_t = Σ_p a_p h_s,  dx = dxp A^T;
     dpre = gelu'(pre) dh,  dC = dpre^T z,  dz = dpre C (added into the latent rows of the
-    unique experts).  v rows are not needed.  The per-pair terms, the token sums (hacc, dxp)
-    and the expert sums (dh, summed over each expert's sorted pairs in a fixed order) come
-    from one library call (ethos_expert_backward); the rest are GEMMs.  The backward is
-    deterministic.  Both execution orders (scatter of v rows, hidden-space reordering)
-    compute this same function, so they share the backward.
+    unique experts).  v rows are not needed.  One library call (ethos_expert_grads) computes
+    all of it; outside its limits the per-pair terms, the token sums (hacc, dxp) and the expert
+    sums (dh, summed over each expert's sorted pairs in a fixed order) come from
+    ethos_expert_backward and the rest are torch GEMMs.  The backward is deterministic.
+    Both execution orders (scatter of v rows, hidden-space reordering) compute this same
+    function, so they share the backward.
 
     The gates enter as `gates_exact` (the values the forward uses) and `gate_path` (a
     float32 tensor of the same values carrying the router's graph), whose gradient is dg.
@@ -103,9 +104,17 @@ class _ExpertStages(torch.autograd.Function):
         # v_s = h_s B^T never needs forming: dY_t . v_s = (dY_t B) . h_s, the dv_s B term of
         # dh_s is sum_p a_p (dY_t B), and dB = dv^T h = dY^T hacc with hacc_t = sum_p a_p h_s.
         x, gates, h, uniq, pair_slot, n_unique, perm, sorted_slot, seg_off, latents, w1, w2 = ctx.saved_tensors
-        seg = {"pair_slot": pair_slot, "perm": perm, "sorted_slot": sorted_slot, "seg_off": seg_off}
+        seg = {"pair_slot": pair_slot, "perm": perm, "sorted_slot": sorted_slot, "seg_off": seg_off, "uniq": uniq,
+               "n_unique": n_unique}
         H, k = ctx.heads, ctx.top_k
         n, d = x.shape
+        # one library call when every operand has the layer's dtype; torch operations for other
+        # sizes and dtypes, and under create_graph
+        if not torch.is_grad_enabled() and all(t == x.dtype for t in ctx.param_dtypes):
+            dyc = dy.contiguous()
+            if hip.expert_grads_supported(x, dyc, h, latents, w1, w2):
+                dx, dg, dlat, dw1, dw2 = hip.expert_grads(x, dyc, h, latents, w1, w2, seg, gates, H, k)
+                return dx, dg.view(gates.shape), dlat, dw1, dw2, None, None, None
         f = torch.float32
         U = int(n_unique.item())
         A, B, C = w2[:d].to(f), w2[d:].to(f), w1.to(f)

@@ -17,6 +17,7 @@
  *   ethos_apply_hidden   the same, by hidden-space reordering (no v rows)
  *   ethos_expert_forward generation + apply + scatter-back in one call (either order)
  *   ethos_expert_backward  per-pair part of the expert stages' backward
+ *   ethos_expert_grads   the expert stages' backward whole: every gradient in one call
  *
  * Conventions (every entry point):
  *   - All pointers are device pointers owned by the caller; nothing is allocated.
@@ -357,6 +358,31 @@ int ethos_expert_backward(const void* h, const float* xp, const float* dyb, cons
                           int64_t n_tok, int32_t n_heads, int32_t top_k, int32_t d_hidden, int32_t dtype,
                           void* workspace, size_t workspace_bytes, float* dscores, float* hacc, float* dxp, float* dh,
                           void* stream);
+
+/*
+ * The expert stages' backward whole (model.py:312-341 differentiated): from the forward's
+ * routing and hidden rows h, and dy [n_tok, d_model] of dtype T,
+ *   dx        [n_tok, d_model]        T        (the part through x_proj only)
+ *   dscores   [n_tok, n_heads, top_k] float32
+ *   dlatents  [n_experts, d_latent]   T        only the unique experts' rows are written: the
+ *                                              caller hands it over filled with zeros
+ *   dw1       [d_hidden, d_latent]    T
+ *   dw2       [2 d_model, d_hidden]   T
+ * with float32 sums throughout, each result rounded once; deterministic.  The number of
+ * unique experts is read on the device (n_unique, at most max_unique).
+ *   x, latents, w1, w2, scores, and the sort's outputs   as for ethos_expert_forward
+ *   workspace  >= ethos_expert_grads_workspace_bytes(...) bytes (scratch)
+ * Limits: d_latent, d_hidden and d_model multiples of 8, d_hidden <= 4096 (bf16) / 2048 (fp32);
+ * x, dy, h, latents, w1, w2 and workspace 16-byte aligned.
+ */
+size_t ethos_expert_grads_workspace_bytes(int64_t n_tok, int32_t n_heads, int32_t top_k, int64_t max_unique,
+                                          int32_t d_latent, int32_t d_hidden, int32_t d_model);
+int ethos_expert_grads(const void* x, const void* dy, const void* h, const void* latents, const void* w1, const void* w2,
+                       const int32_t* uniq_ids, const int32_t* seg_off, const int32_t* n_unique, int64_t max_unique,
+                       const int32_t* perm, const int32_t* sorted_slot, const int32_t* pair_slot, const void* scores,
+                       int64_t n_tok, int32_t n_heads, int32_t top_k, int32_t d_latent, int32_t d_hidden, int32_t d_model,
+                       int32_t dtype, void* workspace, size_t workspace_bytes, void* dx, float* dscores, void* dlatents,
+                       void* dw1, void* dw2, void* stream);
 
 #ifdef __cplusplus
 }

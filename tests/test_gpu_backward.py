@@ -191,3 +191,56 @@ def test_expert_backward_entry_point(dt, n, H, k, dh, E, hot):
     for got, ref, name in ((dg, ref_dg, "dscores"), (hacc, ref_hacc, "hacc"), (dxp, ref_dxp, "dxp"), (dhs, ref_dh, "dh")):
         assert got.shape == ref.shape, name
         assert _nerr(got, ref) < 1e-5, (name, _nerr(got, ref))
+
+
+@pytest.mark.parametrize("dt,n,H,k,dl,dh,d,E", [
+    ("bf16", 1, 1, 1, 8, 8, 8, 1), ("bf16", 33, 2, 4, 16, 40, 72, 37), ("bf16", 129, 3, 4, 136, 264, 200, 700),
+    ("bf16", 700, 4, 8, 128, 512, 256, 9000), ("bf16", 65, 8, 16, 128, 256, 1024, 1),
+    ("fp32", 1, 1, 2, 8, 16, 8, 4), ("fp32", 50, 4, 8, 24, 72, 40, 11), ("fp32", 500, 4, 8, 128, 512, 256, 4096)])
+def test_expert_grads_entry_point(dt, n, H, k, dl, dh, d, E):
+    """ethos_expert_grads against a float64 evaluation of the same derivative: sizes off every
+    tile (64, 128, 32 of the reduction), one pair, one expert, fewer unique experts than the
+    buffers hold, split and unsplit reductions.  float32 sums of at most 9,000 terms: 1e-5;
+    bf16 results are rounded once, at most 2^-8 of each value.  Two runs are bit-identical."""
+    from ethos_amd import hip
+    g = torch.Generator().manual_seed(n + dh + d)
+    tdt = torch.bfloat16 if dt == "bf16" else torch.float32
+    ids = torch.randint(0, E, (n * H * k,), generator=g, dtype=torch.int32)
+    seg = hip.sort_segment(ids.cuda(), E)
+    U, slot, uniq = int(seg["n_unique"].item()), seg["pair_slot"].cpu().long(), seg["uniq"].cpu().long()
+    max_u = seg["uniq"].numel()
+    rn = lambda *s: torch.randn(s, generator=g).to(tdt)  # noqa: E731
+    x, dy, lat = rn(n, d), rn(n, d), rn(E, dl)
+    w1, w2 = (rn(dh, dl) / dl ** 0.5).to(tdt), (rn(2 * d, dh) / d ** 0.5).to(tdt)
+    h = torch.zeros(max_u, dh, dtype=tdt)
+    # c = h . xp of order one: gelu(c) = c (1 + erf) / 2 is good to |c| 2^-24 absolutely, so a c
+    # of -5 alone (gelu 1e-6) would show as 0.3 relative, and one of -2.5 (0.016) as 1e-5
+    h[:U] = (rn(U, dh) * (0.5 / dh ** 0.5)).to(tdt)
+    gates = torch.rand(n, H, k, generator=g).to(tdt)
+    args = [t.cuda() for t in (x, dy, h, lat, w1, w2)]
+    assert hip.expert_grads_supported(*args)
+    got = hip.expert_grads(*args, seg, gates.cuda(), H, k)
+    again = hip.expert_grads(*args, seg, gates.cuda(), H, k)
+    x64, dy64, h64, z, C, W2 = x.double(), dy.double(), h.double(), lat[uniq[:U]].double(), w1.double(), w2.double()
+    A, B = W2[:d], W2[d:]
+    t = torch.arange(n * H * k) // (H * k)
+    xp, dyb, hs, gp = x64 @ A, dy64 @ B / H, h64[slot], gates.double().reshape(-1)
+    grad = lambda v: 0.5 * torch.erfc(-v / 2 ** 0.5) + v * torch.exp(-0.5 * v * v) / (2 * torch.pi) ** 0.5  # noqa: E731
+    c, da = (hs * xp[t]).sum(-1), (hs * dyb[t]).sum(-1)
+    act, dc = torch.nn.functional.gelu(c), gp * grad(c) * da
+    a = act * gp
+    hacc = torch.zeros(n, dh, dtype=torch.float64).index_add_(0, t, a[:, None] * hs)
+    dxp = torch.zeros(n, dh, dtype=torch.float64).index_add_(0, t, dc[:, None] * hs)
+    dhs = torch.zeros(U, dh, dtype=torch.float64).index_add_(0, slot, a[:, None] * dyb[t] + dc[:, None] * xp[t])
+    dpre = grad(z @ C.T) * dhs
+    dlat = torch.zeros(E, dl, dtype=torch.float64)
+    dlat[uniq[:U]] = dpre @ C
+    ref = (dxp @ A.T, (act * da).view(n, H, k), dlat, dpre.T @ z, torch.cat([x64.T @ dxp, dy64.T @ hacc / H]))
+    for i, name in enumerate(("dx", "dgates", "dlatents", "dw1", "dw2")):
+        assert torch.equal(got[i], again[i]), f"{name} differs between two runs"
+        assert got[i].shape == ref[i].shape, name
+        tol = 1e-5 if dt == "fp32" or name == "dgates" else 2.0 ** -8
+        assert _nerr(got[i], ref[i]) < tol, (name, _nerr(got[i], ref[i]))
+    unused = torch.ones(E, dtype=torch.bool)
+    unused[uniq[:U]] = False
+    assert not got[2].cpu()[unused].any()
