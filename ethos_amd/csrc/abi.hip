@@ -611,4 +611,91 @@ int ethos_expert_grads(const void* x, const void* dy, const void* h, const void*
     return hip_status(rc, "ethos_expert_grads");
 }
 
+size_t ethos_query_bn_workspace_bytes(int64_t n_tok, int32_t n_heads, int32_t d_query) {
+    if (n_tok <= 0 || n_heads <= 0 || d_query <= 0) return 256;
+    return ethos::query_bn_workspace_bytes(n_tok, n_heads, d_query);
+}
+
+int ethos_query_bn_train(const void* v, int64_t n_tok, int32_t n_heads, int32_t d_query, int32_t dtype, const void* const* gamma,
+                         const void* const* beta, void* const* running_mean, void* const* running_var,
+                         const float* const* batch_mean, const float* const* batch_var, double momentum, double eps,
+                         void* workspace, size_t workspace_bytes, void* q, void* stream) {
+    g_err[0] = 0;
+    if (!dtype_ok(dtype)) return fail(ETHOS_EDTYPE, "ethos_query_bn_train: unknown dtype %d", dtype);
+    if (n_tok < 2 || n_tok > INT32_MAX || n_heads <= 0 || d_query <= 0)
+        return fail(ETHOS_ESIZE, "ethos_query_bn_train: bad sizes (batch statistics need two tokens)");
+    if (n_heads > ethos::kMaxBnHeads || d_query % 4)
+        return fail(ETHOS_EUNSUPPORTED, "ethos_query_bn_train: at most %d heads and d_query %% 4 == 0", ethos::kMaxBnHeads);
+    if (!v || !gamma || !beta || (!running_mean) != (!running_var) || (!batch_mean) != (!batch_var) || !workspace ||
+        !q)
+        return fail(ETHOS_ENULL, "ethos_query_bn_train: null pointer");
+    for (int h = 0; h < n_heads; ++h)
+        if (!gamma[h] || !beta[h] || (running_mean && (!running_mean[h] || !running_var[h])) ||
+            (batch_mean && (!batch_mean[h] || !batch_var[h])))
+            return fail(ETHOS_ENULL, "ethos_query_bn_train: null pointer (head %d)", h);
+    const size_t need = ethos::query_bn_workspace_bytes(n_tok, n_heads, d_query);
+    if (workspace_bytes < need)
+        return fail(ETHOS_EWORKSPACE, "ethos_query_bn_train: workspace of %zu bytes, %zu needed", workspace_bytes, need);
+    if (!aligned16(v) || !aligned16(workspace) || !aligned16(q))
+        return fail(ETHOS_EALIGN, "ethos_query_bn_train: v, workspace and q must be 16-byte aligned");
+    return hip_status(ethos::launch_query_bn(v, n_tok, n_heads, d_query, dtype, gamma, beta, running_mean, running_var, batch_mean,
+                                             batch_var, momentum, eps, workspace, q, num_cus(), (hipStream_t)stream),
+                      "ethos_query_bn_train");
+}
+
+int ethos_bn_coefficients(int32_t n_heads, int32_t d_query, int32_t dtype, const void* const* gamma, const void* const* beta,
+                          const void* const* running_mean, const void* const* running_var, double eps, float* alpha_out,
+                          float* beta_out, void* stream) {
+    g_err[0] = 0;
+    if (!dtype_ok(dtype)) return fail(ETHOS_EDTYPE, "ethos_bn_coefficients: unknown dtype %d", dtype);
+    if (n_heads <= 0 || d_query <= 0) return fail(ETHOS_ESIZE, "ethos_bn_coefficients: bad sizes");
+    if (n_heads > ethos::kMaxBnHeads)
+        return fail(ETHOS_EUNSUPPORTED, "ethos_bn_coefficients: at most %d heads", ethos::kMaxBnHeads);
+    if (!alpha_out || !beta_out) return fail(ETHOS_ENULL, "ethos_bn_coefficients: null pointer");
+    return hip_status(ethos::launch_bn_coefficients(n_heads, d_query, dtype, gamma, beta, (void* const*)running_mean,
+                                                    (void* const*)running_var, eps, alpha_out, beta_out, (hipStream_t)stream),
+                      "ethos_bn_coefficients");
+}
+
+size_t ethos_gate_grads_workspace_bytes(int64_t n_tok, int32_t n_heads, int32_t top_k, int32_t d_model, int32_t d_query,
+                                        int32_t n_sub) {
+    if (n_tok <= 0 || n_heads <= 0 || top_k <= 0 || d_model <= 0 || d_query <= 0 || n_sub <= 0) return 256;
+    return ethos::gate_grads_workspace_bytes(n_tok, n_heads, top_k, d_model, d_query, n_sub, num_cus());
+}
+
+int ethos_gate_grads(const void* x, const int32_t* ids, const float* dscores, const void* wq, const void* bq,
+                     const void* sub_keys_1, const void* sub_keys_2, const void* const* gamma, const void* const* beta,
+                     const void* const* running_mean, const void* const* running_var, double eps, int64_t n_tok, int32_t d_model,
+                     int32_t n_heads, int32_t d_query, int32_t n_sub, int32_t top_k, int32_t dtype, void* workspace,
+                     size_t workspace_bytes, void* dx, void* dwq, void* dbq, void* dgamma, void* dbeta, void* dkeys_1,
+                     void* dkeys_2, void* stream) {
+    g_err[0] = 0;
+    if (!dtype_ok(dtype)) return fail(ETHOS_EDTYPE, "ethos_gate_grads: unknown dtype %d", dtype);
+    if (n_tok < 0 || n_heads <= 0 || d_query <= 0 || n_sub <= 0 || top_k <= 0 || d_model <= 0)
+        return fail(ETHOS_ESIZE, "ethos_gate_grads: bad sizes");
+    if (d_model % 8 || !ethos::gate_grads_supported(n_heads, d_query, n_sub, top_k))
+        return fail(ETHOS_EUNSUPPORTED,
+                    "ethos_gate_grads: needs d_model %% 8 == 0, d_query %% 8 == 0 and at most 512 with whole lanes, at most %d "
+                    "heads, 1024 sub-keys and top_k 64 (got d_model %d, d_query %d, %d heads, %d, %d)",
+                    ethos::kMaxBnHeads, d_model, d_query, n_heads, n_sub, top_k);
+    if (n_tok > INT32_MAX || n_tok * n_heads * top_k > INT32_MAX) return fail(ETHOS_ESIZE, "ethos_gate_grads: too many pairs");
+    if (n_tok == 0) return 0;
+    if (!x || !ids || !dscores || !wq || !bq || !sub_keys_1 || !sub_keys_2 || !gamma || !beta || (!running_mean) != (!running_var) ||
+        !workspace || !dbq || !dgamma || !dbeta || !dkeys_1 || !dkeys_2)
+        return fail(ETHOS_ENULL, "ethos_gate_grads: null pointer");
+    for (int h = 0; h < n_heads; ++h)
+        if (!gamma[h] || !beta[h] || (running_mean && (!running_mean[h] || !running_var[h])))
+            return fail(ETHOS_ENULL, "ethos_gate_grads: null pointer (head %d)", h);
+    const size_t need = ethos::gate_grads_workspace_bytes(n_tok, n_heads, top_k, d_model, d_query, n_sub, num_cus());
+    if (workspace_bytes < need)
+        return fail(ETHOS_EWORKSPACE, "ethos_gate_grads: workspace of %zu bytes, %zu needed", workspace_bytes, need);
+    if (!aligned16(x) || !aligned16(wq) || !aligned16(sub_keys_1) || !aligned16(sub_keys_2) || !aligned16(workspace))
+        return fail(ETHOS_EALIGN, "ethos_gate_grads: x, wq, the sub-keys and workspace must be 16-byte aligned");
+    return hip_status(ethos::launch_gate_grads(x, ids, dscores, wq, bq, sub_keys_1, sub_keys_2, gamma, beta,
+                                               (void* const*)running_mean, (void* const*)running_var, eps, n_tok, d_model, n_heads,
+                                               d_query, n_sub, top_k, dtype, workspace, dx, dwq, dbq, dgamma, dbeta, dkeys_1,
+                                               dkeys_2, num_cus(), (hipStream_t)stream),
+                      "ethos_gate_grads");
+}
+
 }  // extern "C"

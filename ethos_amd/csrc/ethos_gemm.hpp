@@ -15,7 +15,7 @@ struct Gemm {
     const void* a = nullptr;
     const void* b = nullptr;
     void* c = nullptr;
-    const float* bias = nullptr;       // float32 [n] (not with split > 1)
+    const void* bias = nullptr;        // [n] of B's type (not with split > 1)
     const int32_t* a_rows = nullptr;   // K-stored A: row m of A is row a_rows[m] of `a`
     const int32_t* b_rows = nullptr;   // R-stored B: row k of B is row b_rows[k] of `b`
     const int32_t* c_rows = nullptr;   // row m of C is row c_rows[m] of `c`

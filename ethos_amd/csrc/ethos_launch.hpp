@@ -97,6 +97,21 @@ int launch_expert_grads(const void* x, const void* dy, const void* hid, const vo
                         const int32_t* perm, const int32_t* sorted_slot, const int32_t* pair_slot, const void* gates,
                         int64_t n_tok, int H, int k, int dl, int dh, int d, int dtype, void* ws, void* dx, float* dg,
                         void* dlat, void* dw1, void* dw2, int num_cus, hipStream_t stream);
+// Query BatchNorm and the gates' backward (gate.hip).  Per-head parameters come as host arrays
+// of H device pointers; mean and var null: batch statistics (launch_query_bn: no update).
+constexpr int kMaxBnHeads = 32;
+size_t query_bn_workspace_bytes(int64_t n, int H, int dq);
+int launch_query_bn(const void* v, int64_t n, int H, int dq, int dtype, const void* const* gamma, const void* const* beta,
+                    void* const* mean, void* const* var, const float* const* batch_mean, const float* const* batch_var,
+                    double momentum, double eps, void* ws, void* q, int num_cus, hipStream_t stream);
+int launch_bn_coefficients(int H, int dq, int dtype, const void* const* gamma, const void* const* beta, void* const* mean,
+                           void* const* var, double eps, float* alpha, float* shift, hipStream_t stream);
+bool gate_grads_supported(int H, int dq, int K, int k);
+size_t gate_grads_workspace_bytes(int64_t n, int H, int k, int d, int dq, int K, int num_cus);
+int launch_gate_grads(const void* x, const int32_t* ids, const float* dg, const void* wq, const void* bq, const void* k1,
+                      const void* k2, const void* const* gamma, const void* const* beta, void* const* mean, void* const* var,
+                      double eps, int64_t n, int d, int H, int dq, int K, int k, int dtype, void* ws, void* dx, void* dw, void* db,
+                      void* dgamma, void* dbeta, void* dk1, void* dk2, int num_cus, hipStream_t stream);
 size_t apply_hidden_workspace_bytes(int64_t n_tok, int H, int k, int d, int dh, int dtype);
 int launch_apply_hidden(const void* x, const void* w2, const void* hid, const int32_t* perm,
                         const int32_t* sorted_slot, const int32_t* pair_slot, const void* gates, int64_t n_tok, int H,

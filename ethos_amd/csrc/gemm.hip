@@ -306,7 +306,7 @@ __global__ __launch_bounds__(kGemmThreads, (BM > 64 ? (sizeof(TB) == 4 ? 3 : 4) 
     for (int j = 0; j < NI; ++j) {
         const int n = n0 + wn + j * 32 + (lane & 31);
         const int nc = n < p.n ? n : p.n - 1;
-        const float bias = p.bias ? p.bias[nc] : 0.0f;
+        const float bias = p.bias ? Elem<TB>::to_f32(((const TB*)p.bias)[nc]) : 0.0f;
 #pragma unroll
         for (int i = 0; i < MI; ++i) {
             const int64_t mb = m0 + wm + i * 32;

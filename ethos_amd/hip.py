@@ -58,15 +58,10 @@ def stage_events(events) -> None:
 
 
 def key_norm_bounds(sub_keys_1: torch.Tensor, sub_keys_2: torch.Tensor) -> torch.Tensor:
-    """fp32 [2, K] upper bounds of the sub-key row norms: fp64 norms of the stored
-    values, inflated by 2^-20 and rounded, on the host (once per parameter version)."""
-    import numpy as np
-
-    rows = []
-    for t in (sub_keys_1, sub_keys_2):
-        v = t.detach().float().cpu().numpy().astype(np.float64)
-        rows.append((np.sqrt((v * v).sum(axis=1)) * (1.0 + 2.0 ** -20)).astype(np.float32))
-    return torch.from_numpy(np.stack(rows)).contiguous()
+    """fp32 [2, K] upper bounds of the sub-key row norms, on the tables' device: fp64 norms of
+    the stored values, inflated by 2^-20 and rounded (once per parameter version)."""
+    v = torch.stack((sub_keys_1.detach(), sub_keys_2.detach())).double()
+    return (v.square().sum(dim=2).sqrt() * (1.0 + 2.0 ** -20)).float()
 
 
 def query_proj_prepare(wq: torch.Tensor) -> torch.Tensor | None:
@@ -445,3 +440,106 @@ def expert_grads(x: torch.Tensor, dy: torch.Tensor, h: torch.Tensor, latents: to
                                    dw2.data_ptr(), _stream())
     check(rc, "ethos_expert_grads")
     return dx, dg, dlat, dw1, dw2
+
+
+def _pointers(ts):
+    """A host array of the tensors' device pointers (None: a null array), for the length of a call."""
+    import ctypes
+
+    return (ctypes.c_void_p * len(ts))(*[t.data_ptr() for t in ts]) if ts is not None else None
+
+
+def _need_heads(ts, name: str, dtype, n: int) -> None:
+    for t in ts:
+        _need(t, name, dtype, 1)
+        if t.numel() != n:
+            raise RuntimeError(f"{name} must have {n} values per head, got shape {tuple(t.shape)}")
+
+
+def bn_coefficients(gamma, beta, mean, var, eps: float, dq: int, dtype, device) -> tuple[torch.Tensor, torch.Tensor]:
+    """(alpha, beta) float32 [H, dq] of query_proj from lists of per-head tensors [dq] (a list may
+    be None: gamma, var 1, beta, mean 0)."""
+    lists = [ts for ts in (gamma, beta, mean, var) if ts is not None]
+    for ts in lists:
+        _need_heads(ts, "BatchNorm tensor", dtype, dq)
+    H = len(lists[0])
+    out = torch.empty((2, H, dq), dtype=torch.float32, device=device)
+    rc = load().ethos_bn_coefficients(H, dq, dtype_code(dtype), _pointers(gamma), _pointers(beta), _pointers(mean), _pointers(var),
+                                      float(eps), out[0].data_ptr(), out[1].data_ptr(), _stream())
+    check(rc, "ethos_bn_coefficients")
+    return out[0], out[1]
+
+
+# Heads up to which the BatchNorm and gate kernels take per-head tensors (kMaxBnHeads).
+MAX_BN_HEADS = 32
+
+
+def query_bn_train(v: torch.Tensor, gamma, beta, mean, var, momentum: float, eps: float, batch=None) -> torch.Tensor:
+    """Training-mode BatchNorm of the queries v [n, H, dq] with the batch's statistics, per-head
+    gamma and beta; mean and var (lists, or None) are updated in place.  `batch`: the batch's
+    (means, biased variances), lists of float32 [dq], if the caller has them."""
+    _need(v, "v", dim=3)
+    n, H, dq = v.shape
+    for name, ts in (("gamma", gamma), ("beta", beta), ("running_mean", mean), ("running_var", var)):
+        if ts is not None:
+            if len(ts) != H:
+                raise RuntimeError(f"query_bn_train: {name} must have one tensor per head")
+            _need_heads(ts, name, v.dtype, dq)
+    for ts in batch or ():
+        if len(ts) != H:
+            raise RuntimeError("query_bn_train: batch statistics must have one tensor per head")
+        _need_heads(ts, "batch statistics", torch.float32, dq)
+    batch = batch or (None, None)
+    ws, ws_bytes = workspace(load().ethos_query_bn_workspace_bytes(n, H, dq), v.device)
+    q = torch.empty_like(v)
+    rc = load().ethos_query_bn_train(v.data_ptr(), n, H, dq, dtype_code(v.dtype), _pointers(gamma), _pointers(beta),
+                                     _pointers(mean), _pointers(var), _pointers(batch[0]), _pointers(batch[1]), float(momentum),
+                                     float(eps), ws.data_ptr(), ws_bytes,
+                                     q.data_ptr(), _stream())
+    check(rc, "ethos_query_bn_train")
+    return q
+
+
+def gate_grads_supported(n: int, d: int, H: int, dq: int, K: int, k: int) -> bool:
+    """Whether gate_grads takes these sizes (ethos_gate_grads' limits)."""
+    v = (dq // 2 + 31) // 32
+    lane = 1 if v <= 1 else 2 if v <= 2 else 4 if v <= 4 else 8
+    return (n > 0 and d % 8 == 0 and dq % 8 == 0 and dq <= 512 and (dq // 2) % lane == 0 and H <= MAX_BN_HEADS
+            and K <= 1024 and k <= 64)
+
+
+def gate_grads(x: torch.Tensor, ids: torch.Tensor, dg: torch.Tensor, wq: torch.Tensor, bq: torch.Tensor, k1: torch.Tensor,
+               k2: torch.Tensor, gamma, beta, mean, var, eps: float, want_x: bool = True, want_w: bool = True):
+    """Backward of the routing gates: (dx, dwq [H, dq, d], dbq, dgamma, dbeta [H, dq], dk1, dk2)
+    from dg float32 [n, H, k]; mean and var None: batch statistics.  dx and dwq are None unless
+    wanted."""
+    _need(x, "x", dim=2)
+    _need(ids, "ids", torch.int32, 3)
+    _need(dg, "dg", torch.float32, 3)
+    _need(wq, "wq", x.dtype, 3)
+    _need(bq, "bq", x.dtype, 2)
+    _need(k1, "sub_keys_1", x.dtype, 2)
+    _need(k2, "sub_keys_2", x.dtype, 2)
+    n, d = x.shape
+    H, dq, d2 = wq.shape
+    K = k1.shape[0]
+    if d2 != d or bq.shape != (H, dq) or k1.shape != (K, dq // 2) or k2.shape != k1.shape or ids.shape != dg.shape \
+            or ids.shape[:2] != (n, H):
+        raise RuntimeError("gate_grads: inconsistent shapes")
+    for ts in (gamma, beta, mean, var):
+        if ts is not None:
+            if len(ts) != H:
+                raise RuntimeError("gate_grads: one BatchNorm tensor per head")
+            _need_heads(ts, "BatchNorm tensor", x.dtype, dq)
+    k = ids.shape[2]
+    ws, ws_bytes = workspace(load().ethos_gate_grads_workspace_bytes(n, H, k, d, dq, K), x.device)
+    dx = torch.empty_like(x) if want_x else None
+    dw = torch.empty_like(wq) if want_w else None
+    db = torch.empty_like(bq)
+    dgamma, dbeta, dk1, dk2 = torch.empty_like(bq), torch.empty_like(bq), torch.empty_like(k1), torch.empty_like(k2)
+    rc = load().ethos_gate_grads(x.data_ptr(), ids.data_ptr(), dg.data_ptr(), wq.data_ptr(), bq.data_ptr(), k1.data_ptr(),
+                                 k2.data_ptr(), _pointers(gamma), _pointers(beta), _pointers(mean), _pointers(var), float(eps),
+                                 n, d, H, dq, K, k, dtype_code(x.dtype), ws.data_ptr(), ws_bytes,
+                                 dx.data_ptr() if want_x else None, dw.data_ptr() if want_w else None, db.data_ptr(), dgamma.data_ptr(), dbeta.data_ptr(), dk1.data_ptr(), dk2.data_ptr(), _stream())
+    check(rc, "ethos_gate_grads")
+    return dx, dw, db, dgamma, dbeta, dk1, dk2

@@ -62,6 +62,77 @@ def _gelu_grad(x: torch.Tensor) -> torch.Tensor:
     return cdf + x * pdf
 
 
+def _gate_values(x_flat, ids, w_list, b_list, gammas, betas, k1, k2, stats, epss) -> torch.Tensor:
+    """float32 gates [n, H, k] at the chosen expert ids by torch operations: per-head lists of the
+    projection and BatchNorm parameters (gamma and beta None: not affine), `stats` per head
+    None for batch statistics or (running mean, running variance)."""
+    f = torch.float32
+    H, dq, K = len(w_list), w_list[0].shape[0], k1.shape[0]
+    n = x_flat.shape[0]
+    w = torch.stack(w_list).to(f).reshape(H * dq, -1)
+    b = torch.stack(b_list).to(f).reshape(-1)
+    q = x_flat.to(f) @ w.T + b                                       # [n, H dq]
+    # the H per-head BatchNorms as one over H dq channels (same per-channel statistics)
+    batch = [s is None for s in stats]
+    if (all(batch) or not any(batch)) and len(set(epss)) == 1:
+        cat = lambda ts: torch.cat([t.to(f) for t in ts])  # noqa: E731
+        affine = all(t is not None for t in gammas)
+        q = F.batch_norm(q, None if batch[0] else cat(s[0] for s in stats), None if batch[0] else cat(s[1] for s in stats),
+                         cat(gammas) if affine else None, cat(betas) if affine else None, batch[0], 0.0, epss[0])
+    else:  # heads in different modes or with different eps: one call per head
+        q = q.view(n, H, dq)
+        q = torch.stack([F.batch_norm(q[:, h], None if s is None else s[0].to(f), None if s is None else s[1].to(f),
+                                      None if gammas[h] is None else gammas[h].to(f),
+                                      None if betas[h] is None else betas[h].to(f), s is None, 0.0, epss[h])
+                         for h, s in enumerate(stats)], dim=1)
+    q = q.view(n * H, dq)
+    half = dq // 2
+    # dense sub-scores, then the chosen columns: the backward is a GEMM for the keys
+    s1 = (q[:, :half] @ k1.to(f).T).gather(1, (ids // K).view(n * H, -1))
+    s2 = (q[:, half:] @ k2.to(f).T).gather(1, (ids % K).view(n * H, -1))
+    return torch.softmax(s1 + s2, dim=-1).view(ids.shape)
+
+
+class _GatePath(torch.autograd.Function):
+    """The routing gates as one autograd node: forward the exact gates as float32, backward the
+    derivative of _gate_values (ethos_gate_grads, which recomputes the queries from x).  wq and
+    bq are the packed projections; `params` the tensors the gradients go to: weight and bias
+    per head, both sub-key tables, the BatchNorms' weights, then their biases.  `stats`: None
+    for batch statistics, or (means, variances) [H, d_query] at the time of the forward."""
+
+    @staticmethod
+    def forward(ctx, x, ids, gates, wq, bq, stats, eps, *params):
+        ctx.save_for_backward(x, ids, wq, bq, *(stats or ()), *params)
+        ctx.batch, ctx.eps = stats is None, eps
+        return gates.to(torch.float32, copy=True)
+
+    @staticmethod
+    def backward(ctx, dg):
+        x, ids, wq, bq = ctx.saved_tensors[:4]
+        rest = ctx.saved_tensors[4:]
+        stats, params = (None, rest) if ctx.batch else (rest[:2], rest[2:])
+        H = wq.shape[0]
+        w, b, (k1, k2) = params[0:2 * H:2], params[1:2 * H:2], params[2 * H:2 * H + 2]
+        gamma, beta = params[2 * H + 2:3 * H + 2], params[3 * H + 2:]
+        head = (None,) * 6
+        if torch.is_grad_enabled():  # create_graph: the torch operations' own derivative
+            g = _gate_values(x, ids.long(), w, b, gamma, beta, k1, k2,
+                             [None] * H if stats is None else list(zip(*stats)), [ctx.eps] * H)
+            ts = [x, *params]
+            want = [t for t, need in zip(ts, (ctx.needs_input_grad[0], *ctx.needs_input_grad[7:])) if need]
+            got = dict(zip(map(id, want), torch.autograd.grad(g, want, dg, create_graph=True, allow_unused=True)))
+            return (got.get(id(x)), *head, *(got.get(id(t)) for t in params))
+        dx, dw, db, dgamma, dbeta, dk1, dk2 = hip.gate_grads(
+            x, ids, dg.contiguous(), wq, bq, k1.detach(), k2.detach(), [t.detach() for t in gamma], [t.detach() for t in beta],
+            stats and list(stats[0]), stats and list(stats[1]), ctx.eps, want_x=ctx.needs_input_grad[0],
+            want_w=any(ctx.needs_input_grad[7:7 + 2 * H:2]))
+        grads = [None] * (2 * H)
+        if dw is not None:
+            grads[0::2] = dw.unbind(0)
+        grads[1::2] = db.unbind(0)
+        return (dx, *head, *grads, dk1, dk2, *dgamma.unbind(0), *dbeta.unbind(0))
+
+
 class _ExpertStages(torch.autograd.Function):
     """Expert generation, apply and scatter-back as one autograd node.
 
@@ -173,61 +244,121 @@ class ProductKeyRouter(nn.Module):
         self.sub_keys_2 = nn.Embedding(self.num_sub_keys, self.d_query // 2)
         self._cache_key = None
         self._cache = None
+        self._bn_key = None
+        self._bn = None
+        self._identity = None
         self._key_norms = None
         self._keys_prepared = None
         self._wq_prepared = None
 
     # -- parameter packing (cached until a parameter changes) ---------------------
-    def _packed_sources(self) -> list:
-        """The tensors the packed form is built from, read from the modules' parameter and
-        buffer dicts directly (this runs on every call; nn.Module attribute lookup is slow)."""
+    def _weight_sources(self) -> list:
+        """The projection weights and sub-keys, read from the modules' parameter dicts directly
+        (this runs on every call; nn.Module attribute lookup is slow)."""
         ts = []
         for m in self._modules["query_projs"]._modules.values():
             ts += (m._parameters["weight"], m._parameters["bias"])
         ts += (self._modules["sub_keys_1"]._parameters["weight"], self._modules["sub_keys_2"]._parameters["weight"])
+        return ts
+
+    def _bn_sources(self) -> list:
+        ts = []
         for m in self._modules["query_norms"]._modules.values():
             ts += (m._parameters["weight"], m._parameters["bias"], m._buffers["running_mean"], m._buffers["running_var"])
         return ts
 
-    def _packed(self, dtype: torch.dtype, device: torch.device):
-        key = (dtype, device, tuple((t.data_ptr(), t._version) for t in self._packed_sources() if t is not None))
+    def _packed_sources(self) -> list:
+        """The tensors the packed form is built from."""
+        return self._weight_sources() + self._bn_sources()
+
+    def _packed_weights(self, dtype: torch.dtype, device: torch.device):
+        key = (dtype, device, tuple((t.data_ptr(), t._version) for t in self._weight_sources() if t is not None))
         if key != self._cache_key:
             wq = torch.stack([m.weight.detach() for m in self.query_projs]).to(device=device, dtype=dtype).contiguous()
             bq = torch.stack([m.bias.detach() for m in self.query_projs]).to(device=device, dtype=dtype).contiguous()
             k1 = self.sub_keys_1.weight.detach().to(device=device, dtype=dtype).contiguous()
             k2 = self.sub_keys_2.weight.detach().to(device=device, dtype=dtype).contiguous()
-            alpha, beta = [], []
-            for m in self.query_norms:
-                a, b = _bn_eval_coefficients(m, self.d_query)
-                alpha.append(a)
-                beta.append(b)
-            alpha = torch.from_numpy(np.stack(alpha)).contiguous().to(device)
-            beta = torch.from_numpy(np.stack(beta)).contiguous().to(device)
-            self._key_norms = hip.key_norm_bounds(k1, k2).to(device)
+            self._key_norms = hip.key_norm_bounds(k1, k2)
             # the sub-keys in the scoring MFMAs' fragment order
             self._keys_prepared = hip.route_prepare_keys(k1, k2) if k1.is_cuda else None
             # the projection weights' prepared form (bf16: digit planes), reused by every call
             # until a parameter changes
             self._wq_prepared = hip.query_proj_prepare(wq) if wq.is_cuda else None
-            self._cache = (wq, bq, k1, k2, alpha, beta)
+            self._cache = (wq, bq, k1, k2)
             self._cache_key = key
         return self._cache
+
+    def _bn_coefficients(self, device: torch.device):
+        """(alpha, beta) of the eval-mode BatchNorms, float32 [H, d_query] on the device."""
+        ts = self._bn_sources()
+        key = (device, tuple((t.data_ptr(), t._version) for t in ts if t is not None))
+        if key != self._bn_key:
+            norms, H = list(self.query_norms), self.num_heads
+            one = ts[0].dtype if ts[0] is not None else None
+            if (device.type == "cuda" and H <= hip.MAX_BN_HEADS and len({m.eps for m in norms}) == 1
+                    and all(m.affine and m.track_running_stats for m in norms) and one in (torch.float32, torch.bfloat16)
+                    and all(t is not None and t.dtype == one and t.device == device and t.is_contiguous() for t in ts)):
+                # on the device: the host evaluation below waits for four tensors of every head
+                self._bn = hip.bn_coefficients(*([m.detach() for m in ts[i::4]] for i in range(4)), norms[0].eps, self.d_query,
+                                               one, device)
+            else:
+                ab = [_bn_eval_coefficients(m, self.d_query) for m in norms]
+                self._bn = tuple(torch.from_numpy(np.stack(c)).contiguous().to(device) for c in zip(*ab))
+            self._bn_key = key
+        return self._bn
+
+    def _packed(self, dtype: torch.dtype, device: torch.device):
+        return self._packed_weights(dtype, device) + tuple(self._bn_coefficients(device))
 
     def _bn_uses_batch_stats(self) -> bool:
         return any(m.training or not m.track_running_stats for m in self.query_norms)
 
+    def _bn_one_call(self, x_flat: torch.Tensor) -> bool:
+        """Whether the heads' training-mode BatchNorms run as one library call: all of them on
+        batch statistics with one eps and momentum, affine, in the layer's dtype on its device,
+        without gradients of their own and over at least two tokens (torch refuses fewer)."""
+        norms = list(self.query_norms)
+        m0 = norms[0]
+        ts = [t for t in self._bn_sources() if t is not None]
+        return (x_flat.shape[0] > 1 and self.num_heads <= hip.MAX_BN_HEADS and not torch.is_grad_enabled()
+                and self.d_query % 4 == 0
+                and all(m.affine and m.training and m.eps == m0.eps and m.momentum == m0.momentum
+                        and m.track_running_stats == m0.track_running_stats
+                        and (m.running_mean is not None) == m0.track_running_stats for m in norms)
+                and all(t.dtype == x_flat.dtype and t.device == x_flat.device and t.is_contiguous() for t in ts))
+
     def queries(self, x_flat: torch.Tensor, packed=None) -> torch.Tensor:
         """Per-head queries after BatchNorm, [n, H, d_query] (model.py:215-216).  `packed`:
         the result of _packed for x_flat's dtype and device, if the caller has it."""
-        wq, bq, _, _, alpha, beta = packed if packed is not None else self._packed(x_flat.dtype, x_flat.device)
         if not self._bn_uses_batch_stats():
+            wq, bq, _, _, alpha, beta = packed if packed is not None else self._packed(x_flat.dtype, x_flat.device)
             return hip.query_proj(x_flat, wq, bq, alpha, beta, prepared=self._wq_prepared)
         # Training-mode BatchNorm normalises with batch statistics and updates the
-        # running stats: project with an identity affine, then apply torch's batch_norm
-        # per head on the projected queries.
-        ones = torch.ones_like(alpha)
-        zeros = torch.zeros_like(beta)
-        q_lin = hip.query_proj(x_flat, wq, bq, ones, zeros, prepared=self._wq_prepared)
+        # running stats: project with an identity affine, then normalise the projected queries.
+        wq, bq = (packed if packed is not None else self._packed_weights(x_flat.dtype, x_flat.device))[:2]
+        if self._identity is None or self._identity[0].device != x_flat.device:
+            ones = torch.ones((self.num_heads, self.d_query), dtype=torch.float32, device=x_flat.device)
+            self._identity = (ones, torch.zeros_like(ones))
+        q_lin = hip.query_proj(x_flat, wq, bq, *self._identity, prepared=self._wq_prepared)
+        if self._bn_one_call(x_flat):
+            m0 = self.query_norms[0]
+            ts, track = self._bn_sources(), m0.track_running_stats
+            batch = None
+            if q_lin.dtype == torch.bfloat16:
+                # bf16 sub-scores are full of ties, so the last bit of a mean decides experts:
+                # the statistics are torch's own, head by head as batch_norm takes them, and the
+                # layer chooses what it would choose there (float32 sums of another order move
+                # about 1 row in 400 to another expert at 4,096 tokens, within rounding)
+                qf = q_lin.float()
+                pairs = [torch.var_mean(qf[:, h], 0, unbiased=False) for h in range(self.num_heads)]
+                batch = [p[1] for p in pairs], [p[0] for p in pairs]
+            out = hip.query_bn_train(q_lin, *([t.detach() for t in ts[i::4]] for i in range(2)),
+                                     ts[2::4] if track else None, ts[3::4] if track else None,
+                                     m0.momentum if m0.momentum is not None else 0.1, m0.eps, batch=batch)
+            if track:
+                torch._foreach_add_([m.num_batches_tracked for m in self.query_norms], 1)
+                self._bn_key = None  # the running statistics' version counters do not move
+            return out
         outs = []
         for h, m in enumerate(self.query_norms):
             outs.append(F.batch_norm(q_lin[:, h], m.running_mean, m.running_var,
@@ -237,16 +368,19 @@ class ProductKeyRouter(nn.Module):
             if m.training and m.track_running_stats:
                 m.num_batches_tracked.add_(1)
         # batch_norm updated the running statistics in place without bumping their version
-        # counters, so the eval-mode coefficients cached by _packed are stale
+        # counters, so the cached eval-mode coefficients are stale
         if any(m.training and m.track_running_stats for m in self.query_norms):
-            self._cache_key = None
+            self._bn_key = None
         return torch.stack(outs, dim=1).contiguous()
 
     def route(self, x_flat: torch.Tensor, mark=None):
         """(gates [n, H, k] x.dtype, expert ids [n, H, k] int32).  `mark(stage)`, if given,
         is called after each stage is enqueued (used to place timing events)."""
-        packed = self._packed(x_flat.dtype, x_flat.device)
-        _, _, k1, k2, _, _ = packed
+        if self._bn_uses_batch_stats():
+            packed = self._packed_weights(x_flat.dtype, x_flat.device)
+        else:
+            packed = self._packed(x_flat.dtype, x_flat.device)
+        k1, k2 = packed[2:4]
         q = self.queries(x_flat, packed)
         if mark is not None:
             mark("query_proj")
@@ -262,48 +396,42 @@ class ProductKeyRouter(nn.Module):
         g = softmax(q1 · K1[i1] + q2 · K2[i2]) with i1 = id // K, i2 = id % K.  BatchNorm uses
         the module's mode (batch statistics when training) without touching the running
         statistics, which the routing pass has already updated."""
-        f = torch.float32
-        H, dq, K = self.num_heads, self.d_query, self.num_sub_keys
-        n = x_flat.shape[0]
-        w = torch.stack([m.weight for m in self.query_projs]).to(f).reshape(H * dq, -1)
-        b = torch.stack([m.bias for m in self.query_projs]).to(f).reshape(-1)
-        q = x_flat.to(f) @ w.T + b                                       # [n, H dq]
-        # the H per-head BatchNorms as one over H dq channels (same per-channel statistics)
         norms = list(self.query_norms)
-        batch = [m.training or not m.track_running_stats for m in norms]
-        if all(batch) or not any(batch):
-            cat = lambda ts: torch.cat([t.to(f) for t in ts])  # noqa: E731
-            affine = all(m.affine for m in norms)
-            q = F.batch_norm(q, None if batch[0] else cat(m.running_mean for m in norms),
-                             None if batch[0] else cat(m.running_var for m in norms),
-                             cat(m.weight for m in norms) if affine else None,
-                             cat(m.bias for m in norms) if affine else None,
-                             batch[0], 0.0, norms[0].eps) if len({m.eps for m in norms}) == 1 else None
-        else:
-            q = None
-        if q is None:  # heads in different modes or with different eps: one call per head
-            q = (x_flat.to(f) @ w.T + b).view(n, H, dq)
-            q = torch.stack([F.batch_norm(q[:, h], None if bt else m.running_mean.to(f),
-                                          None if bt else m.running_var.to(f),
-                                          m.weight.to(f) if m.affine else None, m.bias.to(f) if m.affine else None,
-                                          bt, 0.0, m.eps) for h, (m, bt) in enumerate(zip(norms, batch))], dim=1)
-        q = q.view(n * H, dq)
-        half = dq // 2
-        # dense sub-scores, then the chosen columns: the backward is a GEMM for the keys
-        s1 = (q[:, :half] @ self.sub_keys_1.weight.to(f).T).gather(1, (ids // K).view(n * H, -1))
-        s2 = (q[:, half:] @ self.sub_keys_2.weight.to(f).T).gather(1, (ids % K).view(n * H, -1))
-        return torch.softmax(s1 + s2, dim=-1).view(ids.shape)
+        return _gate_values(x_flat, ids, [m.weight for m in self.query_projs], [m.bias for m in self.query_projs],
+                            [m.weight if m.affine else None for m in norms], [m.bias if m.affine else None for m in norms],
+                            self.sub_keys_1.weight, self.sub_keys_2.weight,
+                            [None if m.training or not m.track_running_stats else (m.running_mean, m.running_var)
+                             for m in norms], [m.eps for m in norms])
+
+    def _gate_graph(self, x_flat: torch.Tensor, ids: torch.Tensor, gates: torch.Tensor) -> torch.Tensor:
+        """A float32 [n, H, k] tensor of the gates carrying gate_path's graph (int32 ids): one
+        autograd node whose backward is one library call where that takes the operands, else
+        gate_path."""
+        ws, bn, norms = self._weight_sources(), self._bn_sources(), list(self.query_norms)
+        n, d = x_flat.shape
+        batch = norms[0].training or not norms[0].track_running_stats
+        plain = (hip.gate_grads_supported(n, d, self.num_heads, self.d_query, self.num_sub_keys, self.top_k)
+                 and all((m.training or not m.track_running_stats) == batch and m.affine and m.eps == norms[0].eps for m in norms)
+                 and all(t is not None and t.dtype == x_flat.dtype and t.device == x_flat.device and t.is_contiguous()
+                         for t in ws + bn[0::4] + bn[1::4] + ([] if batch else bn[2::4] + bn[3::4]))
+                 and x_flat.data_ptr() % 16 == 0 and ws[-1].data_ptr() % 16 == 0 and ws[-2].data_ptr() % 16 == 0
+                 # forward-mode derivatives and tracing need the torch operations
+                 and torch.autograd.forward_ad._current_level < 0 and not torch.compiler.is_compiling())
+        if not plain:
+            return self.gate_path(x_flat, ids.long())
+        wq, bq = self._packed_weights(x_flat.dtype, x_flat.device)[:2]
+        stats = None if batch else (torch.stack(bn[2::4]), torch.stack(bn[3::4]))
+        return _GatePath.apply(x_flat, ids, gates, wq, bq, stats, norms[0].eps, *ws, *bn[0::4], *bn[1::4])
 
     def forward(self, x_flat: torch.Tensor):
         """(scores [n, H, k], expert ids [n, H, k] int64) as model.py:208-254.  With autograd
         enabled the scores carry the gradient of the reference's topk + softmax."""
         with torch.no_grad():
             gates, ids = self.route(_as_input(x_flat, 2))
-        ids = ids.long()
         if _wants_grad(x_flat, self):
-            g = self.gate_path(x_flat, ids)
+            g = self._gate_graph(x_flat, ids, gates)
             gates = gates + (g - g.detach()).to(gates.dtype)
-        return gates, ids
+        return gates, ids.long()
 
 
 class EthosExpertLayer(nn.Module):
@@ -384,7 +512,7 @@ class EthosExpertLayer(nn.Module):
             with torch.no_grad():
                 gates, ids = self.router.route(x_flat)
                 seg = hip.sort_segment(ids.view(-1), self.num_experts)
-            g = self.router.gate_path(x_flat, ids.long())
+            g = self.router._gate_graph(x_flat, ids, gates)
             return _ExpertStages.apply(x_flat, g, self.expert_latents.weight, self.generation_network.net[0].weight,
                                        self.generation_network.net[2].weight, self, gates, seg)
         with torch.no_grad():

@@ -17,6 +17,9 @@
  *   ethos_apply_hidden   the same, by hidden-space reordering (no v rows)
  *   ethos_expert_forward generation + apply + scatter-back in one call (either order)
  *   ethos_expert_backward  per-pair part of the expert stages' backward
+ *   ethos_query_bn_train   query BatchNorm with batch statistics (training)
+ *   ethos_bn_coefficients  the eval-mode BatchNorm coefficients of ethos_query_proj
+ *   ethos_gate_grads     the routing gates' backward: x, query projections, BatchNorm, sub-keys
  *   ethos_expert_grads   the expert stages' backward whole: every gradient in one call
  *
  * Conventions (every entry point):
@@ -383,6 +386,58 @@ int ethos_expert_grads(const void* x, const void* dy, const void* h, const void*
                        int64_t n_tok, int32_t n_heads, int32_t top_k, int32_t d_latent, int32_t d_hidden, int32_t d_model,
                        int32_t dtype, void* workspace, size_t workspace_bytes, void* dx, float* dscores, void* dlatents,
                        void* dw1, void* dw2, void* stream);
+
+/*
+ * Query BatchNorm in training mode (model.py:200-202,216 under module.train()): per query
+ * channel (head h, channel e) of v [n_tok, n_heads, d_query] of dtype T,
+ *   q = RN_T((v - mean) / sqrt(var + eps) gamma[h][e] + beta[h][e])
+ * with the batch's mean and biased variance (float64 sums), and, when running_mean and
+ * running_var are given, running = (1 - momentum) running + momentum (mean | unbiased var),
+ * rounded to T.  With batch_mean and batch_var (host arrays of device pointers to float32
+ * [d_query]) those are taken for the batch's statistics.  gamma, beta, running_mean, running_var: host arrays of n_heads device
+ * pointers to [d_query] tensors of dtype T, read during the call only.
+ *   workspace  >= ethos_query_bn_workspace_bytes(...) bytes (scratch)
+ * Limits: n_tok >= 2, n_heads <= 32, d_query % 4 == 0; v, q and workspace 16-byte aligned.
+ */
+size_t ethos_query_bn_workspace_bytes(int64_t n_tok, int32_t n_heads, int32_t d_query);
+int ethos_query_bn_train(const void* v, int64_t n_tok, int32_t n_heads, int32_t d_query, int32_t dtype, const void* const* gamma,
+                         const void* const* beta, void* const* running_mean, void* const* running_var,
+                         const float* const* batch_mean, const float* const* batch_var, double momentum, double eps,
+                         void* workspace, size_t workspace_bytes, void* q, void* stream);
+
+/*
+ * bn_alpha and bn_beta of ethos_query_proj (float32 [n_heads, d_query]) from the modules'
+ * tensors: alpha = fp32(gamma / sqrt(var + eps)), beta = fp32(beta - mean alpha), evaluated in
+ * float64 and rounded once.  The four arrays as for ethos_query_bn_train; an array may be NULL,
+ * and so may an entry (gamma, var 1; beta, mean 0).
+ */
+int ethos_bn_coefficients(int32_t n_heads, int32_t d_query, int32_t dtype, const void* const* gamma, const void* const* beta,
+                          const void* const* running_mean, const void* const* running_var, double eps, float* alpha_out,
+                          float* beta_out, void* stream);
+
+/*
+ * Backward of the routing gates (model.py:215-234 differentiated at the chosen experts):
+ * g = softmax(q1 . K1[id / n_sub] + q2 . K2[id % n_sub]) per (token, head) row, q the per-head
+ * BatchNorm of x Wq^T + bq (batch statistics when running_mean and running_var are NULL), all
+ * recomputed in float32 from x.  From dscores float32 [n_tok, n_heads, top_k]:
+ *   dx [n_tok, d_model], dwq [n_heads, d_query, d_model], dbq, dgamma, dbeta [n_heads, d_query],
+ *   dkeys_1, dkeys_2 [n_sub, d_query / 2], all of dtype T, rounded once; deterministic.  dx and
+ *   dwq may be NULL (not computed).
+ *   x, wq, bq            as for ethos_query_proj
+ *   ids, sub-keys        as for ethos_route_topk
+ *   gamma, beta, running_mean, running_var   as for ethos_query_bn_train
+ *   workspace  >= ethos_gate_grads_workspace_bytes(...) bytes (scratch)
+ * Limits: d_model and d_query multiples of 8, d_query <= 512, n_heads <= 32, n_sub <= 1024,
+ * top_k <= 64; x, wq, the sub-keys and workspace 16-byte aligned.
+ */
+size_t ethos_gate_grads_workspace_bytes(int64_t n_tok, int32_t n_heads, int32_t top_k, int32_t d_model, int32_t d_query,
+                                        int32_t n_sub);
+int ethos_gate_grads(const void* x, const int32_t* ids, const float* dscores, const void* wq, const void* bq,
+                     const void* sub_keys_1, const void* sub_keys_2, const void* const* gamma, const void* const* beta,
+                     const void* const* running_mean, const void* const* running_var, double eps, int64_t n_tok, int32_t d_model,
+                     int32_t n_heads, int32_t d_query, int32_t n_sub, int32_t top_k, int32_t dtype, void* workspace,
+                     size_t workspace_bytes, void* dx, void* dwq, void* dbq, void* dgamma, void* dbeta, void* dkeys_1,
+                     void* dkeys_2, void* stream);
 
 #ifdef __cplusplus
 }

@@ -244,3 +244,113 @@ def test_expert_grads_entry_point(dt, n, H, k, dl, dh, d, E):
     unused = torch.ones(E, dtype=torch.bool)
     unused[uniq[:U]] = False
     assert not got[2].cpu()[unused].any()
+
+
+@pytest.mark.parametrize("dt,n,d,H,dq,K,k,batch", [
+    ("bf16", 2, 8, 1, 8, 3, 1, True), ("bf16", 37, 72, 3, 96, 37, 5, True), ("bf16", 300, 200, 2, 272, 64, 32, False),
+    ("bf16", 1100, 256, 8, 512, 512, 16, True), ("fp32", 1, 8, 2, 16, 2, 2, False), ("fp32", 129, 40, 4, 64, 65, 9, True),
+    ("fp32", 500, 256, 4, 256, 64, 8, True), ("fp32", 4200, 16, 1, 8, 5, 2, True)])
+def test_gate_grads_entry_point(dt, n, d, H, dq, K, k, batch):
+    """ethos_gate_grads against autograd in float64 through the same function, with batch and
+    with running statistics: one token, lanes of 1 to 8 query values, sub-keys shared by a
+    row's pairs, row chunks and splits off their sizes.  float32 queries of d terms, each
+    gradient a sum of up to n H k float32 terms: 3e-5 (the softmax turns a query's absolute
+    error into a relative one); bf16 results are rounded once, 2^-8.  Two runs are bit-identical."""
+    from ethos_amd import hip
+    g = torch.Generator().manual_seed(n + dq)
+    tdt = torch.bfloat16 if dt == "bf16" else torch.float32
+    rn = lambda *s: torch.randn(s, generator=g).to(tdt)  # noqa: E731
+    x, wq, bq, k1, k2 = rn(n, d), (rn(H, dq, d) / d ** 0.5).to(tdt), rn(H, dq), rn(K, dq // 2), rn(K, dq // 2)
+    k1, k2 = (k1 / dq ** 0.5).to(tdt), (k2 / dq ** 0.5).to(tdt)
+    gamma, beta = (1 + 0.1 * rn(H, dq)).to(tdt), rn(H, dq)
+    mean, var = rn(H, dq), (rn(H, dq).abs() + 0.5).to(tdt)
+    ids = torch.randint(0, K * K, (n, H, k), generator=g, dtype=torch.int32)
+    dg = torch.randn(n, H, k, generator=g)
+    assert hip.gate_grads_supported(n, d, H, dq, K, k)
+    heads = lambda t: [v.cuda() for v in t]  # noqa: E731
+    args = [t.cuda() for t in (x, ids, dg, wq, bq, k1, k2)] + [heads(gamma), heads(beta)]
+    args += [None, None] if batch else [heads(mean), heads(var)]
+    got = hip.gate_grads(*args, 1e-5)
+    again = hip.gate_grads(*args, 1e-5)
+    P = [t.double().requires_grad_(True) for t in (x, wq, bq, gamma, beta, k1, k2)]
+    X, W, B, G, Be, K1, K2 = P
+    q = torch.einsum("nd,hqd->nhq", X, W) + B
+    mu, va = (q.mean(0), q.var(0, unbiased=False)) if batch else (mean.double(), var.double())
+    q = (q - mu) / torch.sqrt(va + 1e-5) * G + Be
+    i = ids.long()
+    s = (q[:, :, None, :dq // 2] * K1[i // K]).sum(-1) + (q[:, :, None, dq // 2:] * K2[i % K]).sum(-1)
+    ref = torch.autograd.grad(torch.softmax(s, -1), P, dg.double())
+    for a, b, r, name in zip(got, again, ref, ("dx", "dwq", "dbq", "dgamma", "dbeta", "dk1", "dk2")):
+        assert torch.equal(a, b), f"{name} differs between two runs"
+        assert a.dtype == tdt and a.shape == r.shape
+        if (name == "dbq" and batch) or (k == 1):
+            assert float(a.float().abs().max()) <= 1e-5 * max(1.0, float(ref[1].abs().max())), name  # exactly zero gradient
+            continue
+        if n == 2 and batch:
+            continue  # two tokens: xhat is +-1 and every gradient through it cancels to rounding
+        assert _nerr(a, r) < (3e-5 if dt == "fp32" else 2.0 ** -8), (name, _nerr(a, r))
+
+
+@pytest.mark.parametrize("dt,n,H,dq,track", [("bf16", 2, 1, 4, True), ("fp32", 33, 3, 20, True), ("fp32", 5000, 2, 256, True),
+                                             ("bf16", 4097, 8, 256, True), ("fp32", 70, 5, 64, False)])
+def test_query_bn_train_entry_point(dt, n, H, dq, track):
+    """ethos_query_bn_train against BatchNorm in float64: normalised queries and running
+    statistics within one rounding of the layer's dtype (2^-8 and, float32, 1e-6)."""
+    from ethos_amd import hip
+    g = torch.Generator().manual_seed(n)
+    tdt = torch.bfloat16 if dt == "bf16" else torch.float32
+    v = (torch.randn(n, H, dq, generator=g) * 2 + 3).to(tdt)
+    gamma, beta, mean = (torch.randn(H, dq, generator=g).to(tdt) for _ in range(3))
+    var = torch.rand(H, dq, generator=g).to(tdt)
+    m, s = ([t.cuda().clone() for t in u] for u in (mean, var))
+    q = hip.query_bn_train(v.cuda(), [t.cuda() for t in gamma], [t.cuda() for t in beta], m if track else None,
+                           s if track else None, 0.1, 1e-5)
+    V = v.double()
+    mu, va = V.mean(0), V.var(0, unbiased=False)
+    tol = 2.0 ** -8 if dt == "bf16" else 1e-6
+    assert _nerr(q, (V - mu) / torch.sqrt(va + 1e-5) * gamma.double() + beta.double()) < tol
+    if track:
+        assert _nerr(torch.stack(m), 0.9 * mean.double() + 0.1 * mu) < tol
+        assert _nerr(torch.stack(s), 0.9 * var.double() + 0.1 * va * n / (n - 1)) < tol
+
+
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+def test_bn_coefficients_match_host(dt):
+    """The device's eval-mode BatchNorm coefficients are the host's, bit for bit."""
+    from ethos_amd import hip
+    from ethos_amd.layer import _bn_eval_coefficients
+    g = torch.Generator().manual_seed(0)
+    norms = [torch.nn.BatchNorm1d(520) for _ in range(3)]
+    for m in norms:
+        m.weight.data.copy_(torch.randn(520, generator=g))
+        m.bias.data.copy_(torch.randn(520, generator=g) * 3)
+        m.running_mean.copy_(torch.randn(520, generator=g))
+        m.running_var.copy_(torch.rand(520, generator=g) * 10.0 ** torch.randint(-6, 6, (520,), generator=g))
+        m.to(dt)
+    want = [np.stack(c) for c in zip(*[_bn_eval_coefficients(m, 520) for m in norms])]
+    d = [m.cuda() for m in norms]
+    got = hip.bn_coefficients([m.weight.detach() for m in d], [m.bias.detach() for m in d], [m.running_mean for m in d],
+                              [m.running_var for m in d], norms[0].eps, 520, dt, torch.device("cuda", 0))
+    for a, b in zip(got, want):
+        assert np.array_equal(a.cpu().numpy(), b)
+
+
+@pytest.mark.parametrize("train", [False, True])
+def test_router_second_derivative(train):
+    """The scores' gradient can be differentiated again: create_graph gives the derivative of
+    gate_path's torch operations, for x and the sub-keys."""
+    sh = SHAPES["tiny_fp32"]
+    x, sd = make_inputs(sh, signal=True)
+    m = ethos_amd.EthosExpertLayer(sh.config())
+    m.load_state_dict(sd)
+    r = m.cuda().train(train).router
+    xd = x.cuda().requires_grad_(True)
+    scores, ids = r(xd)
+    w = torch.randn(scores.shape, generator=torch.Generator().manual_seed(2)).cuda()
+    leaves_ = [xd, r.sub_keys_1.weight]
+    first = torch.autograd.grad((scores * w).sum(), leaves_, create_graph=True)
+    second = torch.autograd.grad(sum((t ** 2).sum() for t in first), leaves_)
+    ref1 = torch.autograd.grad((r.gate_path(xd, ids) * w).sum(), leaves_, create_graph=True)
+    ref2 = torch.autograd.grad(sum((t ** 2).sum() for t in ref1), leaves_)
+    for a, b in zip(first + second, ref1 + ref2):
+        assert _nerr(a, b) < 1e-5
