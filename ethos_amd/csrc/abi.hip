@@ -479,7 +479,7 @@ int ethos_token_proj(const void* x, const void* w2, const void* wut, int64_t n_t
     if (!aligned16(x) || !aligned16(w2) || (wut && !aligned16(wut)) || !aligned16(xp_out))
         return fail(ETHOS_EALIGN, "ethos_token_proj: x, w2, wut and xp_out must be 16-byte aligned");
     const int rc = ethos::launch_token_proj_out(x, w2, dtype == ETHOS_BF16 ? wut : nullptr, n_tok, d_model, d_hidden,
-                                                dtype, xp_out, (hipStream_t)stream);
+                                                dtype, xp_out, num_cus(), (hipStream_t)stream);
     if (rc < 0) return fail(ETHOS_ENULL, "ethos_token_proj: bf16 needs wut (W_u^T)");
     return hip_status(rc, "ethos_token_proj");
 }

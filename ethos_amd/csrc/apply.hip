@@ -18,6 +18,7 @@
 // them in registers; every output element is written by exactly one lane, so no
 // atomics are needed and the result is deterministic.
 #include "ethos_common.hpp"
+#include "ethos_dot64.hpp"
 #include "ethos_launch.hpp"
 #include "ethos_rows.hpp"
 #include "ethos_mfma.hpp"
@@ -30,8 +31,6 @@ namespace ethos {
 // ---------------------------------------------------------------------------------
 // Token projection xp = RN_T(x W_u), W_u[i][j] = w2[i * dh + j] for i < d.
 // ---------------------------------------------------------------------------------
-constexpr int kTpT = 64;     // tokens per tile
-constexpr int kTpC = 64;     // hidden columns per tile
 
 // bf16: W_u^T (row n = hidden column, d contiguous values) is first written to the
 // workspace by a tiled transpose of net.2.weight's first d rows, so that both GEMM
@@ -89,55 +88,35 @@ static void launch_tp_bf16(const uint16_t* x, const uint16_t* w, int64_t n_tok, 
 }
 
 // Any shape and dtype: fp64 accumulation in index order, rounded once to T.
-template <typename T>
+template <typename T, int E>
 __global__ __launch_bounds__(256) void token_proj_kernel(const T* __restrict__ x, const T* __restrict__ wu, int n_tok,
                                                          int d, int dh, T* __restrict__ xp) {
-    constexpr int KC = 32;
-    __shared__ double xs[KC][kTpT];
-    __shared__ double ws[KC][kTpC];
-    const int tid = threadIdx.x;
-    const int tx = tid & 15, ty = tid >> 4;
-    const int c0 = blockIdx.x * kTpC;
-    const int t0 = blockIdx.y * kTpT;
-    double acc[4][4];
+    constexpr int V = E / 16;
+    const int tx = threadIdx.x & 15, ty = threadIdx.x >> 4;
+    const int c0 = blockIdx.x * E, t0 = blockIdx.y * E;
+    double acc[V][V] = {};
+    dot64_tile<T, E, true>(x, wu, t0, n_tok, c0, dh, d, acc);
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = 0.0;
-    for (int k0 = 0; k0 < d; k0 += KC) {
-        const int kc = min(KC, d - k0);
-        for (int e = tid; e < kTpT * KC; e += 256) {
-            const int r = e / KC, kk = e % KC;
-            xs[kk][r] = (kk < kc && t0 + r < n_tok) ? Elem<T>::to_f64(x[(int64_t)(t0 + r) * d + k0 + kk]) : 0.0;
-        }
-        for (int e = tid; e < kTpC * KC; e += 256) {
-            const int kk = e / kTpC, r = e % kTpC;
-            ws[kk][r] = (kk < kc && c0 + r < dh) ? Elem<T>::to_f64(wu[(int64_t)(k0 + kk) * dh + c0 + r]) : 0.0;
-        }
-        __syncthreads();
-        for (int kk = 0; kk < kc; ++kk) {
-            double a[4], b[4];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) a[i] = xs[kk][ty * 4 + i];
-#pragma unroll
-            for (int j = 0; j < 4; ++j) b[j] = ws[kk][tx * 4 + j];
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int j = 0; j < 4; ++j) acc[i][j] = fma(a[i], b[j], acc[i][j]);
-        }
-        __syncthreads();
-    }
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int t = t0 + ty * 4 + i;
+    for (int i = 0; i < V; ++i) {
+        const int t = t0 + ty * V + i;
         if (t >= n_tok) continue;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int c = c0 + tx * 4 + j;
+        for (int j = 0; j < V; ++j) {
+            const int c = c0 + tx * V + j;
             if (c < dh) xp[(int64_t)t * dh + c] = Elem<T>::from_f32(Elem<T>::round64(acc[i][j]));
         }
     }
+}
+
+// out [n, m] = RN_T(x [n, d] w [d, m]) as float64 chains.
+template <typename T>
+static void launch_token_chain(const void* x, const void* w, int64_t n, int d, int m, void* out, int num_cus, hipStream_t stream) {
+    if (dot64_tile_edge(n, m, num_cus) == 64)
+        hipLaunchKernelGGL((token_proj_kernel<T, 64>), dim3((unsigned)((m + 63) / 64), (unsigned)((n + 63) / 64)), dim3(256), 0,
+                           stream, (const T*)x, (const T*)w, (int)n, d, m, (T*)out);
+    else
+        hipLaunchKernelGGL((token_proj_kernel<T, 32>), dim3((unsigned)((m + 31) / 32), (unsigned)((n + 31) / 32)), dim3(256), 0,
+                           stream, (const T*)x, (const T*)w, (int)n, d, m, (T*)out);
 }
 
 constexpr int kActGroup = 4;  // pairs whose loads are in flight together
@@ -147,15 +126,15 @@ __global__ __launch_bounds__(256) void apply_act_kernel(const T* __restrict__ xp
                                                         const int32_t* __restrict__ perm,
                                                         const int32_t* __restrict__ sorted_slot,
                                                         const T* __restrict__ gates, int64_t n_pairs, int hk, int dh,
-                                                        float* __restrict__ act) {
+                                                        int span, float* __restrict__ act) {
     typedef typename Vec16<T>::raw Raw;
     const int lane = threadIdx.x & 63;
     const int64_t wave_id = (int64_t)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int64_t n_waves = (int64_t)gridDim.x * 4;
-    const int64_t n_chunks = (n_pairs + 63) / 64;
+    const int64_t n_chunks = (n_pairs + span - 1) / span;
     for (int64_t chunk = wave_id; chunk < n_chunks; chunk += n_waves) {
-        const int64_t i0 = chunk * 64;
-        const int cnt = (int)min((int64_t)64, n_pairs - i0);
+        const int64_t i0 = chunk * span;
+        const int cnt = (int)min((int64_t)span, n_pairs - i0);
         const int my_p = lane < cnt ? perm[i0 + lane] : 0;
         const int my_s = lane < cnt ? sorted_slot[i0 + lane] : 0;
         // Groups of kActGroup consecutive sorted pairs: every h and xp row of a group is
@@ -667,11 +646,17 @@ template <typename T, int CH1>
 static void launch_act_t(const void* xp, const void* hid, const int32_t* perm, const int32_t* sorted_slot,
                          const void* gates, int64_t n_pairs, int hk, int dh, float* act, int num_cus,
                          hipStream_t stream) {
+    // pairs per wave: 64, fewer (whole groups) where that leaves SIMDs without a wave.  8,192 pairs
+    // of 512 floats: 128 waves of 64 pairs 30 us, 1,024 of 8 6.8 us
+    const int64_t waves = (int64_t)num_cus * 4;
+    int64_t span = (n_pairs + waves - 1) / waves;
+    span = (span + kActGroup - 1) / kActGroup * kActGroup;
+    span = span > 64 ? 64 : span < kActGroup ? kActGroup : span;
     const int64_t cap = (int64_t)num_cus * 16;
-    int64_t g1 = ((n_pairs + 63) / 64 + 3) / 4;
+    int64_t g1 = ((n_pairs + span - 1) / span + 3) / 4;
     g1 = g1 > cap ? cap : (g1 < 1 ? 1 : g1);
     hipLaunchKernelGGL((apply_act_kernel<T, CH1>), dim3((unsigned)g1), dim3(256), 0, stream, (const T*)xp,
-                       (const T*)hid, perm, sorted_slot, (const T*)gates, n_pairs, hk, dh, act);
+                       (const T*)hid, perm, sorted_slot, (const T*)gates, n_pairs, hk, dh, (int)span, act);
 }
 
 template <typename T, int CH2>
@@ -812,10 +797,9 @@ size_t apply_workspace_bytes(int64_t n_tok, int H, int k, int dh, int dtype) {
 // `wut_in` (bf16, may be null): W_u^T [dh, d] prepared by the caller; otherwise it is
 // transposed into the workspace here.
 static void launch_token_proj(const void* x, const void* w2, const void* wut_in, int64_t n_tok, int H, int k, int d,
-                              int dh, int dtype, void* ws, hipStream_t stream) {
+                              int dh, int dtype, void* ws, int num_cus, hipStream_t stream) {
     const size_t eb = dtype == kBF16 ? 2 : 4;
     void* xp = ws;
-    const dim3 tgrid((unsigned)((dh + kTpC - 1) / kTpC), (unsigned)((n_tok + kTpT - 1) / kTpT));
     if (dtype == kBF16 && d % kTpK == 0 && dh % 8 == 0) {
         const uint16_t* wut = static_cast<const uint16_t*>(wut_in);
         if (wut == nullptr) {
@@ -826,18 +810,16 @@ static void launch_token_proj(const void* x, const void* w2, const void* wut_in,
         }
         launch_tp_bf16((const uint16_t*)x, (const uint16_t*)wut, n_tok, d, dh, (uint16_t*)xp, stream);
     } else if (dtype == kBF16)
-        hipLaunchKernelGGL(token_proj_kernel<uint16_t>, tgrid, dim3(256), 0, stream, (const uint16_t*)x,
-                           (const uint16_t*)w2, (int)n_tok, d, dh, (uint16_t*)xp);
+        launch_token_chain<uint16_t>(x, w2, n_tok, d, dh, xp, num_cus, stream);
     else
-        hipLaunchKernelGGL(token_proj_kernel<float>, tgrid, dim3(256), 0, stream, (const float*)x, (const float*)w2,
-                           (int)n_tok, d, dh, (float*)xp);
+        launch_token_chain<float>(x, w2, n_tok, d, dh, xp, num_cus, stream);
 }
 
 int launch_token_proj_out(const void* x, const void* w2, const void* wut, int64_t n_tok, int d, int dh, int dtype,
-                          void* xp, hipStream_t stream) {
+                          void* xp, int num_cus, hipStream_t stream) {
     // the bf16 MFMA form reads W_u^T; without it the kernel would transpose into scratch
     if (dtype == kBF16 && d % kTpK == 0 && dh % 8 == 0 && wut == nullptr) return -1;
-    launch_token_proj(x, w2, wut, n_tok, 1, 1, d, dh, dtype, xp, stream);
+    launch_token_proj(x, w2, wut, n_tok, 1, 1, d, dh, dtype, xp, num_cus, stream);
     return (int)hipGetLastError();
 }
 
@@ -851,7 +833,7 @@ int launch_apply(const void* x, const void* w2, const void* hid, const void* v, 
                         ? static_cast<unsigned char*>(ws) + headbuf_offset(n_tok, H, k, dh, eb, dtype)
                         : nullptr;
     if (apply_chunks(dh, dtype) > 8 || apply_chunks(d, dtype) > 8) return -1;
-    launch_token_proj(x, w2, nullptr, n_tok, H, k, d, dh, dtype, ws, stream);
+    launch_token_proj(x, w2, nullptr, n_tok, H, k, d, dh, dtype, ws, num_cus, stream);
     launch_act(xp, hid, perm, sorted_slot, nullptr, nullptr, nullptr, gates, n_tok * H * k, H * k, dh, dtype, act,
                num_cus, stream);
     launch_scatter(v, pair_slot, act, n_tok, H, k, d, dtype, headbuf, out, num_cus, stream);
@@ -896,7 +878,7 @@ int launch_apply_hidden(const void* x, const void* w2, const void* hid, const in
     void* xp = ws;
     float* act = reinterpret_cast<float*>(static_cast<unsigned char*>(ws) + align256((size_t)n_tok * dh * eb));
     if (apply_chunks(dh, dtype) > 8) return -1;
-    launch_token_proj(x, w2, nullptr, n_tok, H, k, d, dh, dtype, ws, stream);
+    launch_token_proj(x, w2, nullptr, n_tok, H, k, d, dh, dtype, ws, num_cus, stream);
     launch_act(xp, hid, perm, sorted_slot, nullptr, nullptr, nullptr, gates, n_tok * H * k, H * k, dh, dtype, act,
                num_cus, stream);
     return launch_hidden_tail(w2, hid, pair_slot, act, n_tok, H, k, d, dh, dtype, ws, out, num_cus, stream);
@@ -932,16 +914,13 @@ static int launch_hidden_tail(const void* w2, const void* hid, const int32_t* pa
     // float64-accumulating projection
     unsigned char* wvt = hs + align256((size_t)n_tok * dh * eb);
     const dim3 tg((unsigned)((dh + 31) / 32), (unsigned)((d + 31) / 32));
-    const dim3 pg((unsigned)((d + kTpC - 1) / kTpC), (unsigned)((n_tok + kTpT - 1) / kTpT));
     if (dtype == kBF16) {
         hipLaunchKernelGGL(transpose_kernel<uint16_t>, tg, dim3(256), 0, stream, (const uint16_t*)wv, d, dh,
                            (uint16_t*)wvt);
-        hipLaunchKernelGGL(token_proj_kernel<uint16_t>, pg, dim3(256), 0, stream, (const uint16_t*)hs,
-                           (const uint16_t*)wvt, (int)n_tok, dh, d, (uint16_t*)out);
+        launch_token_chain<uint16_t>(hs, wvt, n_tok, dh, d, out, num_cus, stream);
     } else {
         hipLaunchKernelGGL(transpose_kernel<float>, tg, dim3(256), 0, stream, (const float*)wv, d, dh, (float*)wvt);
-        hipLaunchKernelGGL(token_proj_kernel<float>, pg, dim3(256), 0, stream, (const float*)hs, (const float*)wvt,
-                           (int)n_tok, dh, d, (float*)out);
+        launch_token_chain<float>(hs, wvt, n_tok, dh, d, out, num_cus, stream);
     }
     return (int)hipGetLastError();
 }
@@ -1003,7 +982,7 @@ int launch_expert_forward(const void* x, const void* latents, int64_t n_experts,
     // the routing ran)
     void* xp = xp_in ? const_cast<void*>(xp_in) : ws;
     float* act = reinterpret_cast<float*>(static_cast<unsigned char*>(ws) + align256((size_t)n_tok * dh * eb));
-    if (!xp_in) launch_token_proj(x, w2, wut, n_tok, H, k, d, dh, dtype, ws, stream);
+    if (!xp_in) launch_token_proj(x, w2, wut, n_tok, H, k, d, dh, dtype, ws, num_cus, stream);
     stage_mark(stream);
     // the hidden rows, with the activations of every tile of at most kActFusedCap pairs
     // computed while its rows are in LDS; then the activation kernel for the rest (the

@@ -436,7 +436,7 @@ int launch_expert_grads(const void* x, const void* dy, const void* hid, const vo
 
     g = Gemm{};  // dpre = gelu'(z W1) dh, in place of dh
     g.a = latents, g.lda = dl, g.a_rows = uniq, g.b = w1, g.ldb = dl, g.c = dhs, g.ldc = dh;
-    g.m = max_u, g.n = dh, g.k = dl, g.dyn = n_unique, g.gelu_grad = true;
+    g.m = max_u, g.n = dh, g.k = dl, g.dyn = n_unique, g.epilogue = kGemmGeluGrad;
     if ((rc = launch_gemm(bf ? kGemmBK_BK : kGemmFK_FK, g, num_cus, stream))) return rc;
 
     g = Gemm{};  // d latents: dpre W1^T into the unique experts' rows

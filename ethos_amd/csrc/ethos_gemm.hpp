@@ -17,6 +17,7 @@ struct Gemm {
     void* c = nullptr;
     const void* bias = nullptr;        // [n] of B's type (not with split > 1)
     const int32_t* a_rows = nullptr;   // K-stored A: row m of A is row a_rows[m] of `a`
+    int64_t a_limit = INT64_MAX;       // an a_rows entry outside [0, a_limit) is a row of zeros
     const int32_t* b_rows = nullptr;   // R-stored B: row k of B is row b_rows[k] of `b`
     const int32_t* c_rows = nullptr;   // row m of C is row c_rows[m] of `c`
     const int32_t* dyn = nullptr;      // device count: m (or, dyn_k, k) is min(m, *dyn)
@@ -27,9 +28,15 @@ struct Gemm {
     bool dyn_k = false;
     bool out_bf16 = false;             // C is bf16 (rounded to nearest even), else float32
     bool transposed = false;           // C is stored [n][m], ldc its row length
-    bool gelu_grad = false;            // C[m][n] = gelu'(sum) * C[m][n] (float32, in place)
+    int epilogue = 0;                  // kGemmPlain, or on the sum (alpha, bias, bf16 unused):
     int split = 1;                     // reduction split over this many workgroups per tile:
     float* part = nullptr;             // [split][m][n] (or [n][m]) float32 partial sums
+};
+
+enum GemmEpilogue {
+    kGemmPlain,
+    kGemmGelu,      // C = gelu(sum)
+    kGemmGeluGrad,  // C = gelu'(sum) C, in place
 };
 
 enum GemmForm {

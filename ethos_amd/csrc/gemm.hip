@@ -1,11 +1,12 @@
-// Float32 matrix products of the training path on the bf16 matrix cores.
+// Float32 matrix products (training path, float32 generator) on the bf16 matrix cores.
 //
 // A float32 operand is split exactly into three bf16 values x = hi + mid + lo (8 significant
-// bits each, truncated, 24 in all), so that its product with a bf16 operand is three bf16
-// MFMAs whose products are exact in float32; two float32 operands take the six products down
-// to 2^-24 of the result (the three left out are below 2^-32 of it).  The sums are float32,
+// bits each, 24 in all), so that its product with a bf16 operand is three bf16 MFMAs whose
+// products are exact in float32; two float32 operands take the six products down to 2^-16 of
+// the result (the three left out are about 2^-26 of it, of either sign).  The sums are float32,
 // as in a float32 GEMM; the bf16 MFMAs run at 16 times the float32 MFMAs' rate, so three of
-// them cost a fifth of one float32 product.
+// them cost a fifth of one float32 product.  Error against float64 (k = 128 | 512, two float32
+// operands): 1.7e-7 | 3.5e-7, by float32 MFMAs 2.1e-7 | 4.0e-7.
 //
 // What bounds it: at these shapes (n or k of 128 to 2,048) a step's loads, which are waited for
 // before the step's products.  So many workgroups per CU rather than many steps in flight per
@@ -30,18 +31,19 @@ namespace {
 constexpr int kGemmK = 32;      // reduction step
 constexpr int kGemmThreads = 256;
 
-// Two float32 values -> their three bf16 planes, one packed word each (a low, b high).  An
-// infinity keeps its remainders at zero; a NaN leaves one in the second plane.
+// Two float32 values -> their three bf16 planes, one packed word each (a low, b high): the upper
+// half (truncated, so that no finite value becomes an infinity), then the remainder and what is
+// left of it, both to nearest, so that the products left out have either sign (all truncated,
+// they would add up to 2^-23 of the result).  An infinity keeps its remainders at zero; a NaN
+// leaves one in the second plane.
 __device__ __forceinline__ void split3(float a, float b, uint32_t& hi, uint32_t& mid, uint32_t& lo) {
     const uint32_t ua = __float_as_uint(a), ub = __float_as_uint(b);
     hi = __builtin_amdgcn_perm(ub, ua, 0x07060302u);
     float ra = a - __uint_as_float(ua & 0xffff0000u), rb = b - __uint_as_float(ub & 0xffff0000u);
     ra = __builtin_isinf(a) ? 0.0f : ra;
     rb = __builtin_isinf(b) ? 0.0f : rb;
-    const uint32_t va = __float_as_uint(ra), vb = __float_as_uint(rb);
-    mid = __builtin_amdgcn_perm(vb, va, 0x07060302u);
-    const float sa = ra - __uint_as_float(va & 0xffff0000u), sb = rb - __uint_as_float(vb & 0xffff0000u);
-    lo = __builtin_amdgcn_perm(__float_as_uint(sb), __float_as_uint(sa), 0x07060302u);
+    mid = pack_bf16x2(ra, rb);
+    lo = pack_bf16x2(ra - __uint_as_float(mid << 16), rb - __uint_as_float(mid & 0xffff0000u));
 }
 
 // 16-byte piece `c` of LDS row `row`, in bf16 elements.
@@ -71,14 +73,17 @@ template <typename T, bool IDX, int ROWS> struct Tile<T, true, IDX, ROWS> {
     static constexpr int W = sizeof(T) / 2;  // 16-byte loads per piece
     const T* src[N];
     uint4 v[N][W];
-    __device__ __forceinline__ void init(const void* base, int64_t ld, const int32_t* rows, int64_t row0, int64_t n_rows,
-                                         int64_t k0, int tid) {
+    bool ok[N];  // IDX: the index is a row
+    __device__ __forceinline__ void init(const void* base, int64_t ld, const int32_t* rows, int64_t limit, int64_t row0,
+                                         int64_t n_rows, int64_t k0, int tid) {
 #pragma unroll
         for (int i = 0; i < N; ++i) {
             const int q = tid + i * kGemmThreads;
             int64_t r = row0 + (q >> 2);
             r = r < n_rows ? r : n_rows - 1;
             if (IDX) r = rows[r];
+            ok[i] = !IDX || (r >= 0 && r < limit);
+            r = ok[i] ? r : 0;
             src[i] = (const T*)base + r * ld + k0 + (q & 3) * 8;
         }
     }
@@ -92,10 +97,10 @@ template <typename T, bool IDX, int ROWS> struct Tile<T, true, IDX, ROWS> {
             for (int w = 0; w < W; ++w) v[i][w] = p[w];
             src[i] += kGemmK;
         }
-        if (left < kGemmK) {
+        if (IDX || left < kGemmK) {
 #pragma unroll
             for (int i = 0; i < N; ++i)
-                if (((tid + i * kGemmThreads) & 3) * 8 >= left)
+                if (!ok[i] || ((tid + i * kGemmThreads) & 3) * 8 >= left)
 #pragma unroll
                     for (int w = 0; w < W; ++w) v[i][w] = make_uint4(0, 0, 0, 0);
         }
@@ -126,8 +131,8 @@ template <typename T, bool IDX, int ROWS> struct Tile<T, false, IDX, ROWS> {
     const int32_t* rows;
     int64_t ld;
     uint32_t v[N][8];
-    __device__ __forceinline__ void init(const void* base, int64_t l, const int32_t* rws, int64_t row0, int64_t n_rows,
-                                         int64_t k0, int tid) {
+    __device__ __forceinline__ void init(const void* base, int64_t l, const int32_t* rws, int64_t /*limit*/, int64_t row0,
+                                         int64_t n_rows, int64_t k0, int tid) {
         ld = l;
         rows = IDX ? rws + k0 : nullptr;
 #pragma unroll
@@ -251,8 +256,8 @@ __global__ __launch_bounds__(kGemmThreads, (BM > 64 ? (sizeof(TB) == 4 ? 3 : 4) 
     if (kb < ke) {
         Tile<TA, AK, IDX && AK, BM> ta;
         Tile<TB, BK, IDX && !BK, BN> tb;
-        ta.init(p.a, p.lda, p.a_rows, m0, m, kb, tid);
-        tb.init(p.b, p.ldb, p.b_rows, n0, p.n, kb, tid);
+        ta.init(p.a, p.lda, p.a_rows, p.a_limit, m0, m, kb, tid);
+        tb.init(p.b, p.ldb, p.b_rows, INT64_MAX, n0, p.n, kb, tid);
         int64_t left = ke - kb;
         ta.load(left < kGemmK ? (int)left : kGemmK, tid);
         tb.load(left < kGemmK ? (int)left : kGemmK, tid);
@@ -311,7 +316,7 @@ __global__ __launch_bounds__(kGemmThreads, (BM > 64 ? (sizeof(TB) == 4 ? 3 : 4) 
         for (int i = 0; i < MI; ++i) {
             const int64_t mb = m0 + wm + i * 32;
             float aux[16];
-            if (p.gelu_grad) {
+            if (p.epilogue == kGemmGeluGrad) {
                 // all sixteen requested before any is used
 #pragma unroll
                 for (int g = 0; g < 16; ++g) {
@@ -331,7 +336,8 @@ __global__ __launch_bounds__(kGemmThreads, (BM > 64 ? (sizeof(TB) == 4 ? 3 : 4) 
                 }
                 const int64_t row = p.c_rows ? p.c_rows[mm] : mm;
                 const int64_t at = p.transposed ? n * p.ldc + row : row * p.ldc + n;
-                if (p.gelu_grad) ((float*)p.c)[at] = gelu_erf_grad(v) * aux[g];
+                if (p.epilogue == kGemmGeluGrad) ((float*)p.c)[at] = gelu_erf_grad(v) * aux[g];
+                else if (p.epilogue == kGemmGelu) ((float*)p.c)[at] = gelu_erf(v);
                 else if (p.out_bf16) ((uint16_t*)p.c)[at] = f32_to_bf16_bits(__builtin_fmaf(p.alpha, v, bias));
                 else ((float*)p.c)[at] = __builtin_fmaf(p.alpha, v, bias);
             }

@@ -11,63 +11,29 @@
 #pragma clang fp contract(off)
 
 #include "ethos_common.hpp"
+#include "ethos_dot64.hpp"
 #include "ethos_launch.hpp"
 #include "ethos_mfma.hpp"
 
 namespace ethos {
 
-constexpr int kQpTM = 64;   // tokens per tile
-constexpr int kQpTN = 64;   // output columns (h*dq + o) per tile
-constexpr int kQpKC = 32;   // reduction chunk staged in LDS
-
-template <typename T>
+template <typename T, int E>
 __global__ __launch_bounds__(256) void qproj_kernel(const T* __restrict__ x, const T* __restrict__ w,
                                                     const T* __restrict__ bias, const float* __restrict__ alpha,
                                                     const float* __restrict__ beta, int n_tok, int d, int ncols,
                                                     T* __restrict__ q) {
-    __shared__ double xs[kQpKC][kQpTM];
-    __shared__ double ws[kQpKC][kQpTN];
-    const int tid = threadIdx.x;
-    const int tx = tid & 15, ty = tid >> 4;
-    const int c0 = blockIdx.x * kQpTN;
-    const int t0 = blockIdx.y * kQpTM;
-
-    double acc[4][4];
+    constexpr int V = E / 16;
+    const int tx = threadIdx.x & 15, ty = threadIdx.x >> 4;
+    const int c0 = blockIdx.x * E, t0 = blockIdx.y * E;
+    double acc[V][V] = {};
+    dot64_tile<T, E, false>(x, w, t0, n_tok, c0, ncols, d, acc);
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = 0.0;
-
-    for (int k0 = 0; k0 < d; k0 += kQpKC) {
-        const int kc = min(kQpKC, d - k0);
-        for (int e = tid; e < kQpTM * kQpKC; e += 256) {
-            const int r = e / kQpKC, kk = e % kQpKC;
-            const bool kin = kk < kc;
-            xs[kk][r] = (kin && t0 + r < n_tok) ? Elem<T>::to_f64(x[(int64_t)(t0 + r) * d + k0 + kk]) : 0.0;
-            ws[kk][r] = (kin && c0 + r < ncols) ? Elem<T>::to_f64(w[(int64_t)(c0 + r) * d + k0 + kk]) : 0.0;
-        }
-        __syncthreads();
-        for (int kk = 0; kk < kc; ++kk) {
-            double a[4], b[4];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) a[i] = xs[kk][ty * 4 + i];
-#pragma unroll
-            for (int j = 0; j < 4; ++j) b[j] = ws[kk][tx * 4 + j];
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int j = 0; j < 4; ++j) acc[i][j] = fma(a[i], b[j], acc[i][j]);
-        }
-        __syncthreads();
-    }
-
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int t = t0 + ty * 4 + i;
+    for (int i = 0; i < V; ++i) {
+        const int t = t0 + ty * V + i;
         if (t >= n_tok) continue;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int c = c0 + tx * 4 + j;
+        for (int j = 0; j < V; ++j) {
+            const int c = c0 + tx * V + j;
             if (c >= ncols) continue;
             const double lin = acc[i][j] + Elem<T>::to_f64(bias[c]);
             const float ql = Elem<T>::round64(lin);
@@ -75,6 +41,13 @@ __global__ __launch_bounds__(256) void qproj_kernel(const T* __restrict__ x, con
             q[(int64_t)t * ncols + c] = Elem<T>::from_f32(qb);
         }
     }
+}
+
+template <typename T, int E>
+static void launch_qproj_chain(const void* x, const void* w, const void* b, const float* alpha, const float* beta, int64_t n_tok,
+                               int d, int ncols, void* q, hipStream_t stream) {
+    hipLaunchKernelGGL((qproj_kernel<T, E>), dim3((ncols + E - 1) / E, (unsigned)((n_tok + E - 1) / E)), dim3(256), 0, stream,
+                       (const T*)x, (const T*)w, (const T*)b, alpha, beta, (int)n_tok, d, ncols, (T*)q);
 }
 
 // ---------------------------------------------------------------------------------
@@ -798,13 +771,13 @@ int launch_qproj(const void* x, const void* w, const void* prepared, const void*
         }
         return (int)hipGetLastError();
     }
-    dim3 grid((ncols + kQpTN - 1) / kQpTN, (unsigned)((n_tok + kQpTM - 1) / kQpTM));
+    const bool wide = dot64_tile_edge(n_tok, ncols, num_cus) == 64;
     if (dtype == kBF16)
-        hipLaunchKernelGGL(qproj_kernel<uint16_t>, grid, dim3(256), 0, stream, (const uint16_t*)x,
-                           (const uint16_t*)w, (const uint16_t*)b, alpha, beta, (int)n_tok, d, ncols, (uint16_t*)q);
+        wide ? launch_qproj_chain<uint16_t, 64>(x, w, b, alpha, beta, n_tok, d, ncols, q, stream)
+             : launch_qproj_chain<uint16_t, 32>(x, w, b, alpha, beta, n_tok, d, ncols, q, stream);
     else
-        hipLaunchKernelGGL(qproj_kernel<float>, grid, dim3(256), 0, stream, (const float*)x, (const float*)w,
-                           (const float*)b, alpha, beta, (int)n_tok, d, ncols, (float*)q);
+        wide ? launch_qproj_chain<float, 64>(x, w, b, alpha, beta, n_tok, d, ncols, q, stream)
+             : launch_qproj_chain<float, 32>(x, w, b, alpha, beta, n_tok, d, ncols, q, stream);
     return (int)hipGetLastError();
 }
 

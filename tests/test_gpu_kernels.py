@@ -708,3 +708,48 @@ def test_sort_segment_token_proj_matches_separate_calls(n_tok, H, k, d, dh, E, d
         assert torch.equal(seg[key], seg_ref[key]), key
     assert torch.equal(seg["uniq"][:U], seg_ref["uniq"][:U]) and torch.equal(seg["seg_off"][:U + 1], seg_ref["seg_off"][:U + 1])
     assert torch.equal(xp, xp_ref)
+
+
+@pytest.mark.parametrize("n,d,cols", [(1, 4, 4), (33, 36, 68), (64, 100, 64), (130, 256, 192)])
+def test_chain_tiles_agree(n, d, cols):
+    """The float32 projections' float64 chains do not depend on the tile edge: a batch tiled by 64
+    (enough tiles for every CU) and its first n rows tiled by 32 give the same bits, and both are
+    the float64 dot product rounded once (a chain of d fused steps is within d 2^-53 of it)."""
+    from ethos_amd import hip
+    g = torch.Generator().manual_seed(n + d)
+    big = 64 * ((256 * 64) // max(64, cols) + 8)  # at least 256 tiles of 64
+    x, w, b = torch.randn(big, d, generator=g), torch.randn(1, cols, d, generator=g), torch.randn(1, cols, generator=g)
+    one, zero = torch.ones(1, cols).cuda(), torch.zeros(1, cols).cuda()
+    xd, wd, bd = x.cuda(), w.cuda(), b.cuda()
+    wide = hip.query_proj(xd, wd, bd, one, zero)
+    small = hip.query_proj(xd[:n].contiguous(), wd, bd, one, zero)
+    assert torch.equal(wide[:n], small)
+    ref = (x[:n].double() @ w[0].double().T + b.double()).float()
+    assert float((small.cpu().view(n, cols) - ref).abs().max()) <= 2.0 ** -23 * float(ref.abs().max())
+    wu = torch.randn(2 * d, cols, generator=g)
+    tw = hip.token_proj(xd, wu.cuda())
+    ts = hip.token_proj(xd[:n].contiguous(), wu.cuda())
+    assert torch.equal(tw[:n], ts)
+    ref = (x[:n].double() @ wu[:d].double()).float()
+    assert float((ts.cpu() - ref).abs().max()) <= 2.0 ** -23 * float(ref.abs().max())
+
+
+@pytest.mark.parametrize("U,max_u,E,dl,dh,d", [(1, 1, 5, 8, 32, 32), (63, 70, 200, 24, 96, 160), (700, 900, 5000, 128, 512, 256)])
+def test_generate_fp32_products(U, max_u, E, dl, dh, d):
+    """float32 generation against float64 on the stored hidden rows (sums of up to 512 float32
+    terms: 1e-6), with fewer unique experts than rows, rows past U untouched and an id outside
+    the table read as a row of zeros."""
+    from ethos_amd import hip
+    g = torch.Generator().manual_seed(U)
+    lat, w1, w2 = torch.randn(E, dl, generator=g), torch.randn(dh, dl, generator=g) / dl ** 0.5, torch.randn(2 * d, dh, generator=g) / dh ** 0.5
+    uniq = torch.randperm(E, generator=g)[:min(E, max_u)].to(torch.int32)
+    uniq[U // 2] = E + 3
+    n_u = torch.tensor([U], dtype=torch.int32).cuda()
+    h, v = hip.generate(lat.cuda(), uniq.cuda(), n_u, uniq.numel(), w1.cuda(), w2.cuda())
+    z = torch.where((uniq < E)[:, None], lat[uniq.long().clamp(max=E - 1)], torch.zeros(()))[:U].double()
+    ref = torch.nn.functional.gelu(z @ w1.double().T)
+    got = h[:U].cpu().double()
+    assert float((got - ref).norm()) <= 1e-6 * float(ref.norm()) + 1e-30
+    assert not got[U // 2].any()
+    vr = got @ w2[d:].double().T
+    assert float((v[:U].cpu().double() - vr).norm()) <= 1e-6 * float(vr.norm()) + 1e-30
