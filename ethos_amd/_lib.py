@@ -21,6 +21,7 @@ _vp = ctypes.c_void_p
 _i64 = ctypes.c_int64
 _i32 = ctypes.c_int32
 _sz = ctypes.c_size_t
+_f32 = ctypes.c_float
 _f64 = ctypes.c_double
 
 # name -> (restype, argtypes); mirrors include/ethos_hip.h
@@ -51,6 +52,10 @@ SIGNATURES = {
     "ethos_expert_backward_workspace_bytes": (_sz, [_i64, _i32, _i32, _i32]),
     "ethos_expert_backward": (ctypes.c_int, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i32, _i32, _i32, _i32, _vp,
                                              _sz, _vp, _vp, _vp, _vp, _vp]),
+    "ethos_rms_norm": (ctypes.c_int, [_vp, _i64, _vp, _i64, _i32, _f32, _i32, _vp, _vp]),
+    "ethos_swiglu": (ctypes.c_int, [_vp, _i64, _i32, _i32, _vp, _vp]),
+    "ethos_mla_attention_workspace_bytes": (_sz, [_i64, _i64]),
+    "ethos_mla_attention": (ctypes.c_int, [_vp, _vp, _vp, _i64, _vp, _vp, _i64, _i64] + [_i32] * 5 + [_f32, _vp, _sz, _vp, _vp]),
     "ethos_query_bn_workspace_bytes": (_sz, [_i64, _i32, _i32]),
     "ethos_query_bn_train": (ctypes.c_int, [_vp, _i64, _i32, _i32, _i32] + [_vp] * 6 + [_f64, _f64, _vp, _sz, _vp, _vp]),
     "ethos_bn_coefficients": (ctypes.c_int, [_i32, _i32, _i32, _vp, _vp, _vp, _vp, _f64, _vp, _vp, _vp]),

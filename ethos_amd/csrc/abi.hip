@@ -698,4 +698,61 @@ int ethos_gate_grads(const void* x, const int32_t* ids, const float* dscores, co
                       "ethos_gate_grads");
 }
 
+int ethos_rms_norm(const void* x, int64_t ldx, const void* weight, int64_t rows, int32_t d, float eps, int32_t dtype, void* y,
+                   void* stream) {
+    g_err[0] = 0;
+    if (!dtype_ok(dtype)) return fail(ETHOS_EDTYPE, "ethos_rms_norm: unknown dtype %d", dtype);
+    const int vec = dtype == ETHOS_BF16 ? 8 : 4;
+    if (rows < 0 || rows > INT32_MAX || d <= 0 || ldx < d) return fail(ETHOS_ESIZE, "ethos_rms_norm: bad sizes");
+    if (d % vec || ldx % vec || d > 512 * vec)
+        return fail(ETHOS_EUNSUPPORTED, "ethos_rms_norm: d and ldx must be multiples of %d, d <= %d", vec, 512 * vec);
+    if (rows == 0) return 0;
+    if (!x || !weight || !y) return fail(ETHOS_ENULL, "ethos_rms_norm: null pointer");
+    if (!aligned16(x) || !aligned16(weight) || !aligned16(y))
+        return fail(ETHOS_EALIGN, "ethos_rms_norm: x, weight and y must be 16-byte aligned");
+    return hip_status(ethos::launch_rms_norm(x, ldx, weight, rows, d, eps, dtype, y, (hipStream_t)stream), "ethos_rms_norm");
+}
+
+int ethos_swiglu(const void* gate_up, int64_t rows, int32_t d, int32_t dtype, void* out, void* stream) {
+    g_err[0] = 0;
+    if (!dtype_ok(dtype)) return fail(ETHOS_EDTYPE, "ethos_swiglu: unknown dtype %d", dtype);
+    const int vec = dtype == ETHOS_BF16 ? 8 : 4;
+    if (rows < 0 || d <= 0) return fail(ETHOS_ESIZE, "ethos_swiglu: bad sizes");
+    if (d % vec) return fail(ETHOS_EUNSUPPORTED, "ethos_swiglu: d must be a multiple of %d", vec);
+    if (rows == 0) return 0;
+    if (!gate_up || !out) return fail(ETHOS_ENULL, "ethos_swiglu: null pointer");
+    if (!aligned16(gate_up) || !aligned16(out)) return fail(ETHOS_EALIGN, "ethos_swiglu: gate_up and out must be 16-byte aligned");
+    return hip_status(ethos::launch_swiglu(gate_up, rows, d, dtype, out, num_cus(), (hipStream_t)stream), "ethos_swiglu");
+}
+
+size_t ethos_mla_attention_workspace_bytes(int64_t n_seq, int64_t seq_len) {
+    if (n_seq <= 0 || seq_len <= 0) return 256;
+    return ethos::mla_attention_workspace_bytes(n_seq, seq_len);
+}
+
+int ethos_mla_attention(const void* q, const void* kv, const void* k_rot, int64_t k_rot_ld, const int64_t* positions,
+                        const float* rates, int64_t n_seq, int64_t seq_len, int32_t n_heads, int32_t nope, int32_t rope, int32_t v_dim,
+                        int32_t dtype, float scale, void* workspace, size_t workspace_bytes, void* out, void* stream) {
+    g_err[0] = 0;
+    if (dtype != ETHOS_BF16) return fail(ETHOS_EDTYPE, "ethos_mla_attention: bf16 only, got dtype %d", dtype);
+    if (n_seq < 0 || seq_len < 0 || n_heads <= 0 || k_rot_ld < rope) return fail(ETHOS_ESIZE, "ethos_mla_attention: bad sizes");
+    if (!ethos::mla_attention_supported(nope, rope, v_dim) || k_rot_ld % 2)
+        return fail(ETHOS_EUNSUPPORTED, "ethos_mla_attention: needs widths 64, 64, 64 (got %d, %d, %d) and an even k_rot_ld", nope,
+                    rope, v_dim);
+    if (n_seq * n_heads > INT32_MAX / 2 || seq_len > INT32_MAX / 2 ||
+        n_seq * n_heads * ((seq_len + 63) / 64) > INT32_MAX / 2 || n_seq * seq_len > INT32_MAX)
+        return fail(ETHOS_ESIZE, "ethos_mla_attention: too many rows");
+    if (n_seq == 0 || seq_len == 0) return 0;
+    if (!q || !kv || !k_rot || !positions || !rates || !workspace || !out)
+        return fail(ETHOS_ENULL, "ethos_mla_attention: null pointer");
+    const size_t need = ethos::mla_attention_workspace_bytes(n_seq, seq_len);
+    if (workspace_bytes < need)
+        return fail(ETHOS_EWORKSPACE, "ethos_mla_attention: workspace of %zu bytes, %zu needed", workspace_bytes, need);
+    if (!aligned16(q) || !aligned16(kv) || !aligned16(workspace) || !aligned16(out) || ((uintptr_t)k_rot & 3u))
+        return fail(ETHOS_EALIGN, "ethos_mla_attention: q, kv, workspace and out must be 16-byte, k_rot 4-byte aligned");
+    return hip_status(ethos::launch_mla_attention(q, kv, k_rot, k_rot_ld, positions, rates, n_seq, seq_len, n_heads, scale, workspace,
+                                                  out, num_cus(), (hipStream_t)stream),
+                      "ethos_mla_attention");
+}
+
 }  // extern "C"

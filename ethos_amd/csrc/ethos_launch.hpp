@@ -132,4 +132,13 @@ int launch_expert_forward(const void* x, const void* latents, int64_t n_experts,
                           const void* gates, int64_t n_tok, int H, int k, int dl, int dh, int d, int dtype, int order,
                           void* ws, void* hout, void* out, int num_cus, hipStream_t stream);
 
+// The language model's blocks (block.hip, attention.hip).
+int launch_rms_norm(const void* x, int64_t ldx, const void* w, int64_t rows, int d, float eps, int dtype, void* y,
+                    hipStream_t stream);
+int launch_swiglu(const void* gu, int64_t rows, int d, int dtype, void* out, int num_cus, hipStream_t stream);
+bool mla_attention_supported(int nope, int rope, int v_dim);
+size_t mla_attention_workspace_bytes(int64_t n_seq, int64_t n);
+int launch_mla_attention(const void* q, const void* kv, const void* k_rot, int64_t k_rot_ld, const int64_t* pos, const float* rate,
+                         int64_t n_seq, int64_t n, int H, float scale, void* ws, void* out, int num_cus, hipStream_t stream);
+
 }  // namespace ethos

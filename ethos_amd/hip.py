@@ -543,3 +543,82 @@ def gate_grads(x: torch.Tensor, ids: torch.Tensor, dg: torch.Tensor, wq: torch.T
                                  dx.data_ptr() if want_x else None, dw.data_ptr() if want_w else None, db.data_ptr(), dgamma.data_ptr(), dbeta.data_ptr(), dk1.data_ptr(), dk2.data_ptr(), _stream())
     check(rc, "ethos_gate_grads")
     return dx, dw, db, dgamma, dbeta, dk1, dk2
+
+
+# ----------------------------------------------------------- the language model's blocks
+def plain(*ts) -> bool:
+    """Whether a library call may stand in for torch operations on these tensors: ordinary HIP
+    tensors of one supported dtype and device, with nothing that follows the operations
+    themselves (gradients, forward-mode derivatives, autocast, tracing, transforms, modes)."""
+    t0 = ts[0]
+    if t0.dtype not in (torch.bfloat16, torch.float32) or t0.device.type != "cuda":
+        return False
+    grad = torch.is_grad_enabled()
+    for t in ts:
+        if (type(t) not in (torch.Tensor, torch.nn.Parameter) or t.dtype != t0.dtype or t.device != t0.device
+                or (grad and t.requires_grad)):
+            return False
+    return not (torch.is_autocast_enabled("cuda") or torch.compiler.is_compiling() or torch.jit.is_tracing()
+                or torch.autograd.forward_ad._current_level >= 0 or torch._C._len_torch_dispatch_stack() > 0
+                or torch._C._len_torch_function_stack() > 0 or torch._C._functorch.peek_interpreter_stack() is not None)
+
+
+def row_stride(x: torch.Tensor) -> int:
+    """Distance between the rows x[..., :] when they are evenly spaced and each contiguous, else 0."""
+    if x.is_contiguous():
+        return x.shape[-1]
+    if x.dim() < 2 or x.stride(-1) != 1:
+        return 0
+    for i in range(x.dim() - 2):
+        if x.stride(i) != x.stride(i + 1) * x.shape[i + 1]:
+            return 0
+    return x.stride(-2)
+
+
+def rms_norm(x: torch.Tensor, weight: torch.Tensor, eps: float) -> torch.Tensor | None:
+    """RMSNorm over the last dimension, or None where the kernel does not take the operands."""
+    d, vec = x.shape[-1], 16 // x.element_size()
+    ld = row_stride(x)
+    if (ld < d or ld % vec or d % vec or d > 512 * vec or weight.shape != (d,) or not weight.is_contiguous()
+            or x.numel() == 0 or x.data_ptr() % 16 or weight.data_ptr() % 16 or x.numel() // d > 2 ** 31 - 1):
+        return None
+    y = torch.empty(x.shape, dtype=x.dtype, device=x.device)
+    rc = load().ethos_rms_norm(x.data_ptr(), ld, weight.data_ptr(), x.numel() // d, d, float(eps), dtype_code(x.dtype),
+                               y.data_ptr(), _stream())
+    check(rc, "ethos_rms_norm")
+    return y
+
+
+def swiglu(gate_up: torch.Tensor) -> torch.Tensor | None:
+    """silu(gate) * up of the halves of [..., 2 d], or None where the kernel does not take it."""
+    d = gate_up.shape[-1] // 2
+    vec = 16 // gate_up.element_size()
+    if not gate_up.is_contiguous() or gate_up.shape[-1] % 2 or d % vec or gate_up.numel() == 0 or gate_up.data_ptr() % 16:
+        return None
+    out = torch.empty((*gate_up.shape[:-1], d), dtype=gate_up.dtype, device=gate_up.device)
+    rc = load().ethos_swiglu(gate_up.data_ptr(), gate_up.numel() // (2 * d), d, dtype_code(gate_up.dtype), out.data_ptr(),
+                             _stream())
+    check(rc, "ethos_swiglu")
+    return out
+
+
+def mla_attention(q: torch.Tensor, kv: torch.Tensor, k_rot: torch.Tensor, positions: torch.Tensor, rates: torch.Tensor,
+                  n_heads: int, nope: int, rope: int, v_dim: int, scale: float) -> torch.Tensor | None:
+    """Causal latent attention: q [b, n, H (nope + rope)] and k_rot [b, n, rope] before rotation,
+    kv [b, n, H (nope + v_dim)] -> [b, n, H v_dim], or None where the kernel does not take the
+    operands."""
+    b, n = q.shape[:2]
+    ld = row_stride(k_rot)
+    if (q.dtype != torch.bfloat16 or (nope, rope, v_dim) != (64, 64, 64) or b * n == 0 or not q.is_contiguous()
+            or not kv.is_contiguous() or ld < rope or ld % 2 or q.data_ptr() % 16 or kv.data_ptr() % 16 or k_rot.data_ptr() % 4
+            or positions.dtype != torch.int64 or positions.numel() != n or not positions.is_contiguous()
+            or positions.device != q.device or rates.dtype != torch.float32 or rates.device != q.device
+            or b * n_heads * ((n + 63) // 64) > 2 ** 30 or b * n > 2 ** 31 - 1):
+        return None
+    ws, ws_bytes = workspace(load().ethos_mla_attention_workspace_bytes(b, n), q.device)
+    out = torch.empty((b, n, n_heads * v_dim), dtype=q.dtype, device=q.device)
+    rc = load().ethos_mla_attention(q.data_ptr(), kv.data_ptr(), k_rot.data_ptr(), ld, positions.data_ptr(), rates.data_ptr(), b, n,
+                                    n_heads, nope, rope, v_dim, dtype_code(q.dtype), float(scale), ws.data_ptr(), ws_bytes,
+                                    out.data_ptr(), _stream())
+    check(rc, "ethos_mla_attention")
+    return out

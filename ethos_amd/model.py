@@ -16,7 +16,11 @@ How it is computed here:
     buffers, which SDPA reads through transposed views; the values sit in a buffer as
     wide as the query/key heads (zero columns beyond v_head_dim), the layout the fused
     SDPA kernels take;
-  - the dense FFN's gate and up projections run as one GEMM.
+  - the dense FFN's gate and up projections run as one GEMM;
+  - where no gradient is wanted, RMSNorm and the SwiGLU product are one HIP kernel each, and
+    the attention (rotations, scores, softmax, values) is a HIP kernel that reads the
+    projections' outputs as they are (bf16, head widths 64 + 64 and 64); under autograd, with a
+    mask, or in other shapes they are torch operations and SDPA.
 The expert layer is EthosExpertLayer (HIP kernels).  Inputs live on a HIP device.
 """
 from __future__ import annotations
@@ -28,6 +32,7 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
+from . import hip
 from .layer import EthosExpertLayer
 
 # the reference's configs/default.yaml, with the benchmarked expert-layer shape (d_query
@@ -68,6 +73,10 @@ class RMSNorm(nn.Module):
         self.eps = eps
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
+        if hip.plain(x, self.weight):
+            y = hip.rms_norm(x, self.weight, self.eps)  # one kernel, the same rounding points
+            if y is not None:
+                return y
         y = F.rms_norm(x.float(), (x.shape[-1],), eps=self.eps)
         return self.weight * y.to(x.dtype)
 
@@ -85,14 +94,18 @@ class Rotary(nn.Module):
         self.base = float(base)
         self._rate = None
 
+    def rates(self, device: torch.device) -> torch.Tensor:
+        """base^(-2i/2m), float32 [m]."""
+        if self._rate is None or self._rate.device != device:
+            # as the reciprocal of the power, the reference's float32 rounding of the
+            # frequencies (model.py:40)
+            self._rate = 1.0 / self.base ** (torch.arange(0, 2 * self.half, 2, device=device,
+                                                          dtype=torch.float32) / (2 * self.half))
+        return self._rate
+
     def rotate(self, r: torch.Tensor, positions: torch.Tensor) -> torch.Tensor:
         """r [batch, seq, ..., 2m], positions [seq] -> the rotated slice, same shape and dtype."""
-        if self._rate is None or self._rate.device != r.device:
-            # rates base^(-2i/2m) as the reciprocal of the power, the reference's float32
-            # rounding of the frequencies (model.py:40)
-            self._rate = 1.0 / self.base ** (torch.arange(0, 2 * self.half, 2, device=r.device,
-                                                          dtype=torch.float32) / (2 * self.half))
-        ang = positions.to(device=r.device, dtype=torch.float32)[:, None] * self._rate[None, :]
+        ang = positions.to(device=r.device, dtype=torch.float32)[:, None] * self.rates(r.device)[None, :]
         shape = (1, positions.numel()) + (1,) * (r.dim() - 3) + (self.half,)
         c = ang.cos().to(r.dtype).view(shape)
         s = ang.sin().to(r.dtype).view(shape)
@@ -133,8 +146,14 @@ class MLAttention(nn.Module):
         # one GEMM for both projections of the block input: [q latent | kv latent | rotary key]
         a = F.linear(x, _stacked(self, (self.q_a_proj, self.kv_a_proj_with_mqa)))
         q_lat, kv_lat, k_rot = a.split((self.q_rank, self.kv_rank, rope), dim=-1)
-        q = self.q_b_proj(self.q_a_layernorm(q_lat)).view(b, n, H, w)
-        kv = self.kv_b_proj(self.kv_a_layernorm(kv_lat)).view(b, n, H, nope + self.vdim)
+        q = self.q_b_proj(self.q_a_layernorm(q_lat))
+        kv = self.kv_b_proj(self.kv_a_layernorm(kv_lat))
+        if attention_mask is None and hip.plain(q, kv, k_rot) and pos.device == q.device:
+            # queries, keys and values read where the projections left them
+            o = hip.mla_attention(q, kv, k_rot, pos, self.rotary.rates(x.device), H, nope, rope, self.vdim, self.scale)
+            if o is not None:
+                return self.o_proj(o)
+        q, kv = q.view(b, n, H, w), kv.view(b, n, H, nope + self.vdim)
         # token-major buffers: q (rotary slice rotated), k (per-head nope part | the shared
         # rotated key), v (zero columns past v_head_dim)
         qb = torch.cat((q[..., :nope], self.rotary.rotate(q[..., nope:], pos)), dim=-1)
@@ -162,7 +181,12 @@ class FFN(nn.Module):
         self.w3 = nn.Linear(config.d_model, config.d_ffn_intermediate, bias=False)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        gate, up = F.linear(x, _stacked(self, (self.w1, self.w3))).chunk(2, dim=-1)
+        gate_up = F.linear(x, _stacked(self, (self.w1, self.w3)))
+        if hip.plain(gate_up):
+            y = hip.swiglu(gate_up)
+            if y is not None:
+                return self.w2(y)
+        gate, up = gate_up.chunk(2, dim=-1)
         return self.w2(F.silu(gate) * up)
 
 

@@ -20,6 +20,7 @@
  *   ethos_query_bn_train   query BatchNorm with batch statistics (training)
  *   ethos_bn_coefficients  the eval-mode BatchNorm coefficients of ethos_query_proj
  *   ethos_gate_grads     the routing gates' backward: x, query projections, BatchNorm, sub-keys
+ *   ethos_rms_norm, ethos_swiglu, ethos_mla_attention  the language model's blocks
  *   ethos_expert_grads   the expert stages' backward whole: every gradient in one call
  *
  * Conventions (every entry point):
@@ -438,6 +439,40 @@ int ethos_gate_grads(const void* x, const int32_t* ids, const float* dscores, co
                      int32_t n_heads, int32_t d_query, int32_t n_sub, int32_t top_k, int32_t dtype, void* workspace,
                      size_t workspace_bytes, void* dx, void* dwq, void* dbq, void* dgamma, void* dbeta, void* dkeys_1,
                      void* dkeys_2, void* stream);
+
+/*
+ * RMSNorm (model.py:19-30): y[r] = RN_T(weight RN_T(x[r] / sqrt(mean(x[r]^2) + eps))), the mean
+ * and the quotient in float32.  x: rows of d values, ldx apart; y [rows, d].
+ * Limits: d and ldx multiples of 8 (bf16) or 4 (fp32), d <= 4096 (bf16) / 2048 (fp32); 16-byte
+ * aligned pointers.
+ */
+int ethos_rms_norm(const void* x, int64_t ldx, const void* weight, int64_t rows, int32_t d, float eps, int32_t dtype, void* y,
+                   void* stream);
+
+/*
+ * The SwiGLU product (model.py:257-265): out [rows, d] = RN_T(RN_T(g / (1 + exp(-g))) u) with g and
+ * u the two halves of gate_up [rows, 2 d].  Limits: d a multiple of 8 (bf16) or 4 (fp32); 16-byte
+ * aligned pointers.
+ */
+int ethos_swiglu(const void* gate_up, int64_t rows, int32_t d, int32_t dtype, void* out, void* stream);
+
+/*
+ * Causal latent attention (model.py:118-160) of n_seq sequences of seq_len tokens, bf16:
+ *   q       [n_seq, seq_len, n_heads, nope + rope], the rotary part not yet rotated
+ *   kv      [n_seq, seq_len, n_heads, nope + v_dim], each head's key part, then its value
+ *   k_rot   [n_seq seq_len] rows of rope values, k_rot_ld apart: the shared rotary key, unrotated
+ *   positions [seq_len] int64, rates [rope / 2] float32: row t is rotated by positions[t] rates[i]
+ *   out     [n_seq, seq_len, n_heads, v_dim]
+ * softmax(scale q k) v over the keys up to the query, float32 scores and sums, the exponentials
+ * rounded to bf16 for the product with v.
+ *   workspace  >= ethos_mla_attention_workspace_bytes(...) bytes (scratch)
+ * Limits: nope, rope and v_dim 64; k_rot_ld even; q, kv, workspace and out 16-byte aligned, k_rot
+ * 4-byte.
+ */
+size_t ethos_mla_attention_workspace_bytes(int64_t n_seq, int64_t seq_len);
+int ethos_mla_attention(const void* q, const void* kv, const void* k_rot, int64_t k_rot_ld, const int64_t* positions,
+                        const float* rates, int64_t n_seq, int64_t seq_len, int32_t n_heads, int32_t nope, int32_t rope, int32_t v_dim,
+                        int32_t dtype, float scale, void* workspace, size_t workspace_bytes, void* out, void* stream);
 
 #ifdef __cplusplus
 }

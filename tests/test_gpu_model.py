@@ -141,3 +141,94 @@ def test_lm_whole_model_workload_full_size():
                             routed=(g_ref, ids_ref))
         check_out(O.to_f32(to_host(y), "bf16")[y_sub], r["out"], "bf16", nerr_max=2e-3)
         check_all_tokens(layer, xf, gates, ids_l, y, f"block {i}")
+
+
+def _attention_double(q, kv, k_rot, pos, rates, H, scale):
+    """The attention of model.py:118-160 in float64 on the bf16 operands, with the rotation's own
+    bf16 roundings (cosines, sines, products and sums)."""
+    b, n, _ = q.shape
+    ang = pos.float()[:, None] * rates
+    c, s = ang.cos().bfloat16(), ang.sin().bfloat16()
+
+    def rotate(r):
+        x, y = r[..., :32], r[..., 32:]
+        cc, ss = (t.view((1, n) + (1,) * (r.dim() - 3) + (32,)) for t in (c, s))
+        return torch.cat((x * cc - y * ss, y * cc + x * ss), -1)
+
+    Q, K = q.view(b, n, H, 128), kv.view(b, n, H, 128)
+    qq = torch.cat((Q[..., :64], rotate(Q[..., 64:])), -1)
+    kk = torch.cat((K[..., :64], rotate(k_rot).unsqueeze(2).expand(b, n, H, 64)), -1)
+    d = lambda t: t.double().permute(0, 2, 1, 3).contiguous()  # noqa: E731
+    S = (d(qq) @ d(kk).transpose(-1, -2).contiguous()) * scale
+    S = S.masked_fill(torch.ones(n, n, dtype=torch.bool, device=q.device).triu(1), float("-inf"))
+    return (torch.softmax(S, -1) @ d(K[..., 64:])).permute(0, 2, 1, 3).reshape(b, n, -1)
+
+
+@pytest.mark.parametrize("b,n,H", [(1, 1, 1), (2, 31, 3), (1, 32, 2), (3, 33, 1), (1, 63, 4), (2, 64, 2), (1, 65, 5), (2, 127, 3),
+                                   (1, 129, 2), (5, 130, 64), (1, 1371, 3)])
+def test_mla_attention_against_float64(b, n, H):
+    """The attention kernel at the edges of its tiles (32 and 64 queries, 64 keys) and both
+    workgroup sizes: exponentials and results each rounded to bf16 once (2^-9 rms each at most),
+    so 4e-3."""
+    import math
+
+    from ethos_amd import hip
+    g = torch.Generator(device="cuda").manual_seed(n)
+    rn = lambda *s: torch.randn(s, generator=g, device="cuda").bfloat16()  # noqa: E731
+    q, kv, a = rn(b, n, H * 128), rn(b, n, H * 128), rn(b, n, 70)
+    k_rot = a[..., 6:]
+    pos = torch.randperm(3 * n, generator=g, device="cuda")[:n]
+    rates = 1.0 / 10000.0 ** (torch.arange(0, 64, 2, device="cuda", dtype=torch.float32) / 64)
+    scale = 1.0 / math.sqrt(128)
+    o = hip.mla_attention(q, kv, k_rot, pos, rates, H, 64, 64, 64, scale)
+    ref = _attention_double(q, kv, k_rot, pos, rates, H, scale)
+    assert o.shape == (b, n, H * 64)
+    err = float((o.double() - ref).norm() / ref.norm())
+    assert err < 4e-3, err
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("rows,d,ld", [(1, 8, 8), (5, 72, 80), (33, 768, 1088), (4, 1000, 1000), (3, 2048, 2056)])
+def test_rms_norm_against_float64(dt, rows, d, ld):
+    """RMSNorm of strided rows: two roundings to the dtype (2^-8 and, float32, 1e-6)."""
+    from ethos_amd import hip
+    g = torch.Generator().manual_seed(d)
+    x = (torch.randn(rows, ld, generator=g) * 3).to(dt).cuda()[:, :d]
+    w = torch.randn(d, generator=g).to(dt).cuda()
+    y = hip.rms_norm(x, w, 1e-6)
+    ref = x.double() * torch.rsqrt(x.double().square().mean(-1, keepdim=True) + 1e-6) * w.double()
+    assert y.shape == x.shape and y.is_contiguous()
+    assert float((y.double() - ref).norm() / ref.norm()) < (2.0 ** -8 if dt == torch.bfloat16 else 1e-6)
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
+def test_swiglu_against_float64(dt):
+    from ethos_amd import hip
+    g = torch.Generator().manual_seed(1)
+    gu = (torch.randn(3, 7, 2 * 136, generator=g) * 4).to(dt).cuda()
+    gu[0, 0, :4] = torch.tensor([90.0, -90.0, 0.0, float("inf")])
+    gu[0, 0, 136:140] = 1.0
+    y = hip.swiglu(gu)
+    a, b = gu.double().chunk(2, -1)
+    ref = a * torch.sigmoid(a) * b
+    assert torch.isinf(y[0, 0, 3]) and y.shape == ref.shape
+    y, ref = y.double().flatten(), ref.flatten()
+    ok = torch.isfinite(ref)
+    assert float((y[ok] - ref[ok]).norm() / ref[ok].norm()) < (2.0 ** -7 if dt == torch.bfloat16 else 1e-6)
+
+
+def test_block_with_and_without_gradients_agree():
+    """A dense block under autograd (torch operations) and without (the kernels): the same
+    function to bf16 rounding, and only the first carries a graph."""
+    from ethos_amd.model import TransformerBlock, lm_config
+    torch.manual_seed(0)
+    block = TransformerBlock(lm_config(), False).cuda().bfloat16()
+    x = torch.randn(2, 97, 1024, device="cuda").bfloat16()
+    pos = torch.arange(97, device="cuda")
+    with torch.no_grad():
+        y = block(x, None, pos)
+    z = block(x, None, pos)
+    assert z.grad_fn is not None
+    z = z.detach()
+    assert y.grad_fn is None
+    assert float((y.float() - z.float()).norm() / z.float().norm()) < 1e-2
