@@ -40,10 +40,26 @@ namespace ethos {
 
 constexpr int kRtWaves = 8;                            // two workgroups per CU: four waves per SIMD
 constexpr int kRtRows = 32;                            // rows of the MFMA tile (and LDS row slots)
-// rows per wave: 4 (32 rows per workgroup) for large batches; 1 (8 rows per workgroup,
-// the MFMA tile's other rows zero) for small ones, which spreads them over 4x as many
-// workgroups and cuts each wave's sequential work by 4
-constexpr int kRtSmallRows = 4096;                     // batches up to this many rows take 1 row per wave
+// Rows per wave: 4 (32 rows per workgroup) for large batches; 1 (8 rows per workgroup, the MFMA
+// tile's other rows zero) or 2 for smaller ones, which spreads them over more workgroups and
+// cuts each wave's sequential work.  The lines follow from whole rounds of workgroups over 256
+// CUs: one row per wave fills the chip at 2,048 rows, two (two workgroups a CU) at 8,192, four at
+// 16,384, or at 8,192 where its LDS (query halves of 512 bytes) leaves room for one workgroup a
+// CU.  us, bf16, 1 | 2 | 4 rows per wave: d_query 256: 2,048 rows 19 | 27 | 40, 4,096 35 | 28 | 40,
+// 8,192 65 | 39 | 42, 16,384 127 | 71 | 57; d_query 512: 4,096 49 | 36 | 51, 12,000 135 | 79 | 95,
+// 24,576 270 | 144 | 145; float32, d_query 256: 4,096 82 | 62 | 91, 6,216 150 | 100 | 92, 12,000
+// 231 | 149 | 177, 16,384 309 | 194 | 180.
+constexpr int64_t kRtOneRows = 2048;
+constexpr int64_t kRtTwoRows = 8192;
+constexpr size_t kRtTwoPerCu = 80 * 1024;              // LDS up to which two workgroups share a CU
+inline int route_rows_per_wave(int64_t rows, size_t smem4) {
+    if (rows <= kRtOneRows) return 1;
+    if (smem4 <= kRtTwoPerCu) return rows <= kRtTwoRows ? 2 : 4;
+    // four rows in whole rounds of 8,192; two while the last round would be under 3/4 full (for
+    // many rounds that no longer matters)
+    const int64_t last = (rows - 1) % kRtTwoRows + 1;
+    return last <= kRtTwoRows * 3 / 4 && rows <= 4 * kRtTwoRows ? 2 : 4;
+}
 constexpr int kRtMaxKc = 32;                           // k_cand <= 32, top_k <= 32
 static_assert(kRtMaxKc <= kWave, "candidate lists hold one entry per lane");
 constexpr int kRtMaxK = 512;                           // sub-keys per table
@@ -299,14 +315,14 @@ __host__ __device__ inline int route_pitch(int K) {
     return (p > 3 * kWave ? p : 3 * kWave) + 4;
 }
 
-// hp: the half-parallel form (two groups of kRtWaves waves, one per query half, kRtWaves rows):
-// score rows for the workgroup's rows of both halves, both halves' staged query tiles, and the
-// second half's candidate lists handed to the first group.
-__host__ __device__ inline RouteSmem route_smem_layout(int K, int dh2, int elem_bytes, bool hp = false) {
+// rows: the workgroup's rows.  hp: the half-parallel form (two groups of kRtWaves waves, one per
+// query half, kRtWaves rows): score rows for the workgroup's rows of both halves, both halves'
+// staged query tiles, and the second half's candidate lists handed to the first group.
+__host__ __device__ inline RouteSmem route_smem_layout(int K, int dh2, int elem_bytes, int rows = kRtRows, bool hp = false) {
     RouteSmem L;
     size_t off = 0;
     L.s_off = off;
-    off += (size_t)(hp ? 2 * kRtWaves : kRtRows) * route_pitch(K) * sizeof(float);
+    off += (size_t)(hp ? 2 : 1) * rows * route_pitch(K) * sizeof(float);
     L.kn_off = off;
     off += (size_t)2 * ((K + 31) / 32) * 32 * sizeof(float);
     L.qs_off = off;
@@ -372,7 +388,7 @@ __global__ __launch_bounds__((kHP ? 2 : 1) * kRtWaves * 64, 4) void route_kernel
     const int hw = kHP ? wave / kRtWaves : 0, wv = kHP ? wave % kRtWaves : wave;
     const int gtid = kHP ? tid % (kRtWaves * 64) : tid;
     const int lrow = lane & 31, lk = (lane >> 5) * M::kKL;
-    const RouteSmem L = route_smem_layout(K, dh2, (int)sizeof(T), kHP);
+    const RouteSmem L = route_smem_layout(K, dh2, (int)sizeof(T), kRtWaves * RPW, kHP);
     const int pitch = route_pitch(K);
     const int kpad = ((K + 31) / 32) * 32;
     constexpr int kRowsWG = kRtWaves * RPW;  // rows of this workgroup (<= kRtRows)
@@ -488,7 +504,7 @@ __global__ __launch_bounds__((kHP ? 2 : 1) * kRtWaves * 64, 4) void route_kernel
                 if (kb < nkb) {
 #pragma unroll
                     for (int i = 0; i < 16; ++i)
-                        if (!kHP || mfma32_row(i, lane) < kRowsWG)  // (kHP: only the live rows have storage)
+                        if (kRowsWG == kRtRows || mfma32_row(i, lane) < kRowsWG)  // (only the live rows have storage)
                             S[mfma32_row(i, lane) * pitch + kb * 32 + lrow] = acc[c][i];
                 }
             }
@@ -538,7 +554,7 @@ __global__ __launch_bounds__((kHP ? 2 : 1) * kRtWaves * 64, 4) void route_kernel
         {
             constexpr int kLPR = kWave / RPW;
             constexpr int kN = QVecF<T>::kN;
-            static_assert(RPW == 1 || RPW == 4, "row groups of 64 or 16 lanes");
+            static_assert(RPW == 1 || RPW == 2 || RPW == 4, "row groups of 64, 32 or 16 lanes");
             const int lr = wv * RPW + lane / kLPR;
             const T* qs = reinterpret_cast<const T*>(qsb + (size_t)lr * L.qs_pitch);
             for (int i = (lane % kLPR) * kN; i < dh2; i += kLPR * kN) {
@@ -554,6 +570,7 @@ __global__ __launch_bounds__((kHP ? 2 : 1) * kRtWaves * 64, 4) void route_kernel
                 sq_row += dpp_f32<kDppXor2>(sq_row);
                 sq_row += dpp_f32<kDppRowHalfMirror>(sq_row);
                 sq_row += dpp_f32<kDppRowMirror>(sq_row);
+                if constexpr (RPW == 2) sq_row += __uint_as_float(xor_lane_u32(__float_as_uint(sq_row), 16));
             }
         }
 #pragma unroll
@@ -867,12 +884,15 @@ static void launch_route_t(const void* q, const void* k1, const void* k2, const 
                            int64_t rows, int dq, int K, int top_k, int kc, void* gates, int32_t* ids,
                            hipStream_t stream) {
     const int dh2 = dq / 2;
-    const bool small = rows <= kRtSmallRows;
-    const int per_wg = kRtWaves * (small ? 1 : 4);
-    const dim3 grid((unsigned)((rows + per_wg - 1) / per_wg));
-    if (small)  // one row per wave, the two query halves in parallel
+    const int rpw = route_rows_per_wave(rows, route_smem_bytes(K, dh2, (int)sizeof(T)));
+    const dim3 grid((unsigned)((rows + kRtWaves * rpw - 1) / (kRtWaves * rpw)));
+    if (rpw == 1)  // one row per wave, the two query halves in parallel
         hipLaunchKernelGGL((route_kernel<T, 1, true, kPrep>), grid, dim3(2 * kRtWaves * 64),
-                           route_smem_layout(K, dh2, (int)sizeof(T), true).total, stream, (const T*)q, (const T*)k1,
+                           route_smem_layout(K, dh2, (int)sizeof(T), kRtWaves, true).total, stream, (const T*)q, (const T*)k1,
+                           (const T*)k2, key_norms, rows, dq, K, top_k, kc, (T*)gates, ids, (const T*)kfrag);
+    else if (rpw == 2)
+        hipLaunchKernelGGL((route_kernel<T, 2, false, kPrep>), grid, dim3(kRtWaves * 64),
+                           route_smem_layout(K, dh2, (int)sizeof(T), 2 * kRtWaves).total, stream, (const T*)q, (const T*)k1,
                            (const T*)k2, key_norms, rows, dq, K, top_k, kc, (T*)gates, ids, (const T*)kfrag);
     else
         hipLaunchKernelGGL((route_kernel<T, 4, false, kPrep>), grid, dim3(kRtWaves * 64),

@@ -753,3 +753,47 @@ def test_generate_fp32_products(U, max_u, E, dl, dh, d):
     assert not got[U // 2].any()
     vr = got @ w2[d:].double().T
     assert float((v[:U].cpu().double() - vr).norm()) <= 1e-6 * float(vr.norm()) + 1e-30
+
+
+@pytest.mark.parametrize("dt,dq,K,rows", [("bf16", 256, 512, 2049), ("bf16", 256, 512, 8193), ("bf16", 512, 512, 9000),
+                                          ("bf16", 512, 512, 16384), ("fp32", 64, 100, 2050), ("fp32", 256, 512, 8192)])
+def test_route_rows_per_wave_agree(dt, dq, K, rows):
+    """One, two and four rows per wave give the same bits: a batch on either side of the lines
+    against its rows routed 2,000 at a time (one row per wave)."""
+    from ethos_amd import hip
+    g = torch.Generator().manual_seed(rows)
+    tdt = torch.bfloat16 if dt == "bf16" else torch.float32
+    k1, k2 = ((torch.randn(K, dq // 2, generator=g) / (dq // 2) ** 0.5).to(tdt).cuda() for _ in range(2))
+    q = torch.randn(rows, dq, generator=g).to(tdt).cuda()
+    kn, kp = hip.key_norm_bounds(k1, k2), hip.route_prepare_keys(k1, k2)
+    for prep in (kp, None):
+        gates, ids = hip.route_topk(q, k1, k2, 16, key_norms=kn, prepared_keys=prep)
+        parts = [hip.route_topk(q[r:r + 2000].contiguous(), k1, k2, 16, key_norms=kn, prepared_keys=prep) for r in range(0, rows, 2000)]
+        assert torch.equal(ids, torch.cat([p[1] for p in parts]))
+        assert torch.equal(gates, torch.cat([p[0] for p in parts]))
+
+
+@pytest.mark.parametrize("n,d,H,dq,wide", [(1, 64, 1, 32, False), (17, 1024, 8, 256, False), (31, 200, 3, 40, True),
+                                           (48, 8, 2, 16, False), (190, 1024, 8, 256, True), (100, 1000, 8, 512, False)])
+def test_query_proj_few_tokens_bit_exact(n, d, H, dq, wide):
+    """The float64-MFMA projection of few tokens (prepared weights) gives the digit form's bits
+    (unprepared weights), which the oracle tests pin: tiles of 16 and 32 tokens, remainders in
+    every size, exponents spread over 40 binades (`wide`: sums that are not exact in float64
+    and results near rounding boundaries), zeros, infinities and NaN."""
+    from ethos_amd import hip
+    g = torch.Generator().manual_seed(n + d)
+    x, wq = torch.randn(n, d, generator=g), torch.randn(H, dq, d, generator=g) / d ** 0.5
+    if wide:
+        x = x * 2.0 ** torch.randint(-20, 21, x.shape, generator=g)
+        wq = wq * 2.0 ** torch.randint(-20, 21, wq.shape, generator=g)
+    if n > 16:
+        x[3] = 0.0
+        x[5, 1], x[6, 2] = float("inf"), float("nan")
+        wq[0, 2, 3] = float("-inf")
+    x, wq, bq = x.bfloat16().cuda(), wq.bfloat16().cuda(), torch.randn(H, dq, generator=g).bfloat16().cuda()
+    al, be = (torch.rand(H, dq, generator=g) + 0.5).cuda(), torch.randn(H, dq, generator=g).cuda()
+    a = hip.query_proj(x, wq, bq, al, be)
+    b = hip.query_proj(x, wq, bq, al, be, prepared=hip.query_proj_prepare(wq))
+    nan = torch.isnan(a.float())
+    assert torch.equal(nan, torch.isnan(b.float()))
+    assert torch.equal(a.view(torch.int16)[~nan], b.view(torch.int16)[~nan])
