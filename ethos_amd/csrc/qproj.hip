@@ -710,6 +710,137 @@ __global__ __launch_bounds__(256) void qproj_split_finish_kernel(const int64_t* 
     }
 }
 
+// ---- few tokens: float64 MFMAs ---------------------------------------------------------------
+// bf16 operands are exact in float64, and so are their products; a float64 sum of them in any
+// order is within d 2^-53 A of the index-order chain's, A >= sum |x_i w_i|.  So few tokens need
+// neither digit planes nor partial sums in memory: one launch computes V with
+// v_mfma_f64_16x16x4, and an element whose V - eps and V + eps (eps = d 2^-51 max|x| |w|_1) give
+// the same rounded result has the chain's; the others (a result within eps of a rounding
+// boundary, or not finite) take the exact chain.
+//
+// A workgroup takes 16 columns and 16 MT tokens; its 8 waves share the reduction, 32 k at a time
+// (lane l: row l % 16 of each tile, 8 consecutive k from 8 (l / 16), which are k step j's A and B
+// operands for j = 0 .. 7: the order within the reduction is free), and add their sums through
+// LDS.  Bound by the round trip of its loads, then (above 32 tokens at 2,048 columns) by the
+// MFMAs.  us, d 1,024, the digit form's three launches | this one: 2,048 columns, 1 token 11.4 |
+// 5.6, 64 15.1 | 8.9, 128 23.7 | 16.1, 192 24.0 | 20.8, 256 24.4 | 26.3; 4,096 columns, 64 25.4 |
+// 14.9, 96 28.3 | 22.1; 1,024 columns, 384 24.2 | 20.6, 512 24.7 | 26.1.  So up to the work of
+// 192 tokens there; tiles of 32 tokens once those of 16 make more than three workgroups a CU
+// (64 tokens, 2,048 columns: 8.9 us in tiles of 16, 9.1 of 32, 14.7 of 64).
+typedef double f64x4_t __attribute__((ext_vector_type(4)));
+constexpr int kQfWaves = 8;
+constexpr int64_t kQfMaxWork = (int64_t)192 * 2048 * 1024;  // multiply-adds
+
+template <int MT>
+__global__ __launch_bounds__(kQfWaves * 64) void qproj_f64_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ w,
+                                                                  const QRowMeta* __restrict__ wmeta,
+                                                                  const uint16_t* __restrict__ bias,
+                                                                  const float* __restrict__ alpha, const float* __restrict__ beta,
+                                                                  int n_tok, int d, int ncols, uint16_t* __restrict__ q) {
+    constexpr int kEl = MT * 256;      // the workgroup's outputs
+    constexpr int kFinChunk = 512;     // products a wave stages for an exact chain
+    __shared__ __align__(16) double part[kQfWaves][kEl < kFinChunk ? kFinChunk : kEl];
+    __shared__ uint32_t amax[MT * 16];
+    const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int c0 = blockIdx.x * 16, t0 = blockIdx.y * 16 * MT;
+    if (tid < MT * 16) amax[tid] = 0;
+    const int r = lane & 15, kq = 8 * (lane >> 4);
+    const uint16_t* wp = w + (int64_t)(c0 + r < ncols ? c0 + r : ncols - 1) * d;
+    const uint16_t* xp[MT];
+#pragma unroll
+    for (int t = 0; t < MT; ++t) xp[t] = x + (int64_t)(t0 + 16 * t + r < n_tok ? t0 + 16 * t + r : n_tok - 1) * d;
+    f64x4_t acc[MT];
+    uint32_t top[MT];
+#pragma unroll
+    for (int t = 0; t < MT; ++t) {
+        acc[t] = f64x4_t{0.0, 0.0, 0.0, 0.0};
+        top[t] = 0;
+    }
+    const int n_chunks = (d + 31) / 32;
+    auto value = [](const uint4& v, int j) {
+        const uint32_t u = j < 2 ? v.x : j < 4 ? v.y : j < 6 ? v.z : v.w;
+        return (double)__uint_as_float(j & 1 ? u & 0xffff0000u : u << 16);
+    };
+    constexpr int kAhead = 2;  // chunks whose loads are in flight together
+    for (int ch = wv; ch < n_chunks; ch += kQfWaves * kAhead) {
+        uint4 b[kAhead], a[kAhead][MT];
+#pragma unroll
+        for (int u = 0; u < kAhead; ++u) {
+            const int k = (ch + u * kQfWaves) * 32 + kq;
+            const int kc = k < d ? k : 0;  // past the row: zeros below
+            b[u] = *reinterpret_cast<const uint4*>(wp + kc);
+#pragma unroll
+            for (int t = 0; t < MT; ++t) a[u][t] = *reinterpret_cast<const uint4*>(xp[t] + kc);
+        }
+#pragma unroll
+        for (int u = 0; u < kAhead; ++u) {
+            if ((ch + u * kQfWaves) * 32 + kq >= d) {
+                b[u] = make_uint4(0, 0, 0, 0);
+#pragma unroll
+                for (int t = 0; t < MT; ++t) a[u][t] = make_uint4(0, 0, 0, 0);
+            }
+#pragma unroll
+            for (int t = 0; t < MT; ++t) {
+                const uint32_t wd[4] = {a[u][t].x, a[u][t].y, a[u][t].z, a[u][t].w};
+#pragma unroll
+                for (int i = 0; i < 4; ++i) top[t] = max(top[t], max(wd[i] & 0x7fffu, (wd[i] >> 16) & 0x7fffu));
+            }
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                const double bv = value(b[u], j);
+#pragma unroll
+                for (int t = 0; t < MT; ++t) acc[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(value(a[u][t], j), bv, acc[t], 0, 0, 0);
+            }
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int t = 0; t < MT; ++t) {
+        atomicMax(&amax[16 * t + r], top[t]);
+        // row 16 t + 4 i + lane / 16, column lane % 16
+#pragma unroll
+        for (int i = 0; i < 4; ++i) part[wv][(16 * t + 4 * i + (lane >> 4)) * 16 + r] = acc[t][i];
+    }
+    __syncthreads();
+    constexpr int kPer = (kEl + kQfWaves * 64 - 1) / (kQfWaves * 64);  // outputs per thread
+    bool unsure[kPer];
+#pragma unroll
+    for (int u = 0; u < kPer; ++u) {
+        const int e = tid + u * kQfWaves * 64;
+        const int t = t0 + e / 16, c = c0 + e % 16;
+        unsure[u] = false;
+        if (e >= kEl || t >= n_tok || c >= ncols) continue;
+        double v = 0.0;
+#pragma unroll
+        for (int i = 0; i < kQfWaves; ++i) v += part[i][e];
+        const float big = __uint_as_float(amax[e / 16] << 16) + 0x1p-126f;
+        const double eps = (double)d * 0x1p-51 * ((double)big * (double)wmeta[c].l1);
+        const double bv = Elem<uint16_t>::to_f64(bias[c]);
+        const float lo = Elem<uint16_t>::round64((v - eps) + bv), hi = Elem<uint16_t>::round64((v + eps) + bv);
+        const bool same = __float_as_uint(lo) == __float_as_uint(hi) && (__float_as_uint(lo) & 0x7f800000u) != 0x7f800000u;
+        unsure[u] = !same;
+        if (same) q[(int64_t)t * ncols + c] = Elem<uint16_t>::from_f32(__builtin_fmaf(lo, alpha[c], beta[c]));
+    }
+    __syncthreads();  // the partial sums are read: the exact chains take their place
+#pragma unroll
+    for (int u = 0; u < kPer; ++u) {
+        for (uint64_t pend = __ballot(unsure[u]); pend != 0; pend = __ballot(unsure[u])) {
+            const int lead = __builtin_ctzll(pend);
+            const int e = wv * 64 + lead + u * kQfWaves * 64;
+            qp_exact_element(x, w, bias, alpha, beta, d, ncols, (int64_t)(t0 + e / 16) * ncols + c0 + e % 16, part[wv], kFinChunk, q);
+            if (lane == lead) unsure[u] = false;
+        }
+    }
+}
+
+template <int MT>
+static void launch_qproj_f64(const void* x, const void* w, const QRowMeta* wmeta, const void* b, const float* alpha, const float* beta,
+                             int64_t n_tok, int d, int ncols, void* q, hipStream_t stream) {
+    hipLaunchKernelGGL((qproj_f64_kernel<MT>), dim3((ncols + 15) / 16, (unsigned)((n_tok + 16 * MT - 1) / (16 * MT))),
+                       dim3(kQfWaves * 64), 0, stream, (const uint16_t*)x, (const uint16_t*)w, wmeta, (const uint16_t*)b, alpha, beta,
+                       (int)n_tok, d, ncols, (uint16_t*)q);
+}
+
 size_t qproj_workspace_bytes(int64_t n_tok, int ncols, int d, int dtype) {
     return dtype == kBF16 && d <= kQiMaxD ? qproj_ws_bytes(n_tok, ncols, d) : 0;
 }
@@ -742,6 +873,16 @@ int launch_qproj(const void* x, const void* w, const void* prepared, const void*
                  const float* beta, int64_t n_tok, int d, int ncols, int dtype, void* ws, void* q, int num_cus,
                  hipStream_t stream) {
     if (dtype == kBF16 && d <= kQiMaxD) {
+        if (prepared && n_tok * ncols <= kQfMaxWork / d) {
+            const int8_t* unused;
+            const QRowMeta* wmeta;
+            prepared_parts(prepared, ncols, d, &unused, &wmeta);
+            if ((int64_t)((ncols + 15) / 16) * ((n_tok + 15) / 16) <= 3 * num_cus)
+                launch_qproj_f64<1>(x, w, wmeta, b, alpha, beta, n_tok, d, ncols, q, stream);
+            else
+                launch_qproj_f64<2>(x, w, wmeta, b, alpha, beta, n_tok, d, ncols, q, stream);
+            return (int)hipGetLastError();
+        }
         const QprojWs W = qproj_ws(ws, n_tok, ncols, d);
         const int8_t* wdig = W.wdig;
         const QRowMeta* wmeta = W.meta + n_tok;
