@@ -52,6 +52,9 @@ SIGNATURES = {
     "ethos_expert_backward_workspace_bytes": (_sz, [_i64, _i32, _i32, _i32]),
     "ethos_expert_backward": (ctypes.c_int, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i32, _i32, _i32, _i32, _vp,
                                              _sz, _vp, _vp, _vp, _vp, _vp]),
+    "ethos_layer_forward_workspace_bytes": (_sz, [_i64] + [_i32] * 4 + [_i64] + [_i32] * 3),
+    "ethos_layer_forward": (ctypes.c_int, [_vp] * 3 + [_sz] + [_vp] * 7 + [_sz] + [_vp] * 4 + [_i64] + [_i32] * 6 + [_i64] +
+                            [_i32] * 4 + [_vp, _sz, _vp, _vp]),
     "ethos_rms_norm": (ctypes.c_int, [_vp, _i64, _vp, _i64, _i32, _f32, _i32, _vp, _vp]),
     "ethos_swiglu": (ctypes.c_int, [_vp, _i64, _i32, _i32, _vp, _vp]),
     "ethos_mla_attention_workspace_bytes": (_sz, [_i64, _i64]),

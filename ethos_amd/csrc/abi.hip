@@ -755,4 +755,113 @@ int ethos_mla_attention(const void* q, const void* kv, const void* k_rot, int64_
                       "ethos_mla_attention");
 }
 
+namespace {
+
+// ethos_layer_forward's workspace: what lives to the end, then one region that the projection (its
+// scratch and the queries), the sort and the expert stages use in turn.
+struct LayerLayout {
+    size_t gates, ids, perm, pair_slot, sorted_slot, uniq, seg_off, n_unique, xp, shared, q, qws, h, ews, total;
+    size_t qws_bytes, sort_bytes, ews_bytes;
+    int64_t n_pairs, max_u;
+};
+
+LayerLayout layer_layout(int64_t n_tok, int H, int k, int d, int dq, int64_t n_experts, int dh, int dtype, int order) {
+    LayerLayout l{};
+    const size_t eb = dtype == ETHOS_BF16 ? 2 : 4;
+    l.n_pairs = n_tok * H * k;
+    l.max_u = l.n_pairs < n_experts ? l.n_pairs : n_experts;
+    l.max_u = l.max_u < 1 ? 1 : l.max_u;
+    size_t at = 0;
+    auto take = [&](size_t bytes) {
+        const size_t r = at;
+        at += (bytes + 255) & ~(size_t)255;
+        return r;
+    };
+    l.gates = take((size_t)l.n_pairs * eb);
+    l.ids = take((size_t)l.n_pairs * 4);
+    l.perm = take((size_t)l.n_pairs * 4);
+    l.pair_slot = take((size_t)l.n_pairs * 4);
+    l.sorted_slot = take((size_t)l.n_pairs * 4);
+    l.uniq = take((size_t)l.max_u * 4);
+    l.seg_off = take((size_t)(l.max_u + 1) * 4);
+    l.n_unique = take(4);
+    l.xp = take((size_t)n_tok * dh * eb);
+    l.shared = at;
+    l.qws_bytes = ethos_query_proj_workspace_bytes(n_tok, d, H, dq, dtype);
+    l.q = take((size_t)n_tok * H * dq * eb);
+    l.qws = take(l.qws_bytes);
+    l.total = at;
+    l.sort_bytes = ethos_sort_workspace_bytes(l.n_pairs, n_experts);
+    at = l.shared;
+    take(l.sort_bytes);
+    l.total = l.total > at ? l.total : at;
+    at = l.shared;
+    l.ews_bytes = ethos_expert_forward_workspace_bytes(n_tok, H, k, l.max_u, d, dh, dtype, order);
+    l.h = take((size_t)l.max_u * dh * eb);
+    l.ews = take(l.ews_bytes);
+    l.total = l.total > at ? l.total : at;
+    return l;
+}
+
+bool layer_sizes_ok(int64_t n_tok, int H, int k, int d, int dq, int64_t n_experts, int dh) {
+    return n_tok > 0 && n_tok <= INT32_MAX && H > 0 && k > 0 && d > 0 && dq > 0 && n_experts > 0 && dh > 0 &&
+           n_tok <= INT32_MAX / H / k;
+}
+
+}  // namespace
+
+size_t ethos_layer_forward_workspace_bytes(int64_t n_tok, int32_t n_heads, int32_t top_k, int32_t d_model, int32_t d_query,
+                                           int64_t n_experts, int32_t d_hidden, int32_t dtype, int32_t order) {
+    if (!layer_sizes_ok(n_tok, n_heads, top_k, d_model, d_query, n_experts, d_hidden)) return 256;
+    return layer_layout(n_tok, n_heads, top_k, d_model, d_query, n_experts, d_hidden, dtype, order).total;
+}
+
+int ethos_layer_forward(const void* x, const void* wq, const void* wq_prepared, size_t wq_prepared_bytes, const void* bq,
+                        const float* bn_alpha, const float* bn_beta, const void* sub_keys_1, const void* sub_keys_2,
+                        const float* key_norms, const void* keys_prepared, size_t keys_prepared_bytes, const void* latents,
+                        const void* w1, const void* w2, const void* wut, int64_t n_tok, int32_t d_model, int32_t n_heads,
+                        int32_t d_query, int32_t n_sub_keys, int32_t top_k, int32_t k_cand, int64_t n_experts, int32_t d_latent,
+                        int32_t d_hidden, int32_t dtype, int32_t order, void* workspace, size_t workspace_bytes, void* out,
+                        void* stream) {
+    g_err[0] = 0;
+    if (!dtype_ok(dtype)) return fail(ETHOS_EDTYPE, "ethos_layer_forward: unknown dtype %d", dtype);
+    if (order != 0 && order != 1) return fail(ETHOS_ESIZE, "ethos_layer_forward: order must be 0 or 1, got %d", order);
+    if (n_tok == 0) return 0;
+    if (!layer_sizes_ok(n_tok, n_heads, top_k, d_model, d_query, n_experts, d_hidden) || d_latent <= 0)
+        return fail(ETHOS_ESIZE, "ethos_layer_forward: bad sizes");
+    if (!workspace) return fail(ETHOS_ENULL, "ethos_layer_forward: null pointer");
+    if (!aligned16(workspace)) return fail(ETHOS_EALIGN, "ethos_layer_forward: workspace must be 16-byte aligned");
+    const LayerLayout l = layer_layout(n_tok, n_heads, top_k, d_model, d_query, n_experts, d_hidden, dtype, order);
+    if (workspace_bytes < l.total)
+        return fail(ETHOS_EWORKSPACE, "ethos_layer_forward: workspace of %zu bytes, %zu needed", workspace_bytes, l.total);
+    unsigned char* w = static_cast<unsigned char*>(workspace);
+    void *q = w + l.q, *gates = w + l.gates, *xp = nullptr;
+    int32_t *ids = (int32_t*)(w + l.ids), *perm = (int32_t*)(w + l.perm), *uniq = (int32_t*)(w + l.uniq);
+    int32_t *seg_off = (int32_t*)(w + l.seg_off), *pair_slot = (int32_t*)(w + l.pair_slot);
+    int32_t *sorted_slot = (int32_t*)(w + l.sorted_slot), *n_unique = (int32_t*)(w + l.n_unique);
+    int rc = wq_prepared ? ethos_query_proj_prepared(x, wq, wq_prepared, wq_prepared_bytes, bq, bn_alpha, bn_beta, n_tok, d_model,
+                                                     n_heads, d_query, dtype, w + l.qws, l.qws_bytes, q, stream)
+                         : ethos_query_proj(x, wq, bq, bn_alpha, bn_beta, n_tok, d_model, n_heads, d_query, dtype, w + l.qws,
+                                            l.qws_bytes, q, stream);
+    if (rc) return rc;
+    const int64_t rows = n_tok * n_heads;
+    rc = keys_prepared ? ethos_route_topk_prepared(q, sub_keys_1, sub_keys_2, key_norms, keys_prepared, keys_prepared_bytes, rows,
+                                                   d_query, n_sub_keys, top_k, k_cand, dtype, gates, ids, stream)
+                       : ethos_route_topk(q, sub_keys_1, sub_keys_2, key_norms, rows, d_query, n_sub_keys, top_k, k_cand, dtype,
+                                          gates, ids, stream);
+    if (rc) return rc;
+    if (dtype == ETHOS_BF16 && l.n_pairs <= ETHOS_SMALL_SORT_PAIRS) {  // with the token projection in the sort's launch
+        xp = w + l.xp;
+        rc = ethos_sort_segment_token_proj(ids, l.n_pairs, n_experts, w + l.shared, l.sort_bytes, perm, uniq, seg_off, pair_slot,
+                                           sorted_slot, n_unique, x, w2, wut, n_tok, d_model, d_hidden, dtype, xp, stream);
+    } else {
+        rc = ethos_sort_segment(ids, l.n_pairs, n_experts, w + l.shared, l.sort_bytes, perm, uniq, seg_off, pair_slot, sorted_slot,
+                                n_unique, stream);
+    }
+    if (rc) return rc;
+    return ethos_expert_forward(x, latents, n_experts, w1, w2, wut, xp, uniq, seg_off, n_unique, l.max_u, perm, sorted_slot,
+                                pair_slot, gates, n_tok, n_heads, top_k, d_latent, d_hidden, d_model, dtype, order, w + l.ews,
+                                l.ews_bytes, w + l.h, out, stream);
+}
+
 }  // extern "C"

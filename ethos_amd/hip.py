@@ -545,6 +545,35 @@ def gate_grads(x: torch.Tensor, ids: torch.Tensor, dg: torch.Tensor, wq: torch.T
     return dx, dw, db, dgamma, dbeta, dk1, dk2
 
 
+def layer_forward(x: torch.Tensor, packed, key_norms: torch.Tensor, keys_prepared: torch.Tensor | None,
+                  wq_prepared: torch.Tensor | None, generator, n_experts: int, top_k: int, hidden_space: bool) -> torch.Tensor:
+    """The eval-mode layer on x [n, d] in one library call.  `packed`: (wq, bq, sub_keys_1,
+    sub_keys_2, alpha, beta) and `generator`: (latents, w1, w2, wut or None) as the stages'
+    wrappers above take them; the caller packs them in x's dtype on its device."""
+    _need(x, "x", dim=2)
+    wq, bq, k1, k2, alpha, beta = packed
+    latents, w1, w2, wut = generator
+    n, d = x.shape
+    H, dq, d2 = wq.shape
+    dh, dl = w1.shape
+    K = k1.shape[0]
+    if d2 != d or w2.shape != (2 * d, dh) or latents.shape != (n_experts, dl) or K * K != n_experts or k1.shape[1] * 2 != dq:
+        raise RuntimeError("layer_forward: inconsistent shapes")
+    code, order = dtype_code(x.dtype), 1 if hidden_space else 0
+    lib = load()
+    ws, ws_bytes = workspace(lib.ethos_layer_forward_workspace_bytes(n, H, top_k, d, dq, n_experts, dh, code, order), x.device)
+    out = torch.empty_like(x)
+    rc = lib.ethos_layer_forward(
+        x.data_ptr(), wq.data_ptr(), wq_prepared.data_ptr() if wq_prepared is not None else None,
+        wq_prepared.numel() if wq_prepared is not None else 0, bq.data_ptr(), alpha.data_ptr(), beta.data_ptr(), k1.data_ptr(),
+        k2.data_ptr(), key_norms.data_ptr(), keys_prepared.data_ptr() if keys_prepared is not None else None,
+        keys_prepared.numel() if keys_prepared is not None else 0, latents.data_ptr(), w1.data_ptr(), w2.data_ptr(),
+        wut.data_ptr() if wut is not None else None, n, d, H, dq, K, top_k, 2 * top_k, n_experts, dl, dh, code, order,
+        ws.data_ptr(), ws_bytes, out.data_ptr(), _stream())
+    check(rc, "ethos_layer_forward")
+    return out
+
+
 # ----------------------------------------------------------- the language model's blocks
 def plain(*ts) -> bool:
     """Whether a library call may stand in for torch operations on these tensors: ordinary HIP

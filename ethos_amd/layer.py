@@ -311,7 +311,7 @@ class ProductKeyRouter(nn.Module):
         return self._packed_weights(dtype, device) + tuple(self._bn_coefficients(device))
 
     def _bn_uses_batch_stats(self) -> bool:
-        return any(m.training or not m.track_running_stats for m in self.query_norms)
+        return any(m.training or not m.track_running_stats for m in self._modules["query_norms"]._modules.values())
 
     def _bn_one_call(self, x_flat: torch.Tensor) -> bool:
         """Whether the heads' training-mode BatchNorms run as one library call: all of them on
@@ -501,7 +501,8 @@ class EthosExpertLayer(nn.Module):
         return self.forward_flat(x_flat).view(b, s, d)
 
     def forward_flat(self, x_flat: torch.Tensor, mark=None, side_stream: torch.cuda.Stream | None = None) -> torch.Tensor:
-        """The layer on [n_tok, d_model] rows (model.py:288-343).  `mark(stage)`, if given, is
+        """The layer on [n_tok, d_model] rows (model.py:288-343), in eval mode one library call;
+        with `mark` or `side_stream` (and in training mode) stage by stage.  `mark(stage)`, if given, is
         called after the query projection, the routing and the sort are enqueued on the
         current stream (the expert stages are one library call; hip.stage_events times the
         stages inside it).  `side_stream`: the token projection x W_u, which needs only x, runs
@@ -515,6 +516,13 @@ class EthosExpertLayer(nn.Module):
             g = self.router._gate_graph(x_flat, ids, gates)
             return _ExpertStages.apply(x_flat, g, self.expert_latents.weight, self.generation_network.net[0].weight,
                                        self.generation_network.net[2].weight, self, gates, seg)
+        router = self._modules["router"]
+        if mark is None and side_stream is None and x_flat.shape[0] > 0 and not router._bn_uses_batch_stats():
+            with torch.no_grad():
+                packed = router._packed(x_flat.dtype, x_flat.device)
+                gen = self._generator_params(x_flat.dtype, x_flat.device)
+                return hip.layer_forward(x_flat, packed, router._key_norms, router._keys_prepared, router._wq_prepared, gen,
+                                         self.num_experts, self.top_k, self.hidden_space)
         with torch.no_grad():
             xp = None
             if side_stream is not None:

@@ -16,6 +16,7 @@
  *   ethos_apply_scatter  per-pair activation and weighted scatter-back into tokens
  *   ethos_apply_hidden   the same, by hidden-space reordering (no v rows)
  *   ethos_expert_forward generation + apply + scatter-back in one call (either order)
+ *   ethos_layer_forward  all of them: the eval-mode layer in one call
  *   ethos_expert_backward  per-pair part of the expert stages' backward
  *   ethos_query_bn_train   query BatchNorm with batch statistics (training)
  *   ethos_bn_coefficients  the eval-mode BatchNorm coefficients of ethos_query_proj
@@ -473,6 +474,26 @@ size_t ethos_mla_attention_workspace_bytes(int64_t n_seq, int64_t seq_len);
 int ethos_mla_attention(const void* q, const void* kv, const void* k_rot, int64_t k_rot_ld, const int64_t* positions,
                         const float* rates, int64_t n_seq, int64_t seq_len, int32_t n_heads, int32_t nope, int32_t rope, int32_t v_dim,
                         int32_t dtype, float scale, void* workspace, size_t workspace_bytes, void* out, void* stream);
+
+/*
+ * The eval-mode layer (model.py:288-343) in one call: ethos_query_proj(_prepared),
+ * ethos_route_topk(_prepared), ethos_sort_segment (with the token projection in its launch for
+ * bf16 batches of at most ETHOS_SMALL_SORT_PAIRS pairs) and ethos_expert_forward, with every
+ * intermediate in the workspace.  The arguments are those calls', with the same limits; an error
+ * is the failing call's.  wq_prepared, key_norms, keys_prepared and wut may be NULL.
+ *   out        [n_tok, d_model] T
+ *   workspace  >= ethos_layer_forward_workspace_bytes(...) bytes, 16-byte aligned (scratch)
+ */
+#define ETHOS_SMALL_SORT_PAIRS 16384
+size_t ethos_layer_forward_workspace_bytes(int64_t n_tok, int32_t n_heads, int32_t top_k, int32_t d_model, int32_t d_query,
+                                           int64_t n_experts, int32_t d_hidden, int32_t dtype, int32_t order);
+int ethos_layer_forward(const void* x, const void* wq, const void* wq_prepared, size_t wq_prepared_bytes, const void* bq,
+                        const float* bn_alpha, const float* bn_beta, const void* sub_keys_1, const void* sub_keys_2,
+                        const float* key_norms, const void* keys_prepared, size_t keys_prepared_bytes, const void* latents,
+                        const void* w1, const void* w2, const void* wut, int64_t n_tok, int32_t d_model, int32_t n_heads,
+                        int32_t d_query, int32_t n_sub_keys, int32_t top_k, int32_t k_cand, int64_t n_experts, int32_t d_latent,
+                        int32_t d_hidden, int32_t dtype, int32_t order, void* workspace, size_t workspace_bytes, void* out,
+                        void* stream);
 
 #ifdef __cplusplus
 }

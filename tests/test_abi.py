@@ -220,3 +220,45 @@ def test_stage_events_argument_errors():
     assert L.ethos_stage_events(None, 17) == -2
     assert L.ethos_stage_events(None, 2) == -2
     assert L.ethos_stage_events(None, 0) == 0
+
+
+def test_layer_forward_argument_errors_are_codes():
+    L = _lib.load()
+    sizes = dict(n=4, d=64, H=2, dq=32, K=16, k=4, E=256, dl=16, dh=32)
+    need = L.ethos_layer_forward_workspace_bytes(4, 2, 4, 64, 32, 256, 32, 1, 0)
+    assert need > 0
+
+    def rc(ws=16, ws_bytes=need, dtype=1, order=0, n=4, x=16):
+        s = sizes
+        return L.ethos_layer_forward(x, 16, None, 0, 16, 16, 16, 16, 16, None, None, 0, 16, 16, 16, None, n, s["d"], s["H"], s["dq"],
+                                     s["K"], s["k"], 2 * s["k"], s["E"], s["dl"], s["dh"], dtype, order, ws, ws_bytes, 16, None)
+
+    assert rc(dtype=7) == -1
+    assert rc(order=2) == -2 and rc(n=-1) == -2
+    assert rc(n=0) == 0
+    assert rc(ws=None) == -3 and rc(x=None) == -3
+    assert rc(ws=8) == -4
+    assert rc(ws_bytes=need - 1) == -5
+
+
+def test_training_entry_points_argument_errors_are_codes():
+    L = _lib.load()
+    P = (ctypes.c_void_p * 2)(16, 16)
+    Z = (ctypes.c_void_p * 2)(16, None)
+    bn = lambda n=8, dq=8, g=P, m=None, dt=1, ws=1 << 30: L.ethos_query_bn_train(  # noqa: E731
+        16, n, 2, dq, dt, g, P, m, m, None, None, 0.1, 1e-5, 16, ws, 16, None)
+    assert bn(dt=7) == -1 and bn(n=1) == -2 and bn(dq=6) == -6 and bn(g=Z) == -3 and bn(m=Z) == -3 and bn(ws=8) == -5
+    assert L.ethos_bn_coefficients(64, 8, 1, None, None, None, None, 1e-5, 16, 16, None) == -6
+    assert L.ethos_bn_coefficients(2, 8, 1, None, None, None, None, 1e-5, None, 16, None) == -3
+    gg = lambda d=64, dq=32, dt=1, g=P, ws=1 << 30, x=16: L.ethos_gate_grads(  # noqa: E731
+        x, 16, 16, 16, 16, 16, 16, g, P, None, None, 1e-5, 4, d, 2, dq, 16, 4, dt, 16, ws, 16, 16, 16, 16, 16, 16, 16, None)
+    assert gg(dt=7) == -1 and gg(d=60) == -6 and gg(dq=520) == -6 and gg(g=Z) == -3 and gg(x=None) == -3 and gg(x=8) == -4
+    assert gg(ws=8) == -5
+    eg = lambda d=64, dt=1, ws=1 << 30, u=8, x=16: L.ethos_expert_grads(  # noqa: E731
+        x, 16, 16, 16, 16, 16, 16, 16, 16, u, 16, 16, 16, 16, 4, 2, 4, 16, 32, d, dt, 16, ws, 16, 16, 16, 16, 16, None)
+    assert eg(dt=7) == -1 and eg(d=60) == -6 and eg(u=0) == -2 and eg(x=None) == -3 and eg(x=8) == -4 and eg(ws=8) == -5
+    assert L.ethos_rms_norm(16, 64, 16, 4, 60, 1e-6, 1, 16, None) == -6 and L.ethos_rms_norm(16, 32, 16, 4, 64, 1e-6, 1, 16, None) == -2
+    assert L.ethos_swiglu(16, 4, 60, 1, 16, None) == -6 and L.ethos_swiglu(None, 4, 64, 1, 16, None) == -3
+    at = lambda dt=1, v=64, ld=64, ws=1 << 20, q=16: L.ethos_mla_attention(  # noqa: E731
+        q, 16, 16, ld, 16, 16, 1, 8, 2, 64, 64, v, dt, 0.1, 16, ws, 16, None)
+    assert at(dt=0) == -1 and at(v=32) == -6 and at(ld=65) == -6 and at(q=None) == -3 and at(q=8) == -4 and at(ws=8) == -5

@@ -276,3 +276,22 @@ def test_library_stream_is_torch_current_stream():
     with torch.cuda.stream(s):
         assert hip._stream() == s.cuda_stream == torch.cuda.current_stream().cuda_stream
     assert hip._stream() == torch.cuda.current_stream().cuda_stream
+
+
+@pytest.mark.parametrize("name,n,hidden", [("tiny", 1, False), ("tiny", 48, True), ("tiny_fp32", 47, False), ("cfg3", 64, False),
+                                           ("cfg3", 129, False), ("cfg3", 300, True), ("cfg1", 256, True)])
+def test_one_call_forward_matches_stages(name, n, hidden):
+    """The eval-mode layer as one library call gives the bits of its stages called one by one
+    (forward_flat with `mark`): both execution orders, both dtypes, on either side of the small
+    sort's limit (128 tokens of 128 pairs)."""
+    sh = SHAPES[name]
+    x, sd = make_inputs(sh.with_tokens(n), signal=True)
+    m = ethos_amd.EthosExpertLayer(sh.config(), hidden_space=hidden).to(sh.torch_dtype)
+    m.load_state_dict(sd)
+    m = m.cuda().eval()
+    xd = x.cuda()
+    seen = []
+    with torch.no_grad():
+        a = m.forward_flat(xd)
+        b = m.forward_flat(xd, mark=seen.append)
+    assert seen and torch.equal(a, b)
