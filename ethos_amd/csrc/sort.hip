@@ -726,6 +726,18 @@ constexpr int kSmallMax = 16384;
 constexpr int kSmallChunks = kSmallMax / 64;                 // 256
 constexpr int kSmallPer = kSmallChunks / kSmallWaves;        // chunks per wave at most
 
+// Most batches need no radix passes: the words differ, so any order-preserving spread over
+// buckets (the key's top 11 bits; places within a bucket in the order the LDS counters give
+// them) followed by ranking each word among its bucket's words ends in the one sorted order.
+// When some bucket holds more than kSmallBucketMax words (few distinct experts) the ranking
+// would cost more than the passes, which then run (they cost 0.5 to 1.5 us more than without
+// the attempt).  us, routed pairs of 262,144 experts, passes | buckets: 128 pairs 7.7 | 5.6,
+// 4,096 14.7 | 10.0, 8,192 23.3 | 15.8, 16,384 40.0 | 28.9.
+constexpr int kSmallBucketBits = 11, kSmallBuckets = 1 << kSmallBucketBits;
+constexpr uint32_t kSmallBucketMax = 96, kSmallCrowded = 24;
+constexpr int kSmallSample = 256;
+static_assert(kSmallBuckets == 2 * kSmallWaves * 64, "two buckets a thread");
+
 // LDS of the small sort: the words twice, per-wave digit counts (then bases, < 2^14), head
 // flags per chunk, heads before each chunk, wave sums.
 constexpr size_t kSmallBufB = 2 * (size_t)kSmallMax * 4, kSmallCntB = (size_t)kSmallWaves * kRadix * 2;
@@ -747,23 +759,96 @@ __device__ __forceinline__ void sort_small_body(unsigned char* lds, const int32_
     const int n_chunks = (n + 63) / 64;
     const int cpw = (n_chunks + kSmallWaves - 1) / kSmallWaves;  // chunks per wave (<= kSmallPer)
     const int c0 = wave * cpw;
+    constexpr int kIn = kSmallMax / (kSmallWaves * 64), kStep = kSmallWaves * 64;
+    uint32_t* hist = reinterpret_cast<uint32_t*>(lds + kSmallBufB);  // then each bucket's first position
+    const int bsh = vb + (key_bits_ > kSmallBucketBits ? key_bits_ - kSmallBucketBits : 0);  // word -> bucket
+    bool bucketed;
     {
         // all of the thread's ids in flight at once (one workgroup: latency, not bandwidth)
-        constexpr int kIn = kSmallMax / (kSmallWaves * 64);
-        uint32_t k[kIn];
+        uint32_t word[kIn], off[kIn];
 #pragma unroll
         for (int j = 0; j < kIn; ++j) {
-            const int i = tid + j * kSmallWaves * 64;
-            k[j] = i < n ? (uint32_t)ids[i] : 0u;
+            const int i = tid + j * kStep;
+            word[j] = i < n ? (uint32_t)ids[i] : 0u;
         }
+        for (int e = tid; e < kSmallBuckets; e += kStep) hist[e] = 0;
+        __syncthreads();
 #pragma unroll
         for (int j = 0; j < kIn; ++j) {
-            const int i = tid + j * kSmallWaves * 64;
-            const uint32_t kk = k[j] > kmax ? kmax : k[j];  // ids outside [0, 2^key_bits) (a caller error) stay in range
-            if (i < n) buf[0][i] = (kk << vb) | (uint32_t)i;
+            if (j * kStep >= n) break;
+            const uint32_t kk = word[j] > kmax ? kmax : word[j];  // ids outside [0, 2^key_bits) (a caller error) stay in range
+            word[j] = (kk << vb) | (uint32_t)(tid + j * kStep);
         }
+        // one bucket's counter takes its words one after the other: the first 256 words tell a
+        // crowded one before the rest are counted
+        off[0] = tid < kSmallSample && tid < n ? atomicAdd(&hist[word[0] >> bsh], 1u) : 0u;
+        const bool crowded = __syncthreads_or(off[0] >= (n <= kSmallSample ? kSmallBucketMax : kSmallCrowded));
+        if (!crowded) {
+            if (tid >= kSmallSample && tid < n) off[0] = atomicAdd(&hist[word[0] >> bsh], 1u);
+#pragma unroll
+            for (int j = 1; j < kIn; ++j) {
+                if (j * kStep >= n) break;
+                off[j] = tid + j * kStep < n ? atomicAdd(&hist[word[j] >> bsh], 1u) : 0u;
+            }
+        }
+        uint32_t top = 0;
+        if (!crowded) {
+            __syncthreads();
+            // two buckets a thread: their first positions, and the largest count
+            const uint32_t n0 = hist[2 * tid], n1 = hist[2 * tid + 1];
+            uint32_t inc = n0 + n1;
+            top = n0 > n1 ? n0 : n1;
+#pragma unroll
+            for (int o = 1; o < 64; o <<= 1) {
+                const uint32_t u = __shfl_up(inc, o, 64), v = __shfl_xor(top, o, 64);
+                if (lane >= o) inc += u;
+                top = top > v ? top : v;
+            }
+            if (lane == 63) {
+                wsum[wave] = inc;
+                cbase[wave] = top;
+            }
+            __syncthreads();
+            uint32_t run = inc - n0 - n1;
+            top = 0;
+#pragma unroll
+            for (int w = 0; w < kSmallWaves; ++w) {
+                run += w < wave ? wsum[w] : 0u;
+                top = top > cbase[w] ? top : cbase[w];
+            }
+            hist[2 * tid] = run;
+            hist[2 * tid + 1] = run + n0;
+            if (tid == kStep - 1) hist[kSmallBuckets] = run + n0 + n1;
+            __syncthreads();
+        }
+        bucketed = !crowded && top <= kSmallBucketMax;
+#pragma unroll
+        for (int j = 0; j < kIn; ++j) {
+            if (j * kStep >= n) break;
+            const int i = tid + j * kStep;
+            if (i < n) buf[0][bucketed ? hist[word[j] >> bsh] + off[j] : (uint32_t)i] = word[j];
+        }
+        __syncthreads();
     }
     int cur = 0;
+    if (bucketed) {
+        // each word's place in its bucket: the words below it there (all words differ)
+        for (int i = tid; i < n; i += kStep) {
+            const uint32_t wd = buf[0][i];
+            const uint32_t b0 = hist[wd >> bsh], b1 = hist[(wd >> bsh) + 1];
+            uint32_t r = b0;
+            uint32_t q = b0;
+            for (; q + 4 <= b1; q += 4) {
+                const uint32_t x0 = buf[0][q], x1 = buf[0][q + 1], x2 = buf[0][q + 2], x3 = buf[0][q + 3];
+                r += (x0 < wd ? 1u : 0u) + (x1 < wd ? 1u : 0u) + (x2 < wd ? 1u : 0u) + (x3 < wd ? 1u : 0u);
+            }
+            for (; q < b1; ++q) r += buf[0][q] < wd ? 1u : 0u;
+            buf[1][r] = wd;
+        }
+        cur = 1;
+        passes = 0;
+        __syncthreads();
+    }
     for (int p = 0; p < passes; ++p) {
         const int shift = vb + kRadixBits * p;
         for (int e = tid; e < kSmallWaves * kRadix; e += kSmallWaves * 64) cnt[e / kRadix][e % kRadix] = 0;
@@ -901,6 +986,7 @@ __global__ __launch_bounds__(kSmallWaves * 64) void sort_small_kernel(const int3
 // The small sort in workgroup 0 and the bf16 token projection xp = RN(x W_u) in the
 // others (tile b - 1: column tile (b - 1) % nct, token tile (b - 1) / nct), which needs
 // only x: the tiles run on CUs the single sorting workgroup leaves idle.
+static_assert((size_t)(kSmallBuckets + 1) * 4 <= kSmallCntB, "the buckets fit the digit counts' storage");
 static_assert(kSmallLds >= (size_t)kTpLds, "the projection tile's ring fits the sort's LDS");
 __global__ __launch_bounds__(kSmallWaves * 64) void sort_small_tp_kernel(
     const int32_t* __restrict__ ids, int n, int key_bits_, int vb, int passes, int32_t* __restrict__ perm,
