@@ -25,6 +25,8 @@
 //     the later blocks' head parts, in block order.
 // launch_expert_grads runs the whole node: xp and dYB first, then these kernels, then the
 // weight, input and latent gradients as float32 matrix products (gemm.hip).
+#include <algorithm>
+
 #include "ethos_common.hpp"
 #include "ethos_gelu.hpp"
 #include "ethos_gemm.hpp"
@@ -362,8 +364,9 @@ size_t pad256(size_t n) { return (n + 255) & ~(size_t)255; }
 
 // Offsets in expert_grads' workspace.
 struct GradsLayout {
-    size_t xp, dyb, hacc, dxp, dhs, pairs, part, total;
+    size_t xp, dyb, hacc, dxp, dhs, pairs, w1p, part, total;
     int split_w2, split_w1;
+    bool one_pass;  // room for latent_grad.hip (which takes bf16 only)
 };
 
 GradsLayout grads_layout(int64_t n_tok, int H, int k, int64_t max_u, int dl, int dh, int d, int num_cus) {
@@ -375,11 +378,14 @@ GradsLayout grads_layout(int64_t n_tok, int H, int k, int64_t max_u, int dl, int
     l.dxp = 3 * tok;
     l.dhs = 4 * tok;
     l.pairs = l.dhs + pad256((size_t)max_u * dh * sizeof(float));
-    l.part = l.pairs + pad256(expert_backward_workspace_bytes(n_tok * H * k, dh));
+    l.one_pass = latent_grad_fits(max_u, dl, dh);
+    l.w1p = l.pairs + pad256(expert_backward_workspace_bytes(n_tok * H * k, dh));
+    l.part = l.w1p + (l.one_pass ? pad256((size_t)dh * dl * 4) : 0);
     l.split_w2 = gemm_split(dh, d, n_tok, num_cus);
     l.split_w1 = gemm_split(dh, dl, max_u, num_cus);
     const size_t p2 = l.split_w2 > 1 ? (size_t)l.split_w2 * dh * d : 0, p1 = l.split_w1 > 1 ? (size_t)l.split_w1 * dh * dl : 0;
-    l.total = l.part + pad256((p1 > p2 ? p1 : p2) * sizeof(float));
+    const size_t p0 = l.one_pass ? (size_t)latent_grad_parts(max_u, num_cus) * dh * dl : 0;
+    l.total = l.part + pad256(std::max({p0, p1, p2}) * sizeof(float));
     return l;
 }
 
@@ -393,8 +399,8 @@ size_t expert_grads_workspace_bytes(int64_t n_tok, int H, int k, int64_t max_u, 
 // float32 operands (gemm.hip), and the number of unique experts stays on the device: the
 // products over the experts' rows read it there, so the host does not wait for the routing.
 // 4,096 tokens, 200,070 experts, bf16: about 4.0 ms as library float32 GEMMs with the GELU
-// derivative as a chain of elementwise passes over [U, d_hidden], 0.99 ms as here (dpre 200 us,
-// expert sums 173, d latents 158, d W1 130, pairs 95, d W2 83, the token products 105).
+// derivative as a chain of elementwise passes over [U, d_hidden], 0.83 ms as here (d latents and
+// d W1 in one pass 338 us, expert sums 173, pairs 95, d W2 83, the token products 105).
 int launch_expert_grads(const void* x, const void* dy, const void* hid, const void* latents, const void* w1, const void* w2,
                         const int32_t* uniq, const int32_t* seg_off, const int32_t* n_unique, int64_t max_u,
                         const int32_t* perm, const int32_t* sorted_slot, const int32_t* pair_slot, const void* gates,
@@ -433,6 +439,9 @@ int launch_expert_grads(const void* x, const void* dy, const void* hid, const vo
     g.a = dxp, g.lda = dh, g.b = w2, g.ldb = dh, g.c = dx, g.ldc = d;
     g.m = n_tok, g.n = d, g.k = dh, g.out_bf16 = bf;
     if ((rc = launch_gemm(bf ? kGemmFK_BK : kGemmFK_FK, g, num_cus, stream))) return rc;
+
+    if (bf && l.one_pass)
+        return launch_latent_grad(dhs, latents, w1, uniq, n_unique, max_u, dh, w + l.w1p, part, dlat, dw1, num_cus, stream);
 
     g = Gemm{};  // dpre = gelu'(z W1) dh, in place of dh
     g.a = latents, g.lda = dl, g.a_rows = uniq, g.b = w1, g.ldb = dl, g.c = dhs, g.ldc = dh;

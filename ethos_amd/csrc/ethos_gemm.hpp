@@ -54,5 +54,19 @@ enum GemmForm {
 // CU, each with at least 256 of the reduction.
 int gemm_split(int64_t m, int n, int64_t k, int num_cus);
 int launch_gemm(GemmForm form, const Gemm& g, int num_cus, hipStream_t stream);
+// c = alpha * (the sum of `split` partial results [rows][cols], in order).
+int launch_gemm_reduce(const float* part, int split, int64_t rows, int64_t cols, float alpha, bool out_bf16, void* c, int64_t ldc,
+                       hipStream_t stream);
+
+// d latents and d W1 of the experts from dh in one pass (latent_grad.hip); w1p: d_hidden x 128
+// floats of workspace (W1 in two orders), part: latent_grad_parts() x d_hidden x 128 floats.
+// Taken when up to 16,384 unique experts or more are possible (a tile of 64 for each CU: 49 us against 94
+// as products); with fewer, part of the CUs would be idle in both forms and the products, which
+// spread over more workgroups, are kept.
+constexpr int64_t kLatentGradRows = 16384;
+bool latent_grad_fits(int64_t max_u, int dl, int dh);
+int latent_grad_parts(int64_t max_u, int num_cus);
+int launch_latent_grad(const float* dhs, const void* latents, const void* w1, const int32_t* uniq, const int32_t* n_unique,
+                       int64_t max_u, int dh, void* w1p, float* part, void* dlat, void* dw1, int num_cus, hipStream_t stream);
 
 }  // namespace ethos

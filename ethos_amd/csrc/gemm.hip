@@ -24,27 +24,13 @@
 #include "ethos_gelu.hpp"
 #include "ethos_gemm.hpp"
 #include "ethos_mfma.hpp"
+#include "ethos_split.hpp"
 
 namespace ethos {
 namespace {
 
 constexpr int kGemmK = 32;      // reduction step
 constexpr int kGemmThreads = 256;
-
-// Two float32 values -> their three bf16 planes, one packed word each (a low, b high): the upper
-// half (truncated, so that no finite value becomes an infinity), then the remainder and what is
-// left of it, both to nearest, so that the products left out have either sign (all truncated,
-// they would add up to 2^-23 of the result).  An infinity keeps its remainders at zero; a NaN
-// leaves one in the second plane.
-__device__ __forceinline__ void split3(float a, float b, uint32_t& hi, uint32_t& mid, uint32_t& lo) {
-    const uint32_t ua = __float_as_uint(a), ub = __float_as_uint(b);
-    hi = __builtin_amdgcn_perm(ub, ua, 0x07060302u);
-    float ra = a - __uint_as_float(ua & 0xffff0000u), rb = b - __uint_as_float(ub & 0xffff0000u);
-    ra = __builtin_isinf(a) ? 0.0f : ra;
-    rb = __builtin_isinf(b) ? 0.0f : rb;
-    mid = pack_bf16x2(ra, rb);
-    lo = pack_bf16x2(ra - __uint_as_float(mid << 16), rb - __uint_as_float(mid & 0xffff0000u));
-}
 
 // 16-byte piece `c` of LDS row `row`, in bf16 elements.
 __device__ __forceinline__ int lds_slot(int row, int c) { return (row * 4 + (c ^ ((row >> 2) & 3))) * 8; }
@@ -365,6 +351,19 @@ __global__ __launch_bounds__(256) void gemm_reduce_kernel(const float* __restric
     }
 }
 
+}  // namespace
+
+int launch_gemm_reduce(const float* part, int split, int64_t rows, int64_t cols, float alpha, bool out_bf16, void* c, int64_t ldc,
+                       hipStream_t stream) {
+    int64_t rb = (rows * cols + 255) / 256;
+    rb = rb > 4096 ? 4096 : rb;
+    hipLaunchKernelGGL(gemm_reduce_kernel, dim3((unsigned)rb), dim3(256), 0, stream, part, split, rows, cols, alpha,
+                       out_bf16 ? 1 : 0, c, ldc);
+    return (int)hipGetLastError();
+}
+
+namespace {
+
 template <typename TA, bool AK, typename TB, bool BK, bool IDX, int BM, int BN>
 int launch_t(const Gemm& g, hipStream_t stream) {
     const int64_t mt = (g.m + BM - 1) / BM, nt = (g.n + BN - 1) / BN;
@@ -375,10 +374,7 @@ int launch_t(const Gemm& g, hipStream_t stream) {
                        stream, g);
     if (g.split > 1) {
         const int64_t rows = g.transposed ? g.n : g.m, cols = g.transposed ? g.m : g.n;
-        int64_t rb = (rows * cols + 255) / 256;
-        rb = rb > 4096 ? 4096 : rb;
-        hipLaunchKernelGGL(gemm_reduce_kernel, dim3((unsigned)rb), dim3(256), 0, stream, g.part, g.split, rows, cols, g.alpha,
-                           g.out_bf16 ? 1 : 0, g.c, g.ldc);
+        return launch_gemm_reduce(g.part, g.split, rows, cols, g.alpha, g.out_bf16, g.c, g.ldc, stream);
     }
     return (int)hipGetLastError();
 }

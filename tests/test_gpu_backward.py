@@ -196,6 +196,11 @@ def test_expert_backward_entry_point(dt, n, H, k, dh, E, hot):
 @pytest.mark.parametrize("dt,n,H,k,dl,dh,d,E", [
     ("bf16", 1, 1, 1, 8, 8, 8, 1), ("bf16", 33, 2, 4, 16, 40, 72, 37), ("bf16", 129, 3, 4, 136, 264, 200, 700),
     ("bf16", 700, 4, 8, 128, 512, 256, 9000), ("bf16", 65, 8, 16, 128, 256, 1024, 1),
+    # one pass over the experts (16,384 pairs or more): less than a tile of 64, tiles off their
+    # end, one and several tiles a workgroup, one and two passes of 256 columns
+    ("bf16", 128, 8, 16, 128, 512, 64, 37), ("bf16", 130, 8, 16, 128, 256, 72, 65),
+    ("bf16", 140, 8, 16, 128, 512, 64, 262144), ("bf16", 300, 8, 16, 128, 256, 64, 30011),
+    ("bf16", 310, 8, 16, 128, 512, 64, 40000),
     ("fp32", 1, 1, 2, 8, 16, 8, 4), ("fp32", 50, 4, 8, 24, 72, 40, 11), ("fp32", 500, 4, 8, 128, 512, 256, 4096)])
 def test_expert_grads_entry_point(dt, n, H, k, dl, dh, d, E):
     """ethos_expert_grads against a float64 evaluation of the same derivative: sizes off every
