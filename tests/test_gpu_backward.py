@@ -359,3 +359,29 @@ def test_router_second_derivative(train):
     ref2 = torch.autograd.grad(sum((t ** 2).sum() for t in ref1), leaves_)
     for a, b in zip(first + second, ref1 + ref2):
         assert _nerr(a, b) < 1e-5
+
+
+@pytest.mark.parametrize("n,H,dq", [(2, 8, 256), (500, 8, 256), (1024, 16, 256), (1025, 16, 256), (2048, 8, 256), (2049, 8, 256),
+                                    (4096, 8, 256), (8192, 3, 256), (8193, 8, 256), (700, 4, 512), (3000, 5, 512),
+                                    (33, 4, 128)])
+def test_training_queries_are_per_head_batch_norms(n, H, dq):
+    """bf16 training-mode queries and running statistics are those of statistics taken a head at
+    a time, bit for bit, whatever number of heads shares a reduction."""
+    import ethos_amd
+    from ethos_amd import hip
+    from ethos_amd.model import lm_config
+    torch.manual_seed(n + H)
+    r = ethos_amd.EthosExpertLayer(lm_config(d_model=64, num_experts=64, top_k=2, num_routing_heads=H, d_query=dq, d_latent=8,
+                                             d_intermediate_hypernet=16)).to(torch.bfloat16).cuda().train().router
+    x = torch.randn(n, 64, device="cuda").to(torch.bfloat16)
+    with torch.no_grad():
+        q = r.queries(x)
+        v = hip.query_proj(x, *r._packed_weights(x.dtype, x.device)[:2], *r._identity, prepared=r._wq_prepared)
+        pairs = [torch.var_mean(v[:, h].float(), 0, unbiased=False) for h in range(H)]
+        norms = list(r.query_norms)
+        mean, var = [torch.zeros_like(m.running_mean) for m in norms], [torch.ones_like(m.running_var) for m in norms]
+        ref = hip.query_bn_train(v, [m.weight.detach() for m in norms], [m.bias.detach() for m in norms], mean, var, norms[0].momentum,
+                                 norms[0].eps, batch=([p[1] for p in pairs], [p[0] for p in pairs]))
+    assert torch.equal(q, ref)
+    for m, a, b in zip(norms, mean, var):
+        assert torch.equal(m.running_mean, a) and torch.equal(m.running_var, b)
