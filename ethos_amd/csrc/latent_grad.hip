@@ -17,8 +17,8 @@
 // one another with a barrier between, so that per tile of 64 and SIMD about 13,000 cycles of MFMA
 // and 26,000 of VALU (gelu', the splits) hardly overlap, with two waves to hide any latency.
 // Measured, 200,070 experts of 512 hidden values: 318 us and 20 us to add up the workgroups' d W1,
-// against 502 us as products (dpre 201, d latents 175, d W1 116 + 10);
-// 512 tokens' 108 + 16 against 185, 128 tokens' (16,384 pairs) 36 + 12 against 94.
+// against 502 us as products (dpre 201, d latents 175, d W1 116 + 10); for 512 tokens' pairs 108
+// and 16 against 185, for 128 tokens' (16,384 pairs) 36 and 12 against 94.
 // W1's fragments are requested a phase ahead: 350 us when each was requested where it is used.
 #include "ethos_common.hpp"
 #include "ethos_gelu.hpp"
@@ -113,7 +113,8 @@ __global__ __launch_bounds__(kLgThreads, 2) void latent_grad_kernel(const float*
         int32_t id = id_of(m0), next_id = id_of(m0 + step);
         load_z(id);
         load_d(m0, 0);
-        // W1's fragments of a pass, requested a phase before their use (again for each tile)
+        // W1's fragments of a pass, four steps at a time, requested a phase or a group of products
+        // before their use (again for each tile)
         bf16x8_t fw[8], fp[16];
         auto load_w = [&](int pass, int k0) {
             const unsigned at = fresh(tid & 63) * 8;
