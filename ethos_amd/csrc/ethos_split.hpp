@@ -7,8 +7,7 @@ namespace ethos {
 
 // Two float32 values -> their three bf16 planes, one packed word each (a low, b high): the upper
 // half (truncated, so that no finite value becomes an infinity), then the remainder and what is
-// left of it, both to nearest, so that the products left out have either sign (all truncated,
-// they would add up to 2^-23 of the result).  An infinity keeps its remainders at zero; a NaN
+// left of it, both to nearest; their sum is the value.  An infinity keeps its remainders at zero; a NaN
 // leaves one in the second plane.
 __device__ __forceinline__ void split3(float a, float b, uint32_t& hi, uint32_t& mid, uint32_t& lo) {
     const uint32_t ua = __float_as_uint(a), ub = __float_as_uint(b);

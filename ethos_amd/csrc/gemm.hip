@@ -1,12 +1,13 @@
 // Float32 matrix products (training path, float32 generator) on the bf16 matrix cores.
 //
-// A float32 operand is split exactly into three bf16 values x = hi + mid + lo (8 significant
-// bits each, 24 in all), so that its product with a bf16 operand is three bf16 MFMAs whose
-// products are exact in float32; two float32 operands take the six products down to 2^-16 of
-// the result (the three left out are about 2^-26 of it, of either sign).  The sums are float32,
-// as in a float32 GEMM; the bf16 MFMAs run at 16 times the float32 MFMAs' rate, so three of
-// them cost a fifth of one float32 product.  Error against float64 (k = 128 | 512, two float32
-// operands): 1.7e-7 | 3.5e-7, by float32 MFMAs 2.1e-7 | 4.0e-7.
+// A float32 operand is split into three bf16 values x = hi + mid + lo (8 significant bits each,
+// 24 in all: exact down to 2^-110, where lo leaves bf16's range), so that its product with a bf16
+// operand is three bf16 MFMAs whose products are exact in float32, and two float32 operands take
+// nine.  The sums are float32, as in a float32 GEMM; the bf16 MFMAs run at 16 times the float32
+// MFMAs' rate, so three of them cost a fifth of one float32 product and nine a little over half.
+// Six of the nine (down to 2^-16 of the result) leave out up to 2^-22 of a product that a float32
+// multiply-add keeps; all nine cost the float32 layer of 256 tokens 114.9 us against 113.3, and
+// a training step of 500 tokens nothing that shows.
 //
 // What bounds it: at these shapes (n or k of 128 to 2,048) a step's loads, which are waited for
 // before the step's products.  So many workgroups per CU rather than many steps in flight per
@@ -275,7 +276,6 @@ __global__ __launch_bounds__(kGemmThreads, (BM > 64 ? (sizeof(TB) == 4 ? 3 : 4) 
                 // smallest products first
 #pragma unroll
                 for (int q = PA + PB - 2; q >= 0; --q) {
-                    if (q > 2) continue;
 #pragma unroll
                     for (int qa = 0; qa < PA; ++qa) {
                         const int qb = q - qa;

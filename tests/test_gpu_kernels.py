@@ -755,6 +755,26 @@ def test_generate_fp32_products(U, max_u, E, dl, dh, d):
     assert float((v[:U].cpu().double() - vr).norm()) <= 1e-6 * float(vr.norm()) + 1e-30
 
 
+@pytest.mark.parametrize("dl,U", [(8, 5), (16, 300)])
+def test_generate_fp32_products_keep_every_bit(dl, U):
+    """float32 operands whose lower bits are as large as they can be, all of one sign, in sums of
+    8 and 16 terms (one step of the matrix cores): no partial product may be left out.  A sum of
+    nine exact partial results rounds nine times, of which only the last three at more than 2^-8
+    of it: within 2^-22.5 of the result, where leaving out the smallest three is 2^-22 by itself."""
+    from ethos_amd import hip
+    g = torch.Generator().manual_seed(dl)
+    # 1 + (2^-7 - 2^-14) + 2^-16 and neighbours: 8 bits, then 8 bits just below one of theirs, then
+    # a last part of nearly half of one of those
+    top = 1.0 + 2.0 ** -7 - 2.0 ** -15 * torch.randint(1, 5, (U + dl * 64,), generator=g) + 2.0 ** -16 - 2.0 ** -22
+    lat = top[:U, None].expand(U, dl).contiguous().float()
+    w1 = top[U:].view(64, dl).float()
+    n_u = torch.tensor([U], dtype=torch.int32).cuda()
+    h, _ = hip.generate(lat.cuda(), torch.arange(U, dtype=torch.int32).cuda(), n_u, U, w1.cuda(), torch.zeros(64, 64).cuda(), with_v=False)
+    ref = lat.double() @ w1.double().T  # above 8, where the GELU is the identity in float32
+    err = float(((h.cpu().double() - ref) / ref).abs().max())
+    assert err < 2.0 ** -22.5, err
+
+
 @pytest.mark.parametrize("dt,dq,K,rows", [("bf16", 256, 512, 2049), ("bf16", 256, 512, 8193), ("bf16", 512, 512, 9000),
                                           ("bf16", 512, 512, 16384), ("fp32", 64, 100, 2050), ("fp32", 256, 512, 8192)])
 def test_route_rows_per_wave_agree(dt, dq, K, rows):
