@@ -7,7 +7,9 @@
 // MFMAs' rate, so three of them cost a fifth of one float32 product and nine a little over half.
 // Six of the nine (down to 2^-16 of the result) leave out up to 2^-22 of a product that a float32
 // multiply-add keeps; all nine cost the float32 layer of 256 tokens 114.9 us against 113.3, and
-// a training step of 500 tokens nothing that shows.
+// a training step of 500 tokens nothing that shows.  A sum with an infinity in it comes out as NaN
+// and is taken again as a float32 chain (the step of 4,096 tokens with one infinite output gradient,
+// whose gradients are then NaN nearly everywhere: 2.3 -> 3.3 ms).
 //
 // What bounds it: at these shapes (n or k of 128 to 2,048) a step's loads, which are waited for
 // before the step's products.  So many workgroups per CU rather than many steps in flight per
@@ -203,6 +205,42 @@ __host__ __device__ inline GemmGroups gemm_groups(int split, int64_t mt, int nt)
     return split >= 8 ? GemmGroups{split, (int)mt * nt} : GemmGroups{split * mt, nt};
 }
 
+// The rows of C in use and one part's [kb, ke) of the reduction (all of it when not split).
+struct GemmRange {
+    int64_t m, kb, ke;
+};
+__device__ __forceinline__ GemmRange gemm_range(const Gemm& p, int part_id) {
+    GemmRange r{p.m, 0, p.k};
+    if (p.dyn) {
+        const int64_t d = *p.dyn;
+        if (p.dyn_k) r.ke = d < r.ke ? d : r.ke;
+        else r.m = d < r.m ? d : r.m;
+    }
+    if (p.split > 1) {
+        const int64_t k = r.ke, per = ((k + p.split - 1) / p.split + kGemmK - 1) / kGemmK * kGemmK;
+        r.kb = per * part_id;
+        r.ke = r.kb + per < k ? r.kb + per : k;
+    }
+    return r;
+}
+
+// One output's sum over a part of the reduction as a float32 chain: what an infinity needs, which
+// against the other operand's lower planes gives NaNs (times zero) and infinities of either sign.
+template <typename TA, bool AK, typename TB, bool BK, bool IDX>
+__device__ __forceinline__ float gemm_chain(const Gemm& p, int64_t m, int n, int part_id) {
+    const GemmRange r = gemm_range(p, part_id);
+    const int64_t row = IDX && AK ? (int64_t)p.a_rows[m] : m;
+    const bool zeros = IDX && AK && (row < 0 || row >= p.a_limit);
+    float s = 0.0f;
+    for (int64_t k = r.kb; k < r.ke && s == s; ++k) {  // (a NaN stays one)
+        const int64_t kr = IDX && !BK ? (int64_t)p.b_rows[k] : k;
+        const float a = zeros ? 0.0f : Elem<TA>::to_f32(((const TA*)p.a)[AK ? row * p.lda + k : k * p.lda + row]);
+        const float b = Elem<TB>::to_f32(((const TB*)p.b)[BK ? (int64_t)n * p.ldb + k : kr * p.ldb + n]);
+        s = __builtin_fmaf(a, b, s);
+    }
+    return s;
+}
+
 template <typename TA, bool AK, typename TB, bool BK, bool IDX, int BM, int BN>
 __global__ __launch_bounds__(kGemmThreads, (BM > 64 ? (sizeof(TB) == 4 ? 3 : 4) : 4)) void gemm_kernel(Gemm p) {
     constexpr int PA = Planes<TA>::kN, PB = Planes<TB>::kN;
@@ -211,12 +249,6 @@ __global__ __launch_bounds__(kGemmThreads, (BM > 64 ? (sizeof(TB) == 4 ? 3 : 4) 
     __shared__ __align__(16) uint16_t lds[kBuf];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    int64_t m = p.m, k = p.k;
-    if (p.dyn) {
-        const int64_t d = *p.dyn;
-        if (p.dyn_k) k = d < k ? d : k;
-        else m = d < m ? d : m;
-    }
     const int nt = (p.n + BN - 1) / BN;
     const int64_t mt = (p.m + BM - 1) / BM;
     const GemmGroups gg = gemm_groups(p.split, mt, nt);
@@ -225,14 +257,9 @@ __global__ __launch_bounds__(kGemmThreads, (BM > 64 ? (sizeof(TB) == 4 ? 3 : 4) 
     const int part_id = (int)(tile / (mt * nt));
     const int64_t m0 = tile / nt % mt * BM;
     const int n0 = (int)(tile % nt) * BN;
+    const GemmRange range = gemm_range(p, part_id);
+    const int64_t m = range.m, kb = range.kb, ke = range.ke;
     if (group >= gg.groups || m0 >= m) return;
-    // this workgroup's part of the reduction (all of it when not split)
-    int64_t kb = 0, ke = k;
-    if (p.split > 1) {
-        const int64_t per = ((k + p.split - 1) / p.split + kGemmK - 1) / kGemmK * kGemmK;
-        kb = per * part_id;
-        ke = kb + per < k ? kb + per : k;
-    }
     f32x16_t acc[MI][NI];
 #pragma unroll
     for (int i = 0; i < MI; ++i)
@@ -293,6 +320,20 @@ __global__ __launch_bounds__(kGemmThreads, (BM > 64 ? (sizeof(TB) == 4 ? 3 : 4) 
     }
 
     float* part = p.split > 1 ? p.part + (size_t)part_id * (size_t)p.m * (size_t)p.n : nullptr;
+    auto emit = [&](int64_t mm, int n, float v, float bias, float aux) {
+        if (part) {
+            part[p.transposed ? (int64_t)n * p.m + mm : mm * p.n + n] = v;
+            return;
+        }
+        const int64_t row = p.c_rows ? p.c_rows[mm] : mm;
+        const int64_t at = p.transposed ? n * p.ldc + row : row * p.ldc + n;
+        if (p.epilogue == kGemmGeluGrad) ((float*)p.c)[at] = gelu_erf_grad(v) * aux;
+        else if (p.epilogue == kGemmGelu) ((float*)p.c)[at] = gelu_erf(v);
+        else if (p.out_bf16) ((uint16_t*)p.c)[at] = f32_to_bf16_bits(__builtin_fmaf(p.alpha, v, bias));
+        else ((float*)p.c)[at] = __builtin_fmaf(p.alpha, v, bias);
+    };
+    constexpr bool kPlanes = PA + PB > 2;
+    uint64_t again = 0;  // (planes) this thread's outputs (j, i, g) that came out as NaN
 #pragma unroll
     for (int j = 0; j < NI; ++j) {
         const int n = n0 + wn + j * 32 + (lane & 31);
@@ -301,7 +342,7 @@ __global__ __launch_bounds__(kGemmThreads, (BM > 64 ? (sizeof(TB) == 4 ? 3 : 4) 
 #pragma unroll
         for (int i = 0; i < MI; ++i) {
             const int64_t mb = m0 + wm + i * 32;
-            float aux[16];
+            float aux[16] = {};
             if (p.epilogue == kGemmGeluGrad) {
                 // all sixteen requested before any is used
 #pragma unroll
@@ -315,18 +356,19 @@ __global__ __launch_bounds__(kGemmThreads, (BM > 64 ? (sizeof(TB) == 4 ? 3 : 4) 
             for (int g = 0; g < 16; ++g) {
                 const int64_t mm = mb + mfma32_row(g, lane);
                 if (mm >= m) continue;
-                const float v = acc[i][j][g];
-                if (part) {
-                    part[p.transposed ? (int64_t)n * p.m + mm : mm * p.n + n] = v;
-                    continue;
-                }
-                const int64_t row = p.c_rows ? p.c_rows[mm] : mm;
-                const int64_t at = p.transposed ? n * p.ldc + row : row * p.ldc + n;
-                if (p.epilogue == kGemmGeluGrad) ((float*)p.c)[at] = gelu_erf_grad(v) * aux[g];
-                else if (p.epilogue == kGemmGelu) ((float*)p.c)[at] = gelu_erf(v);
-                else if (p.out_bf16) ((uint16_t*)p.c)[at] = f32_to_bf16_bits(__builtin_fmaf(p.alpha, v, bias));
-                else ((float*)p.c)[at] = __builtin_fmaf(p.alpha, v, bias);
+                if (kPlanes && acc[i][j][g] != acc[i][j][g]) again |= 1ull << ((j * MI + i) * 16 + g);
+                else emit(mm, n, acc[i][j][g], bias, aux[g]);
             }
+        }
+    }
+    if constexpr (kPlanes) {
+        for (; again != 0; again &= again - 1) {
+            const int e = __builtin_ctzll(again), g = e & 15, i = (e >> 4) % MI, j = (e >> 4) / MI;
+            const int64_t mm = m0 + wm + i * 32 + mfma32_row(g, lane);
+            const int n = n0 + wn + j * 32 + (lane & 31);
+            const float bias = p.bias ? Elem<TB>::to_f32(((const TB*)p.bias)[n]) : 0.0f;
+            const float aux = p.epilogue == kGemmGeluGrad ? ((const float*)p.c)[mm * p.ldc + n] : 0.0f;
+            emit(mm, n, gemm_chain<TA, AK, TB, BK, IDX>(p, mm, n, part_id), bias, aux);
         }
     }
 }

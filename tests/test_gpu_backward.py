@@ -251,6 +251,31 @@ def test_expert_grads_entry_point(dt, n, H, k, dl, dh, d, E):
     assert not got[2].cpu()[unused].any()
 
 
+@pytest.mark.parametrize("dt", ["fp32", "bf16"])
+def test_expert_grads_infinite_output_gradient(dt):
+    """One infinite value of dy: its column of d W_v is the infinity times each sum of hidden
+    rows, with that sum's sign, and the other columns are those of a finite dy."""
+    from ethos_amd import hip
+    g = torch.Generator().manual_seed(5)
+    n, H, k, dl, dh, d, E = 70, 2, 4, 16, 72, 40, 50
+    tdt = torch.bfloat16 if dt == "bf16" else torch.float32
+    rn = lambda *s: torch.randn(s, generator=g).to(tdt)  # noqa: E731
+    seg = hip.sort_segment(torch.randint(0, E, (n * H * k,), generator=g, dtype=torch.int32).cuda(), E)
+    x, dy, lat, w1, w2 = rn(n, d), rn(n, d), rn(E, dl), rn(dh, dl), rn(2 * d, dh)
+    h, gates = rn(seg["uniq"].numel(), dh), torch.rand(n, H, k, generator=g).to(tdt).cuda()
+    args = [t.cuda() for t in (x, dy, h, lat, w1, w2)]
+    plain = hip.expert_grads(*args, seg, gates, H, k)[4][d:]
+    alone = torch.zeros(n, d, dtype=tdt, device="cuda")
+    alone[31, 9] = 1.0
+    sign = torch.sign(hip.expert_grads(args[0], alone, *args[2:], seg, gates, H, k)[4][d + 9].float())
+    assert int((sign > 0).sum()) > 10 and int((sign < 0).sum()) > 10
+    args[1][31, 9] = float("inf")
+    got = hip.expert_grads(*args, seg, gates, H, k)[4][d:]
+    assert torch.equal(got[9].float(), sign * float("inf"))
+    rest = torch.arange(d, device="cuda") != 9
+    assert torch.equal(got[rest], plain[rest])
+
+
 @pytest.mark.parametrize("dt,n,d,H,dq,K,k,batch", [
     ("bf16", 2, 8, 1, 8, 3, 1, True), ("bf16", 37, 72, 3, 96, 37, 5, True), ("bf16", 300, 200, 2, 272, 64, 32, False),
     ("bf16", 1100, 256, 8, 512, 512, 16, True), ("fp32", 1, 8, 2, 16, 2, 2, False), ("fp32", 129, 40, 4, 64, 65, 9, True),

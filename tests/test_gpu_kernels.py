@@ -775,6 +775,28 @@ def test_generate_fp32_products_keep_every_bit(dl, U):
     assert err < 2.0 ** -22.5, err
 
 
+@pytest.mark.parametrize("short", [True, False])
+def test_generate_fp32_infinities(short):
+    """A latent row with an infinity gives what float32 products give, infinities and NaNs where
+    they do: with weights of 8 significant bits (whose lower parts are zeros) and of all 24."""
+    from ethos_amd import hip
+    g = torch.Generator().manual_seed(3)
+    U, dl, dh = 150, 24, 160
+    lat, w1 = torch.randn(U, dl, generator=g), torch.randn(dh, dl, generator=g)
+    w1 = w1.bfloat16().float() if short else w1
+    lat[7, 3], lat[9, 0], lat[11, 5], lat[100, 1] = float("inf"), float("-inf"), float("nan"), float("inf")
+    lat[100, 2] = float("-inf")
+    w1[5, 3] = 0.0
+    n_u = torch.tensor([U], dtype=torch.int32).cuda()
+    h, _ = hip.generate(lat.cuda(), torch.arange(U, dtype=torch.int32).cuda(), n_u, U, w1.cuda(), torch.zeros(64, dh).cuda(), with_v=False)
+    h, ref = h.cpu().double(), torch.nn.functional.gelu(lat.double() @ w1.double().T)
+    odd = ~torch.isfinite(ref)
+    assert int((ref == float("inf")).sum()) > 100 and int(torch.isnan(ref).sum()) > 300
+    assert torch.equal(torch.isnan(h), torch.isnan(ref))
+    assert torch.equal(h[odd & ~torch.isnan(ref)], ref[odd & ~torch.isnan(ref)])
+    assert float((h[~odd] - ref[~odd]).norm()) <= 1e-6 * float(ref[~odd].norm())
+
+
 @pytest.mark.parametrize("dt,dq,K,rows", [("bf16", 256, 512, 2049), ("bf16", 256, 512, 8193), ("bf16", 512, 512, 9000),
                                           ("bf16", 512, 512, 16384), ("fp32", 64, 100, 2050), ("fp32", 256, 512, 8192)])
 def test_route_rows_per_wave_agree(dt, dq, K, rows):
