@@ -20,6 +20,7 @@ def _stream_fast() -> int:
 # The current device's current stream as a hipStream_t; the raw accessor skips the Python
 # device bookkeeping of torch.cuda.current_stream (a few microseconds per call).
 _stream = _stream_fast if hasattr(torch._C, "_cuda_getCurrentRawStream") else _stream_slow
+_current_device = getattr(torch._C, "_cuda_getDevice", torch.cuda.current_device)
 
 
 def _need(t: torch.Tensor, name: str, dtype=None, dim=None) -> None:
@@ -577,10 +578,12 @@ def layer_forward(x: torch.Tensor, packed, key_norms: torch.Tensor, keys_prepare
 # ----------------------------------------------------------- the language model's blocks
 def plain(*ts) -> bool:
     """Whether a library call may stand in for torch operations on these tensors: ordinary HIP
-    tensors of one supported dtype and device, with nothing that follows the operations
-    themselves (gradients, forward-mode derivatives, autocast, tracing, transforms, modes)."""
+    tensors of one supported dtype on the current device (a call goes to that device's stream),
+    with nothing that follows the operations themselves (gradients, forward-mode derivatives,
+    autocast, tracing, transforms, modes)."""
     t0 = ts[0]
-    if t0.dtype not in (torch.bfloat16, torch.float32) or t0.device.type != "cuda":
+    if (t0.dtype not in (torch.bfloat16, torch.float32) or t0.device.type != "cuda"
+            or t0.device.index != _current_device()):
         return False
     grad = torch.is_grad_enabled()
     for t in ts:

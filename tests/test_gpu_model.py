@@ -232,3 +232,27 @@ def test_block_with_and_without_gradients_agree():
     z = z.detach()
     assert y.grad_fn is None
     assert float((y.float() - z.float()).norm() / z.float().norm()) < 1e-2
+
+
+def test_blocks_on_another_device_stay_torch_operations(monkeypatch):
+    """A library call goes to the current device's stream: norms, FFN and attention whose tensors
+    are on another device than the current one (here: the current one taken for the second) are
+    torch operations."""
+    from ethos_amd import hip
+    from ethos_amd.model import TransformerBlock, lm_config
+    torch.manual_seed(0)
+    block = TransformerBlock(lm_config(), False).cuda().bfloat16()
+    x, pos = torch.randn(1, 33, 1024, device="cuda").bfloat16(), torch.arange(33, device="cuda")
+    with torch.no_grad():
+        y = block(x, None, pos)
+        called = []
+        for name in ("rms_norm", "swiglu", "mla_attention"):
+            monkeypatch.setattr(hip, name, lambda *a, name=name: called.append(name))
+        block(x, None, pos)
+        assert set(called) == {"rms_norm", "swiglu", "mla_attention"}
+        called.clear()
+        monkeypatch.setattr(hip, "_current_device", lambda: 1)
+        assert not hip.plain(x)
+        z = block(x, None, pos)
+        assert not called
+    assert float((y.float() - z.float()).norm() / z.float().norm()) < 1e-2
