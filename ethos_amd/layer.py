@@ -244,6 +244,7 @@ class ProductKeyRouter(nn.Module):
         self.sub_keys_2 = nn.Embedding(self.num_sub_keys, self.d_query // 2)
         self._cache_key = None
         self._cache = None
+        self._train_pass = 0
         self._bn_key = None
         self._bn = None
         self._identity = None
@@ -251,7 +252,7 @@ class ProductKeyRouter(nn.Module):
         self._keys_prepared = None
         self._wq_prepared = None
 
-    # -- parameter packing (cached until a parameter changes) ---------------------
+    # -- parameter packing (cached until a parameter changes; made anew by every training pass) ---
     def _weight_sources(self) -> list:
         """The projection weights and sub-keys, read from the modules' parameter dicts directly
         (this runs on every call; nn.Module attribute lookup is slow)."""
@@ -271,8 +272,16 @@ class ProductKeyRouter(nn.Module):
         """The tensors the packed form is built from."""
         return self._weight_sources() + self._bn_sources()
 
-    def _packed_weights(self, dtype: torch.dtype, device: torch.device):
-        key = (dtype, device, tuple((t.data_ptr(), t._version) for t in self._weight_sources() if t is not None))
+    def _pack_mode(self) -> int:
+        """Part of the packed forms' keys.  Evaluation (0) trusts the parameters' version counters.
+        A training pass has its own number: between two of them an optimizer may write through
+        `.data` or pointers, which moves no counter, so each packs anew, and so does the first
+        evaluation after them."""
+        return self._train_pass if any(m.training for m in self._modules["query_norms"]._modules.values()) else 0
+
+    def _packed_weights(self, dtype: torch.dtype, device: torch.device, mode: int | None = None):
+        key = (dtype, device, self._pack_mode() if mode is None else mode,
+               tuple((t.data_ptr(), t._version) for t in self._weight_sources() if t is not None))
         if key != self._cache_key:
             wq = torch.stack([m.weight.detach() for m in self.query_projs]).to(device=device, dtype=dtype).contiguous()
             bq = torch.stack([m.bias.detach() for m in self.query_projs]).to(device=device, dtype=dtype).contiguous()
@@ -308,7 +317,8 @@ class ProductKeyRouter(nn.Module):
         return self._bn
 
     def _packed(self, dtype: torch.dtype, device: torch.device):
-        return self._packed_weights(dtype, device) + tuple(self._bn_coefficients(device))
+        """What an evaluation reads: the packed weights and the BatchNorm coefficients."""
+        return self._packed_weights(dtype, device, 0) + tuple(self._bn_coefficients(device))
 
     def _bn_uses_batch_stats(self) -> bool:
         return any(m.training or not m.track_running_stats for m in self._modules["query_norms"]._modules.values())
@@ -335,7 +345,10 @@ class ProductKeyRouter(nn.Module):
             return hip.query_proj(x_flat, wq, bq, alpha, beta, prepared=self._wq_prepared)
         # Training-mode BatchNorm normalises with batch statistics and updates the
         # running stats: project with an identity affine, then normalise the projected queries.
-        wq, bq = (packed if packed is not None else self._packed_weights(x_flat.dtype, x_flat.device))[:2]
+        if packed is None:
+            self._train_pass += 1
+            packed = self._packed_weights(x_flat.dtype, x_flat.device)
+        wq, bq = packed[:2]
         if self._identity is None or self._identity[0].device != x_flat.device:
             ones = torch.ones((self.num_heads, self.d_query), dtype=torch.float32, device=x_flat.device)
             self._identity = (ones, torch.zeros_like(ones))
@@ -385,6 +398,7 @@ class ProductKeyRouter(nn.Module):
         """(gates [n, H, k] x.dtype, expert ids [n, H, k] int32).  `mark(stage)`, if given,
         is called after each stage is enqueued (used to place timing events)."""
         if self._bn_uses_batch_stats():
+            self._train_pass += 1
             packed = self._packed_weights(x_flat.dtype, x_flat.device)
         else:
             packed = self._packed(x_flat.dtype, x_flat.device)
@@ -476,11 +490,13 @@ class EthosExpertLayer(nn.Module):
             self._modules["expert_latents"]._parameters["weight"], gen["0"]._parameters["weight"],
             gen["2"]._parameters["weight"]]
 
-    def _generator_params(self, dtype, device):
+    def _generator_params(self, dtype, device, mode: int | None = None):
         """(latents, W1, W2, W_u^T): the generator weights in the layer dtype on the device,
-        and (bf16) the transpose of W2's first d_model rows, cached until a weight changes."""
+        and (bf16) the transpose of W2's first d_model rows, cached until a weight changes (as
+        ProductKeyRouter._pack_mode says)."""
         ps = (self.expert_latents.weight, self.generation_network.net[0].weight, self.generation_network.net[2].weight)
-        key = (dtype, device, tuple((p.data_ptr(), p._version) for p in ps))
+        mode = self._modules["router"]._pack_mode() if mode is None else mode
+        key = (dtype, device, mode, tuple((p.data_ptr(), p._version) for p in ps))
         if key != self._gen_key:
             if all(p.dtype == dtype and p.device == device and p.is_contiguous() for p in ps):
                 gen = tuple(p.detach() for p in ps)
@@ -528,7 +544,7 @@ class EthosExpertLayer(nn.Module):
         if mark is None and side_stream is None and x_flat.shape[0] > 0 and not router._bn_uses_batch_stats():
             with torch.no_grad():
                 packed = router._packed(x_flat.dtype, x_flat.device)
-                gen = self._generator_params(x_flat.dtype, x_flat.device)
+                gen = self._generator_params(x_flat.dtype, x_flat.device, 0)
                 return hip.layer_forward(x_flat, packed, router._key_norms, router._keys_prepared, router._wq_prepared, gen,
                                          self.num_experts, self.top_k, self.hidden_space)
         with torch.no_grad():

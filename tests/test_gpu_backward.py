@@ -410,3 +410,39 @@ def test_training_queries_are_per_head_batch_norms(n, H, dq):
     assert torch.equal(q, ref)
     for m, a, b in zip(norms, mean, var):
         assert torch.equal(m.running_mean, a) and torch.equal(m.running_var, b)
+
+
+@pytest.mark.parametrize("name", ["tiny_fp32", "tiny"])
+def test_training_sees_weights_written_without_a_version_step(name):
+    """A training pass, and the first evaluation after one, read the parameters as they are, also
+    where an optimizer wrote them through `.data`: outputs and gradients are those of a new module
+    with the same values."""
+    sh = SHAPES[name]
+    x, sd = make_inputs(sh, signal=True)
+    xd = x.cuda().view(sh.batch, -1, sh.d_model)
+
+    def new(state, train):
+        m = ethos_amd.EthosExpertLayer(sh.config()).to(sh.torch_dtype)
+        m.load_state_dict(state)
+        return m.cuda().train(train)
+
+    def step(m):
+        m.zero_grad()
+        y = m(xd)
+        y.float().square().sum().backward()
+        return [y.detach()] + [p.grad.clone() for p in m.parameters()]
+
+    m = new(sd, True)
+    step(m)
+    for _ in range(2):
+        versions = [p._version for p in m.parameters()]
+        for p in m.parameters():
+            p.data.mul_(1.25)
+        assert versions == [p._version for p in m.parameters()]
+        state = {k: v.clone() for k, v in m.state_dict().items()}
+        for a, b in zip(step(m), step(new(state, True))):
+            assert torch.equal(a, b)
+    for p in m.parameters():
+        p.data.mul_(0.75)
+    with torch.no_grad():
+        assert torch.equal(m.eval()(xd), new(m.state_dict(), False)(xd))
