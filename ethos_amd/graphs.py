@@ -11,8 +11,9 @@ expert stages; on ROCm 7 the fork and join cost more GPU time than the overlap s
 tokens: 0.167 against 0.153 ms per replayed step), so it is off by default.
 
 The replay gives the eager forward's output bit for bit (the same kernels on the same
-inputs).  The graph holds the layer's packed parameters by address: when a parameter or a
-BatchNorm buffer changes (its version counter moves), the next call captures again.
+inputs).  The graph reads the layer's packed parameters by address and keeps them alive: when a
+parameter or a BatchNorm buffer changes (its version counter, or the count of training batches,
+moves), the next call captures again.
 """
 from __future__ import annotations
 
@@ -50,8 +51,12 @@ class CapturedLayer:
         self._capture()
 
     def _state(self):
-        # looked up afresh on every call: a parameter replaced by a new object counts as a change
-        return tuple((t.data_ptr(), t._version) for t in self.layer._param_sources() if t is not None)
+        # looked up afresh on every call: a parameter replaced by a new object counts as a change.
+        # A training pass writes the running statistics without moving their counters, but moves
+        # that of the batch counts.
+        layer = self.layer
+        ts = layer._param_sources() + layer._modules["router"]._batch_counts()
+        return tuple((t.data_ptr(), t._version) for t in ts if t is not None)
 
     def _capture(self) -> None:
         layer = self.layer
@@ -69,6 +74,9 @@ class CapturedLayer:
         self.graph = torch.cuda.CUDAGraph()
         with torch.no_grad(), torch.cuda.graph(self.graph):
             self.output = layer.forward_flat(self.input, side_stream=side)
+        # what the graph reads by address, kept here: the layer may pack again for other calls
+        # (another dtype, a training pass) while the graph stays valid
+        self._holds = layer.packed_tensors()
         self._key = self._state()
 
     def __call__(self, x: torch.Tensor) -> torch.Tensor:

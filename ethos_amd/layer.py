@@ -268,6 +268,9 @@ class ProductKeyRouter(nn.Module):
             ts += (m._parameters["weight"], m._parameters["bias"], m._buffers["running_mean"], m._buffers["running_var"])
         return ts
 
+    def _batch_counts(self) -> list:
+        return [m._buffers["num_batches_tracked"] for m in self._modules["query_norms"]._modules.values()]
+
     def _packed_sources(self) -> list:
         """The tensors the packed form is built from."""
         return self._weight_sources() + self._bn_sources()
@@ -489,6 +492,11 @@ class EthosExpertLayer(nn.Module):
         return self._modules["router"]._packed_sources() + [
             self._modules["expert_latents"]._parameters["weight"], gen["0"]._parameters["weight"],
             gen["2"]._parameters["weight"]]
+
+    def packed_tensors(self) -> list:
+        """The packed forms that the last evaluation read."""
+        r = self.router
+        return [t for t in (*r._cache, *r._bn, r._key_norms, r._keys_prepared, r._wq_prepared, *self._gen) if t is not None]
 
     def _generator_params(self, dtype, device, mode: int | None = None):
         """(latents, W1, W2, W_u^T): the generator weights in the layer dtype on the device,

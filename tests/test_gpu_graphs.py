@@ -72,6 +72,51 @@ def test_captured_layer_recaptures_after_a_parameter_change():
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("eager_between", [False, True])
+def test_captured_layer_recaptures_after_new_running_statistics(eager_between):
+    """Training-mode passes without an optimizer step change only the BatchNorms' running
+    statistics (whose version counters stand still): the next call captures again, also after an
+    eager evaluation of other data has packed the new statistics."""
+    sh = SHAPES["cfg3"]
+    _, sd = make_inputs(sh, signal=True)
+    m = _layer(sh, sd)
+    cap = CapturedLayer(m, sh.n_tok)
+    x, other = _inputs(sh, 2)
+    before, graph = cap(x).clone(), cap.graph
+    with torch.no_grad():
+        m.train()
+        for _ in range(20):
+            m.forward_flat(other * 3)
+        m.eval()
+        if eager_between:
+            m.forward_flat(other)
+        got = cap(x).clone()
+        want = m.forward_flat(x)
+    torch.cuda.synchronize()
+    assert cap.graph is not graph
+    assert torch.equal(got, want) and not torch.equal(got, before)
+
+
+@pytest.mark.gpu
+def test_captured_layer_keeps_what_its_graph_reads():
+    """An eager pass in another dtype packs the parameters again; the replayed graph reads the
+    earlier packed forms, which no later allocation may take over."""
+    sh = SHAPES["cfg3"]
+    _, sd = make_inputs(sh, signal=True)
+    m = _layer(sh, sd)
+    cap = CapturedLayer(m, sh.n_tok)
+    x = _inputs(sh, 1)[0]
+    before, graph = cap(x).clone(), cap.graph
+    with torch.no_grad():
+        m.forward_flat(x.float())
+    fill = [torch.full((1 << k,), float("nan"), device="cuda") for k in range(10, 23) for _ in range(4)]
+    got = cap(x)
+    torch.cuda.synchronize()
+    assert cap.graph is graph and torch.equal(got, before)
+    del fill
+
+
+@pytest.mark.gpu
 def test_captured_layer_rejects_other_shapes():
     sh = SHAPES["tiny"]
     _, sd = make_inputs(sh)
