@@ -112,16 +112,23 @@ class _GatePath(torch.autograd.Function):
         rest = ctx.saved_tensors[4:]
         stats, params = (None, rest) if ctx.batch else (rest[:2], rest[2:])
         H = wq.shape[0]
-        w, b, (k1, k2) = params[0:2 * H:2], params[1:2 * H:2], params[2 * H:2 * H + 2]
-        gamma, beta = params[2 * H + 2:3 * H + 2], params[3 * H + 2:]
         head = (None,) * 6
+
+        def split(ps):  # projection weights, biases, both sub-key tables, BatchNorm weights, biases
+            return ps[0:2 * H:2], ps[1:2 * H:2], ps[2 * H:2 * H + 2], ps[2 * H + 2:3 * H + 2], ps[3 * H + 2:]
+
         if torch.is_grad_enabled():  # create_graph: the torch operations' own derivative
-            g = _gate_values(x, ids.long(), w, b, gamma, beta, k1, k2,
+            # with respect to a view of each argument, which ends there: heads may share a
+            # parameter, and x may itself come from one
+            need = (ctx.needs_input_grad[0], *ctx.needs_input_grad[7:])
+            ts = [t.view_as(t) if n else t for t, n in zip((x, *params), need)]
+            w, b, (k1, k2), gamma, beta = split(ts[1:])
+            g = _gate_values(ts[0], ids.long(), w, b, gamma, beta, k1, k2,
                              [None] * H if stats is None else list(zip(*stats)), [ctx.eps] * H)
-            ts = [x, *params]
-            want = [t for t, need in zip(ts, (ctx.needs_input_grad[0], *ctx.needs_input_grad[7:])) if need]
-            got = dict(zip(map(id, want), torch.autograd.grad(g, want, dg, create_graph=True, allow_unused=True)))
-            return (got.get(id(x)), *head, *(got.get(id(t)) for t in params))
+            got = iter(torch.autograd.grad(g, [t for t, n in zip(ts, need) if n], dg, create_graph=True, allow_unused=True))
+            out = [next(got) if n else None for n in need]
+            return (out[0], *head, *out[1:])
+        w, b, (k1, k2), gamma, beta = split(params)
         dx, dw, db, dgamma, dbeta, dk1, dk2 = hip.gate_grads(
             x, ids, dg.contiguous(), wq, bq, k1.detach(), k2.detach(), [t.detach() for t in gamma], [t.detach() for t in beta],
             stats and list(stats[0]), stats and list(stats[1]), ctx.eps, want_x=ctx.needs_input_grad[0],

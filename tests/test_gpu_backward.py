@@ -386,6 +386,34 @@ def test_router_second_derivative(train):
         assert _nerr(a, b) < 1e-5
 
 
+@pytest.mark.parametrize("train", [False, True])
+def test_router_second_derivative_of_shared_parameters(train):
+    """Two heads with one projection, one table for both sub-key halves, and rows that are
+    themselves computed from a parameter of the router: create_graph counts each use once, as
+    torch's own graph of gate_path does."""
+    sh = SHAPES["tiny_fp32"]
+    x, sd = make_inputs(sh, signal=True)
+    m = ethos_amd.EthosExpertLayer(sh.config())
+    m.load_state_dict(sd)
+    r = m.cuda().train(train).router
+    r.query_projs[1] = r.query_projs[0]
+    r.sub_keys_2 = r.sub_keys_1
+    leaves_ = [r.query_projs[0].weight, r.query_projs[0].bias, r.sub_keys_1.weight, r.query_norms[0].weight]
+    w = torch.randn(sh.n_tok, sh.num_heads, sh.top_k, generator=torch.Generator().manual_seed(2)).cuda()
+    both = []
+    for own in (True, False):
+        xd = x.cuda() * (1.0 + r.sub_keys_1.weight.mean())
+        with torch.no_grad():
+            _, ids = r(xd)
+        s = r(xd)[0] if own else r.gate_path(xd, ids)
+        first = torch.autograd.grad((s * w).sum(), leaves_, create_graph=True)
+        both.append(first + torch.autograd.grad(sum((t ** 2).sum() for t in first), leaves_, retain_graph=True))
+    # a projection's bias has no gradient under batch statistics: rounding alone on both sides
+    for i, (a, b) in enumerate(zip(*both)):
+        if not (train and i % 4 == 1):
+            assert _nerr(a, b) < 1e-5, i
+
+
 @pytest.mark.parametrize("n,H,dq", [(2, 8, 256), (500, 8, 256), (1024, 16, 256), (1025, 16, 256), (2048, 8, 256), (2049, 8, 256),
                                     (4096, 8, 256), (8192, 3, 256), (8193, 8, 256), (700, 4, 512), (3000, 5, 512),
                                     (33, 4, 128)])
