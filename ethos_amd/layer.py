@@ -28,6 +28,7 @@ cases; the reference's Triton layer (kernels.py:145-221) has no backward at all.
 """
 from __future__ import annotations
 
+import contextlib
 import math
 
 import numpy as np
@@ -53,6 +54,15 @@ def _bn_eval_coefficients(m: nn.BatchNorm1d, n: int):
     alpha = (w / np.sqrt(var + float(m.eps))).astype(np.float32)
     beta = (b - mu * alpha.astype(np.float64)).astype(np.float32)
     return alpha, beta
+
+
+@contextlib.contextmanager
+def _packing():
+    """Around the making of what is kept between calls: ordinary tensors without a graph, also where
+    the call that makes them runs under torch.inference_mode (a later one may save them for a
+    backward)."""
+    with torch.inference_mode(False), torch.no_grad():
+        yield
 
 
 def _gelu_grad(x: torch.Tensor) -> torch.Tensor:
@@ -293,16 +303,17 @@ class ProductKeyRouter(nn.Module):
         key = (dtype, device, self._pack_mode() if mode is None else mode,
                tuple((t.data_ptr(), t._version) for t in self._weight_sources() if t is not None))
         if key != self._cache_key:
-            wq = torch.stack([m.weight.detach() for m in self.query_projs]).to(device=device, dtype=dtype).contiguous()
-            bq = torch.stack([m.bias.detach() for m in self.query_projs]).to(device=device, dtype=dtype).contiguous()
-            k1 = self.sub_keys_1.weight.detach().to(device=device, dtype=dtype).contiguous()
-            k2 = self.sub_keys_2.weight.detach().to(device=device, dtype=dtype).contiguous()
-            self._key_norms = hip.key_norm_bounds(k1, k2)
-            # the sub-keys in the scoring MFMAs' fragment order
-            self._keys_prepared = hip.route_prepare_keys(k1, k2) if k1.is_cuda else None
-            # the projection weights' prepared form (bf16: digit planes), reused by every call
-            # until a parameter changes
-            self._wq_prepared = hip.query_proj_prepare(wq) if wq.is_cuda else None
+            with _packing():
+                wq = torch.stack([m.weight.detach() for m in self.query_projs]).to(device=device, dtype=dtype).contiguous()
+                bq = torch.stack([m.bias.detach() for m in self.query_projs]).to(device=device, dtype=dtype).contiguous()
+                k1 = self.sub_keys_1.weight.detach().to(device=device, dtype=dtype).contiguous()
+                k2 = self.sub_keys_2.weight.detach().to(device=device, dtype=dtype).contiguous()
+                self._key_norms = hip.key_norm_bounds(k1, k2)
+                # the sub-keys in the scoring MFMAs' fragment order
+                self._keys_prepared = hip.route_prepare_keys(k1, k2) if k1.is_cuda else None
+                # the projection weights' prepared form (bf16: digit planes), reused by every call
+                # until a parameter changes
+                self._wq_prepared = hip.query_proj_prepare(wq) if wq.is_cuda else None
             self._cache = (wq, bq, k1, k2)
             self._cache_key = key
         return self._cache
@@ -312,17 +323,18 @@ class ProductKeyRouter(nn.Module):
         ts = self._bn_sources()
         key = (device, tuple((t.data_ptr(), t._version) for t in ts if t is not None))
         if key != self._bn_key:
-            norms, H = list(self.query_norms), self.num_heads
-            one = ts[0].dtype if ts[0] is not None else None
-            if (device.type == "cuda" and H <= hip.MAX_BN_HEADS and len({m.eps for m in norms}) == 1
-                    and all(m.affine and m.track_running_stats for m in norms) and one in (torch.float32, torch.bfloat16)
-                    and all(t is not None and t.dtype == one and t.device == device and t.is_contiguous() for t in ts)):
-                # on the device: the host evaluation below waits for four tensors of every head
-                self._bn = hip.bn_coefficients(*([m.detach() for m in ts[i::4]] for i in range(4)), norms[0].eps, self.d_query,
-                                               one, device)
-            else:
-                ab = [_bn_eval_coefficients(m, self.d_query) for m in norms]
-                self._bn = tuple(torch.from_numpy(np.stack(c)).contiguous().to(device) for c in zip(*ab))
+            with _packing():
+                norms, H = list(self.query_norms), self.num_heads
+                one = ts[0].dtype if ts[0] is not None else None
+                if (device.type == "cuda" and H <= hip.MAX_BN_HEADS and len({m.eps for m in norms}) == 1
+                        and all(m.affine and m.track_running_stats for m in norms) and one in (torch.float32, torch.bfloat16)
+                        and all(t is not None and t.dtype == one and t.device == device and t.is_contiguous() for t in ts)):
+                    # on the device: the host evaluation below waits for four tensors of every head
+                    self._bn = hip.bn_coefficients(*([m.detach() for m in ts[i::4]] for i in range(4)), norms[0].eps, self.d_query,
+                                                   one, device)
+                else:
+                    ab = [_bn_eval_coefficients(m, self.d_query) for m in norms]
+                    self._bn = tuple(torch.from_numpy(np.stack(c)).contiguous().to(device) for c in zip(*ab))
             self._bn_key = key
         return self._bn
 
@@ -360,8 +372,9 @@ class ProductKeyRouter(nn.Module):
             packed = self._packed_weights(x_flat.dtype, x_flat.device)
         wq, bq = packed[:2]
         if self._identity is None or self._identity[0].device != x_flat.device:
-            ones = torch.ones((self.num_heads, self.d_query), dtype=torch.float32, device=x_flat.device)
-            self._identity = (ones, torch.zeros_like(ones))
+            with _packing():
+                ones = torch.ones((self.num_heads, self.d_query), dtype=torch.float32, device=x_flat.device)
+                self._identity = (ones, torch.zeros_like(ones))
         q_lin = hip.query_proj(x_flat, wq, bq, *self._identity, prepared=self._wq_prepared)
         if self._bn_one_call(x_flat):
             m0 = self.query_norms[0]
@@ -513,11 +526,12 @@ class EthosExpertLayer(nn.Module):
         mode = self._modules["router"]._pack_mode() if mode is None else mode
         key = (dtype, device, mode, tuple((p.data_ptr(), p._version) for p in ps))
         if key != self._gen_key:
-            if all(p.dtype == dtype and p.device == device and p.is_contiguous() for p in ps):
-                gen = tuple(p.detach() for p in ps)
-            else:
-                gen = tuple(p.detach().to(device=device, dtype=dtype).contiguous() for p in ps)
-            wut = gen[2][: self.d_model].t().contiguous() if dtype == torch.bfloat16 else None
+            with _packing():
+                if all(p.dtype == dtype and p.device == device and p.is_contiguous() for p in ps):
+                    gen = tuple(p.detach() for p in ps)
+                else:
+                    gen = tuple(p.detach().to(device=device, dtype=dtype).contiguous() for p in ps)
+                wut = gen[2][: self.d_model].t().contiguous() if dtype == torch.bfloat16 else None
             self._gen = gen + (wut,)
             self._gen_key = key
         return self._gen

@@ -365,6 +365,31 @@ def test_bn_coefficients_match_host(dt):
         assert np.array_equal(a.cpu().numpy(), b)
 
 
+@pytest.mark.parametrize("name", ["tiny_fp32", "tiny"])
+def test_backward_after_inference_mode(name):
+    """What a call under torch.inference_mode packs serves a later call with gradients, in eval
+    and in training mode, and with the model in another dtype than its input."""
+    sh = SHAPES[name]
+    x, sd = make_inputs(sh, signal=True)
+    xd = x.cuda().view(sh.batch, -1, sh.d_model)
+    other = torch.float32 if sh.torch_dtype == torch.bfloat16 else torch.bfloat16
+    for train, dt in ((False, sh.torch_dtype), (True, sh.torch_dtype), (False, other)):
+        grads = []
+        for first in (False, True):
+            m = ethos_amd.EthosExpertLayer(sh.config()).to(sh.torch_dtype)
+            m.load_state_dict(sd)
+            m = m.cuda().train(train)
+            if first:
+                with torch.inference_mode():
+                    m.eval()(xd.to(dt))
+                    m.train(train)
+            y = m(xd.to(dt))
+            y.float().square().sum().backward()
+            grads.append([p.grad for p in m.parameters()])
+        for a, b in zip(*grads):
+            assert torch.equal(a, b)
+
+
 @pytest.mark.parametrize("train", [False, True])
 def test_router_second_derivative(train):
     """The scores' gradient can be differentiated again: create_graph gives the derivative of
