@@ -65,6 +65,41 @@ def _packing():
         yield
 
 
+class _Made:
+    """The key of tensors that are made once and read by later calls on any stream: another stream's
+    first call waits for their making and holds their memory from then on.  What a graph capture
+    makes exists only after a replay, so it serves no call outside (`once`: the key is that of a
+    single pass, which may go on using it).  A copied or unpickled module makes its own."""
+
+    def __init__(self, key=None, tensors=(), once: bool = False):
+        self.key, self.event = key, None
+        self.tensors = [t for t in tensors if t is not None and t.is_cuda]
+        if not self.tensors:
+            return
+        if torch.cuda.is_current_stream_capturing():
+            self.key = key if once else None
+        else:
+            self.event, self.streams = torch.cuda.Event(), {hip._stream()}
+            self.event.record()
+
+    def fits(self, key) -> bool:
+        if key != self.key:
+            return False
+        if self.event is not None:
+            s = hip._stream()
+            # (a capture starts after the work before it: torch.cuda.graph waits for the device)
+            if s not in self.streams and not torch.cuda.is_current_stream_capturing():
+                stream = torch.cuda.current_stream()
+                stream.wait_event(self.event)
+                for t in self.tensors:
+                    t.record_stream(stream)
+                self.streams.add(s)
+        return True
+
+    def __reduce__(self):
+        return _Made, ()
+
+
 def _gelu_grad(x: torch.Tensor) -> torch.Tensor:
     """Derivative of the erf GELU x·Φ(x): Φ(x) + x·φ(x)."""
     cdf = 0.5 * (1.0 + torch.erf(x * (1.0 / math.sqrt(2.0))))
@@ -259,11 +294,12 @@ class ProductKeyRouter(nn.Module):
         self.query_norms = nn.ModuleList([nn.BatchNorm1d(self.d_query) for _ in range(self.num_heads)])
         self.sub_keys_1 = nn.Embedding(self.num_sub_keys, self.d_query // 2)
         self.sub_keys_2 = nn.Embedding(self.num_sub_keys, self.d_query // 2)
-        self._cache_key = None
+        self._cache_made = _Made()
         self._cache = None
         self._train_pass = 0
-        self._bn_key = None
+        self._bn_made = _Made()
         self._bn = None
+        self._identity_made = _Made()
         self._identity = None
         self._key_norms = None
         self._keys_prepared = None
@@ -300,9 +336,9 @@ class ProductKeyRouter(nn.Module):
         return self._train_pass if any(m.training for m in self._modules["query_norms"]._modules.values()) else 0
 
     def _packed_weights(self, dtype: torch.dtype, device: torch.device, mode: int | None = None):
-        key = (dtype, device, self._pack_mode() if mode is None else mode,
-               tuple((t.data_ptr(), t._version) for t in self._weight_sources() if t is not None))
-        if key != self._cache_key:
+        mode = self._pack_mode() if mode is None else mode
+        key = (dtype, device, mode, tuple((t.data_ptr(), t._version) for t in self._weight_sources() if t is not None))
+        if not self._cache_made.fits(key):
             with _packing():
                 wq = torch.stack([m.weight.detach() for m in self.query_projs]).to(device=device, dtype=dtype).contiguous()
                 bq = torch.stack([m.bias.detach() for m in self.query_projs]).to(device=device, dtype=dtype).contiguous()
@@ -315,14 +351,14 @@ class ProductKeyRouter(nn.Module):
                 # until a parameter changes
                 self._wq_prepared = hip.query_proj_prepare(wq) if wq.is_cuda else None
             self._cache = (wq, bq, k1, k2)
-            self._cache_key = key
+            self._cache_made = _Made(key, (*self._cache, self._key_norms, self._keys_prepared, self._wq_prepared), mode > 0)
         return self._cache
 
     def _bn_coefficients(self, device: torch.device):
         """(alpha, beta) of the eval-mode BatchNorms, float32 [H, d_query] on the device."""
         ts = self._bn_sources()
         key = (device, tuple((t.data_ptr(), t._version) for t in ts if t is not None))
-        if key != self._bn_key:
+        if not self._bn_made.fits(key):
             with _packing():
                 norms, H = list(self.query_norms), self.num_heads
                 one = ts[0].dtype if ts[0] is not None else None
@@ -335,7 +371,7 @@ class ProductKeyRouter(nn.Module):
                 else:
                     ab = [_bn_eval_coefficients(m, self.d_query) for m in norms]
                     self._bn = tuple(torch.from_numpy(np.stack(c)).contiguous().to(device) for c in zip(*ab))
-            self._bn_key = key
+            self._bn_made = _Made(key, self._bn)
         return self._bn
 
     def _packed(self, dtype: torch.dtype, device: torch.device):
@@ -371,10 +407,11 @@ class ProductKeyRouter(nn.Module):
             self._train_pass += 1
             packed = self._packed_weights(x_flat.dtype, x_flat.device)
         wq, bq = packed[:2]
-        if self._identity is None or self._identity[0].device != x_flat.device:
+        if not self._identity_made.fits(x_flat.device):
             with _packing():
                 ones = torch.ones((self.num_heads, self.d_query), dtype=torch.float32, device=x_flat.device)
                 self._identity = (ones, torch.zeros_like(ones))
+            self._identity_made = _Made(x_flat.device, self._identity)
         q_lin = hip.query_proj(x_flat, wq, bq, *self._identity, prepared=self._wq_prepared)
         if self._bn_one_call(x_flat):
             m0 = self.query_norms[0]
@@ -401,7 +438,7 @@ class ProductKeyRouter(nn.Module):
                                      m0.momentum if m0.momentum is not None else 0.1, m0.eps, batch=batch)
             if track:
                 torch._foreach_add_([m.num_batches_tracked for m in self.query_norms], 1)
-                self._bn_key = None  # the running statistics' version counters do not move
+                self._bn_made = _Made()  # the running statistics' version counters do not move
             return out
         outs = []
         for h, m in enumerate(self.query_norms):
@@ -414,7 +451,7 @@ class ProductKeyRouter(nn.Module):
         # batch_norm updated the running statistics in place without bumping their version
         # counters, so the cached eval-mode coefficients are stale
         if any(m.training and m.track_running_stats for m in self.query_norms):
-            self._bn_key = None
+            self._bn_made = _Made()
         return torch.stack(outs, dim=1).contiguous()
 
     def route(self, x_flat: torch.Tensor, mark=None):
@@ -501,7 +538,7 @@ class EthosExpertLayer(nn.Module):
         self.generation_network = ExpertGenerationNetwork(config.d_latent, config.d_model,
                                                           config.d_intermediate_hypernet)
         self.router = ProductKeyRouter(config)
-        self._gen_key = None
+        self._gen_made = _Made()
         self._gen = None
 
     def _param_sources(self) -> list:
@@ -525,7 +562,7 @@ class EthosExpertLayer(nn.Module):
         ps = (self.expert_latents.weight, self.generation_network.net[0].weight, self.generation_network.net[2].weight)
         mode = self._modules["router"]._pack_mode() if mode is None else mode
         key = (dtype, device, mode, tuple((p.data_ptr(), p._version) for p in ps))
-        if key != self._gen_key:
+        if not self._gen_made.fits(key):
             with _packing():
                 if all(p.dtype == dtype and p.device == device and p.is_contiguous() for p in ps):
                     gen = tuple(p.detach() for p in ps)
@@ -533,7 +570,7 @@ class EthosExpertLayer(nn.Module):
                     gen = tuple(p.detach().to(device=device, dtype=dtype).contiguous() for p in ps)
                 wut = gen[2][: self.d_model].t().contiguous() if dtype == torch.bfloat16 else None
             self._gen = gen + (wut,)
-            self._gen_key = key
+            self._gen_made = _Made(key, (t for t in self._gen if all(t is None or t.data_ptr() != p.data_ptr() for p in ps)), mode > 0)
         return self._gen
 
     def _expert_stages(self, x_flat: torch.Tensor, gates: torch.Tensor, seg: dict, xp: torch.Tensor | None = None):

@@ -295,3 +295,63 @@ def test_one_call_forward_matches_stages(name, n, hidden):
         a = m.forward_flat(xd)
         b = m.forward_flat(xd, mark=seen.append)
     assert seen and torch.equal(a, b)
+
+
+def _two_layers(name):
+    sh = SHAPES[name]
+    x, sd = make_inputs(sh, signal=True)
+    ms = []
+    for _ in range(2):
+        m = ethos_amd.EthosExpertLayer(sh.config()).to(sh.torch_dtype)
+        m.load_state_dict(sd)
+        ms.append(m.cuda().eval())
+    return x.cuda(), ms
+
+
+@pytest.mark.parametrize("name", ["cfg3", "tiny_fp32"])
+def test_packed_parameters_made_on_another_stream(name):
+    """A stream's first call after another stream's packed the parameters (behind 50 ms of other
+    work) waits for them, in eval mode and, for the BatchNorm coefficients alone, after a training
+    pass; the packed tensors outlive a repacking while that stream still reads them."""
+    x, (m, ref) = _two_layers(name)
+    a, b = torch.cuda.Stream(), torch.cuda.Stream()
+    with torch.no_grad():
+        want = ref.forward_flat(x)
+        for train in (False, True):
+            if train:
+                for v in (m, ref):
+                    v.train().forward_flat(x)
+                    v.eval()
+                want = ref.forward_flat(x)
+            torch.cuda.synchronize()
+            with torch.cuda.stream(a):
+                torch.cuda._sleep(100_000_000)
+                m.forward_flat(x)
+            with torch.cuda.stream(b):
+                got = m.forward_flat(x)
+                torch.cuda._sleep(100_000_000)
+                again = m.forward_flat(x)
+            with torch.cuda.stream(a):  # packs again, in memory that must not be b's
+                m.forward_flat(x.to(torch.float32 if x.dtype == torch.bfloat16 else torch.bfloat16))
+            torch.cuda.synchronize()
+            assert torch.equal(got, want) and torch.equal(again, want)
+
+
+def test_packing_inside_a_capture_serves_only_the_graph():
+    """A graph captured from a layer that has not run yet packs the parameters in every replay;
+    eager calls before the first replay pack their own.  Copies of a used layer pack their own."""
+    import copy
+    x, (m, ref) = _two_layers("cfg3")
+    with torch.no_grad():
+        want = ref.forward_flat(x)
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            out = m.forward_flat(x)
+        assert torch.equal(m.forward_flat(x), want)
+        for _ in range(3):
+            out.zero_()
+            graph.replay()
+            assert torch.equal(out, want)
+            assert torch.equal(m.forward_flat(x), want)
+        assert torch.equal(copy.deepcopy(m)(x[None])[0], want)
