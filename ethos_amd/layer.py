@@ -384,16 +384,20 @@ class ProductKeyRouter(nn.Module):
     def _bn_one_call(self, x_flat: torch.Tensor) -> bool:
         """Whether the heads' training-mode BatchNorms run as one library call: all of them on
         batch statistics with one eps and momentum, affine, in the layer's dtype on its device,
-        without gradients of their own and over at least two tokens (torch refuses fewer)."""
+        without gradients of their own, over at least two tokens (torch refuses fewer), and with
+        running statistics of their own (heads that share them update them one after the other)."""
         norms = list(self.query_norms)
         m0 = norms[0]
-        ts = [t for t in self._bn_sources() if t is not None]
+        ts = self._bn_sources()
+        updated = sorted(t.data_ptr() for t in ts[2::4] + ts[3::4] if t is not None)
+        ts = [t for t in ts if t is not None]
         return (x_flat.shape[0] > 1 and self.num_heads <= hip.MAX_BN_HEADS and not torch.is_grad_enabled()
                 and self.d_query % 4 == 0
                 and all(m.affine and m.training and m.eps == m0.eps and m.momentum == m0.momentum
                         and m.track_running_stats == m0.track_running_stats
                         and (m.running_mean is not None) == m0.track_running_stats for m in norms)
-                and all(t.dtype == x_flat.dtype and t.device == x_flat.device and t.is_contiguous() for t in ts))
+                and all(t.dtype == x_flat.dtype and t.device == x_flat.device and t.is_contiguous() for t in ts)
+                and all(q - p >= self.d_query * x_flat.element_size() for p, q in zip(updated, updated[1:])))
 
     def queries(self, x_flat: torch.Tensor, packed=None) -> torch.Tensor:
         """Per-head queries after BatchNorm, [n, H, d_query] (model.py:215-216).  `packed`:

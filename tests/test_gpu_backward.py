@@ -499,3 +499,26 @@ def test_training_sees_weights_written_without_a_version_step(name):
         p.data.mul_(0.75)
     with torch.no_grad():
         assert torch.equal(m.eval()(xd), new(m.state_dict(), False)(xd))
+
+
+def test_training_queries_of_heads_that_share_a_norm():
+    """Two heads with one BatchNorm module: normalised by their own batches, and the running
+    statistics updated twice, in the heads' order, as by batch_norm a head at a time."""
+    from ethos_amd import hip
+    sh = SHAPES["tiny_fp32"]
+    x, sd = make_inputs(sh, signal=True)
+    m = ethos_amd.EthosExpertLayer(sh.config())
+    m.load_state_dict(sd)
+    r, x = m.cuda().train().router, x.cuda()
+    r.query_norms[1] = r.query_norms[0]
+    norms = list(r.query_norms)
+    mean, var = norms[0].running_mean.clone(), norms[0].running_var.clone()
+    with torch.no_grad():
+        q = r.queries(x)
+        v = hip.query_proj(x, *r._packed_weights(x.dtype, x.device)[:2], *r._identity)
+        for h in range(2):
+            ref = torch.nn.functional.batch_norm(v[:, h], mean, var, norms[0].weight, norms[0].bias, True, 0.1, norms[0].eps)
+            assert torch.equal(q[:, h], ref)
+    assert torch.equal(norms[0].running_mean, mean) and torch.equal(norms[0].running_var, var)
+    assert int(norms[0].num_batches_tracked) == int(sd["router.query_norms.0.num_batches_tracked"] if
+                                                    "router.query_norms.0.num_batches_tracked" in sd else 0) + 2

@@ -71,3 +71,22 @@ def test_loop_faithful_baseline_reproduces_reference(name):
         y = loop_faithful.layer(x, sd, sh.num_heads, sh.top_k)
     assert np.array_equal(ids.numpy().astype(np.int32), f["ref_indices"])
     assert np.array_equal(O.from_torch(y), f["ref_out"])
+
+
+def test_shared_running_statistics_are_not_updated_in_one_call():
+    """The one-call training BatchNorm updates every head's running statistics at once: heads whose
+    statistics are one tensor, or overlap, take the calls one after the other."""
+    m = ethos_amd.EthosExpertLayer(SHAPES["tiny_fp32"].config()).train().router
+    x = torch.randn(6, m.d_model)
+    with torch.no_grad():
+        assert m._bn_one_call(x)
+        own = m.query_norms[1]
+        m.query_norms[1] = m.query_norms[0]
+        assert not m._bn_one_call(x)
+        m.query_norms[1] = own
+        both = torch.zeros(m.d_query + 4)
+        m.query_norms[0].running_mean, own.running_var = both[:-4], both[4:]
+        assert not m._bn_one_call(x)
+        both = torch.zeros(2 * m.d_query)
+        m.query_norms[0].running_mean, own.running_var = both[:m.d_query], both[m.d_query:]
+        assert m._bn_one_call(x)
