@@ -160,6 +160,14 @@ __device__ __forceinline__ int row_bcast(int v) {
     return __builtin_amdgcn_update_dpp(0, v, 0x150 + I, 0xf, 0xf, false);
 }
 
+// Four floats at any float's address (one 16-byte access; callers' xp, dyb and dh need no more
+// than their own alignment).
+typedef float f32x4_any_t __attribute__((ext_vector_type(4), aligned(4)));
+__device__ __forceinline__ float4 load_any4(const float* p) {
+    const f32x4_any_t v = *reinterpret_cast<const f32x4_any_t*>(p);
+    return make_float4(v.x, v.y, v.z, v.w);
+}
+
 struct SumPos {  // a lane's position
     int t, s, to;   // token, slot, and after this position: 0 go on, 1 store to dh, 2 to head, 3 to tail
     float a, dc;
@@ -180,8 +188,8 @@ struct SumStep {
                                                 float4* y) {
         if constexpr (U < kSumUnroll) {
             const int64_t at = (int64_t)row_bcast<I + U>(me.t) * dh + col;
-            y[U] = *reinterpret_cast<const float4*>(dyb + at);
-            x[U] = *reinterpret_cast<const float4*>(xp + at);
+            y[U] = load_any4(dyb + at);
+            x[U] = load_any4(xp + at);
             load<U + 1>(me, xp, dyb, dh, col, x, y);
         }
     }
@@ -198,7 +206,7 @@ struct SumStep {
             acc.w = __builtin_fmaf(dc, x[U].w, __builtin_fmaf(a, y[U].w, acc.w));
             if (to != 0) {
                 float* dst = (to == 1 ? dhs + (int64_t)s * dh : to == 2 ? head : tail) + col;
-                if (in) *reinterpret_cast<float4*>(dst) = acc;
+                if (in) *reinterpret_cast<f32x4_any_t*>(dst) = f32x4_any_t{acc.x, acc.y, acc.z, acc.w};
                 acc = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
             }
             add<U + 1>(me, dh, col, in, acc, x, y, dhs, head, tail);

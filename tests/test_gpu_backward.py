@@ -193,6 +193,31 @@ def test_expert_backward_entry_point(dt, n, H, k, dh, E, hot):
         assert _nerr(got, ref) < 1e-5, (name, _nerr(got, ref))
 
 
+@pytest.mark.parametrize("dh,skip", [(96, 1), (512, 2), (40, 3)])
+def test_expert_backward_takes_rows_at_any_float(dh, skip):
+    """xp, dyb, the token sums and dh at addresses that are aligned to a float only: the bits of
+    the aligned call."""
+    from ethos_amd import hip
+    from ethos_amd._lib import load
+    g = torch.Generator().manual_seed(dh)
+    n, H, k, E = 150, 2, 8, 300
+    seg = hip.sort_segment(torch.randint(0, E, (n * H * k,), generator=g, dtype=torch.int32).cuda(), E)
+    U, at = int(seg["n_unique"].item()), lambda rows: torch.zeros(rows * dh + 4, device="cuda")[skip:skip + rows * dh].view(rows, dh)
+    h, gates = torch.randn(U, dh, generator=g).cuda(), torch.rand(n, H, k, generator=g).cuda()
+    xp, dyb = (torch.randn(n, dh, generator=g).cuda() for _ in range(2))
+    want = hip.expert_backward(h, xp, dyb, seg, gates, H, k, U)
+    px, py = at(n).copy_(xp), at(n).copy_(dyb)
+    assert px.data_ptr() % 16 and py.data_ptr() % 16
+    dg, got = torch.empty_like(gates), [at(n), at(n), at(U)]
+    ws, size = hip.workspace(load().ethos_expert_backward_workspace_bytes(n, H, k, dh), h.device)
+    rc = load().ethos_expert_backward(h.data_ptr(), px.data_ptr(), py.data_ptr(), seg["pair_slot"].data_ptr(), seg["perm"].data_ptr(),
+                                      seg["sorted_slot"].data_ptr(), seg["seg_off"].data_ptr(), gates.data_ptr(), n, H, k, dh, 0,
+                                      ws.data_ptr(), size, dg.data_ptr(), *[t.data_ptr() for t in got], hip._stream())
+    assert rc == 0
+    for a, b in zip([dg] + got, want):
+        assert torch.equal(a.view(b.shape), b)
+
+
 @pytest.mark.parametrize("dt,n,H,k,dl,dh,d,E", [
     ("bf16", 1, 1, 1, 8, 8, 8, 1), ("bf16", 33, 2, 4, 16, 40, 72, 37), ("bf16", 129, 3, 4, 136, 264, 200, 700),
     ("bf16", 700, 4, 8, 128, 512, 256, 9000), ("bf16", 65, 8, 16, 128, 256, 1024, 1),
