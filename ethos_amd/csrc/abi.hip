@@ -119,11 +119,10 @@ size_t ethos_query_proj_workspace_bytes(int64_t n_tok, int32_t d_model, int32_t 
     return b < 256 ? 256 : b;
 }
 
-static int query_proj_impl(const char* name, const void* x, const void* wq, const void* prepared, const void* bq,
-                           const float* bn_alpha, const float* bn_beta, int64_t n_tok, int32_t d_model,
-                           int32_t n_heads, int32_t d_query, int32_t dtype, void* workspace, size_t workspace_bytes,
-                           void* q_out, void* stream) {
-    g_err[0] = 0;
+static int query_proj_checks(const char* name, const void* x, const void* wq, const void* prepared, const void* bq,
+                             const float* bn_alpha, const float* bn_beta, int64_t n_tok, int32_t d_model,
+                             int32_t n_heads, int32_t d_query, int32_t dtype, const void* workspace,
+                             size_t workspace_bytes, const void* q_out) {
     if (!dtype_ok(dtype)) return fail(ETHOS_EDTYPE, "%s: unknown dtype %d", name, dtype);
     if (n_tok < 0 || d_model <= 0 || n_heads <= 0 || d_query <= 0)
         return fail(ETHOS_ESIZE, "%s: bad sizes n_tok=%lld d_model=%d n_heads=%d d_query=%d", name,
@@ -140,6 +139,18 @@ static int query_proj_impl(const char* name, const void* x, const void* wq, cons
             (d_model % 8))
             return fail(ETHOS_EALIGN, "%s: x, wq, prepared, workspace 16-byte aligned and d_model %% 8 == 0", name);
     }
+    return 0;
+}
+
+static int query_proj_impl(const char* name, const void* x, const void* wq, const void* prepared, const void* bq,
+                           const float* bn_alpha, const float* bn_beta, int64_t n_tok, int32_t d_model,
+                           int32_t n_heads, int32_t d_query, int32_t dtype, void* workspace, size_t workspace_bytes,
+                           void* q_out, void* stream) {
+    g_err[0] = 0;
+    if (const int rc = query_proj_checks(name, x, wq, prepared, bq, bn_alpha, bn_beta, n_tok, d_model, n_heads, d_query, dtype,
+                                         workspace, workspace_bytes, q_out))
+        return rc;
+    if (n_tok == 0) return 0;
     if (ethos::qproj_weights_bytes(n_heads * d_query, d_model, dtype) == 0) prepared = nullptr;
     return hip_status(ethos::launch_qproj(x, wq, prepared, bq, bn_alpha, bn_beta, n_tok, d_model, n_heads * d_query,
                                           dtype, workspace, q_out, num_cus(), (hipStream_t)stream),
@@ -177,18 +188,25 @@ int ethos_query_proj_prepare(const void* wq, int32_t d_model, int32_t n_heads, i
                       "ethos_query_proj_prepare");
 }
 
+static int query_prepared_checks(const char* name, const void* prepared, size_t prepared_bytes, int64_t n_tok, int32_t d_model,
+                                 int32_t n_heads, int32_t d_query, int32_t dtype) {
+    const size_t need = ethos_query_proj_weights_bytes(d_model, n_heads, d_query, dtype);
+    if (need > 0 && n_tok > 0) {
+        if (!prepared) return fail(ETHOS_ENULL, "%s: null prepared weights", name);
+        if (prepared_bytes < need)
+            return fail(ETHOS_EWORKSPACE, "%s: prepared weights of %zu bytes, %zu needed", name, prepared_bytes, need);
+    }
+    return 0;
+}
+
 int ethos_query_proj_prepared(const void* x, const void* wq, const void* prepared, size_t prepared_bytes,
                               const void* bq, const float* bn_alpha, const float* bn_beta, int64_t n_tok,
                               int32_t d_model, int32_t n_heads, int32_t d_query, int32_t dtype, void* workspace,
                               size_t workspace_bytes, void* q_out, void* stream) {
-    const size_t need = ethos_query_proj_weights_bytes(d_model, n_heads, d_query, dtype);
-    if (need > 0 && n_tok > 0) {
-        g_err[0] = 0;
-        if (!prepared) return fail(ETHOS_ENULL, "ethos_query_proj_prepared: null prepared weights");
-        if (prepared_bytes < need)
-            return fail(ETHOS_EWORKSPACE, "ethos_query_proj_prepared: prepared weights of %zu bytes, %zu needed",
-                        prepared_bytes, need);
-    }
+    g_err[0] = 0;
+    if (const int rc = query_prepared_checks("ethos_query_proj_prepared", prepared, prepared_bytes, n_tok, d_model, n_heads,
+                                             d_query, dtype))
+        return rc;
     return query_proj_impl("ethos_query_proj_prepared", x, wq, prepared, bq, bn_alpha, bn_beta, n_tok, d_model,
                            n_heads, d_query, dtype, workspace, workspace_bytes, q_out, stream);
 }
@@ -212,16 +230,30 @@ static int route_checks(const char* name, int64_t n_rows, int32_t d_query, int32
     return 0;
 }
 
+static int route_pointer_checks(const char* name, const void* q, const void* sub_keys_1, const void* sub_keys_2,
+                                const void* out_scores, const void* out_ids) {
+    if (!q || !sub_keys_1 || !sub_keys_2 || !out_scores || !out_ids) return fail(ETHOS_ENULL, "%s: null pointer", name);
+    if (!aligned16(q) || !aligned16(sub_keys_1) || !aligned16(sub_keys_2))
+        return fail(ETHOS_EALIGN, "%s: q and sub-key tables must be 16-byte aligned", name);
+    return 0;
+}
+
+static int route_prepared_checks(const char* name, const void* prepared, size_t prepared_bytes, int32_t d_query,
+                                 int32_t n_sub_keys, int32_t dtype) {
+    if (!prepared) return fail(ETHOS_ENULL, "%s: null pointer", name);
+    const size_t need = ethos::route_keys_bytes(n_sub_keys, d_query / 2, dtype);
+    if (prepared_bytes < need) return fail(ETHOS_ESIZE, "%s: prepared holds %zu bytes, needs %zu", name, prepared_bytes, need);
+    if (!aligned16(prepared)) return fail(ETHOS_EALIGN, "%s: prepared must be 16-byte aligned", name);
+    return 0;
+}
+
 int ethos_route_topk(const void* q, const void* sub_keys_1, const void* sub_keys_2, const float* key_norms,
                      int64_t n_rows, int32_t d_query, int32_t n_sub_keys, int32_t top_k, int32_t k_cand, int32_t dtype,
                      void* out_scores, int32_t* out_ids, void* stream) {
     g_err[0] = 0;
     if (const int rc = route_checks("ethos_route_topk", n_rows, d_query, n_sub_keys, top_k, k_cand, dtype)) return rc;
     if (n_rows == 0) return 0;
-    if (!q || !sub_keys_1 || !sub_keys_2 || !out_scores || !out_ids)
-        return fail(ETHOS_ENULL, "ethos_route_topk: null pointer");
-    if (!aligned16(q) || !aligned16(sub_keys_1) || !aligned16(sub_keys_2))
-        return fail(ETHOS_EALIGN, "ethos_route_topk: q and sub-key tables must be 16-byte aligned");
+    if (const int rc = route_pointer_checks("ethos_route_topk", q, sub_keys_1, sub_keys_2, out_scores, out_ids)) return rc;
     return hip_status(ethos::launch_route(q, sub_keys_1, sub_keys_2, key_norms, nullptr, n_rows, d_query, n_sub_keys,
                                           top_k, k_cand, dtype, out_scores, out_ids, (hipStream_t)stream),
                       "ethos_route_topk");
@@ -259,13 +291,9 @@ int ethos_route_topk_prepared(const void* q, const void* sub_keys_1, const void*
     if (const int rc = route_checks("ethos_route_topk_prepared", n_rows, d_query, n_sub_keys, top_k, k_cand, dtype))
         return rc;
     if (n_rows == 0) return 0;
-    if (!q || !sub_keys_1 || !sub_keys_2 || !prepared || !out_scores || !out_ids)
-        return fail(ETHOS_ENULL, "ethos_route_topk_prepared: null pointer");
-    if (prepared_bytes < ethos::route_keys_bytes(n_sub_keys, d_query / 2, dtype))
-        return fail(ETHOS_ESIZE, "ethos_route_topk_prepared: prepared holds %zu bytes, needs %zu", prepared_bytes,
-                    ethos::route_keys_bytes(n_sub_keys, d_query / 2, dtype));
-    if (!aligned16(q) || !aligned16(sub_keys_1) || !aligned16(sub_keys_2) || !aligned16(prepared))
-        return fail(ETHOS_EALIGN, "ethos_route_topk_prepared: q, sub-key tables and prepared must be 16-byte aligned");
+    if (const int rc = route_prepared_checks("ethos_route_topk_prepared", prepared, prepared_bytes, d_query, n_sub_keys, dtype))
+        return rc;
+    if (const int rc = route_pointer_checks("ethos_route_topk_prepared", q, sub_keys_1, sub_keys_2, out_scores, out_ids)) return rc;
     return hip_status(ethos::launch_route(q, sub_keys_1, sub_keys_2, key_norms, prepared, n_rows, d_query, n_sub_keys,
                                           top_k, k_cand, dtype, out_scores, out_ids, (hipStream_t)stream),
                       "ethos_route_topk_prepared");
@@ -484,6 +512,44 @@ int ethos_token_proj(const void* x, const void* w2, const void* wut, int64_t n_t
     return hip_status(rc, "ethos_token_proj");
 }
 
+static int expert_forward_checks(const char* name, const void* x, const void* latents, int64_t n_experts, const void* w1, const void* w2,
+                                 const void* wut, const void* xp, const int32_t* uniq_ids, const int32_t* seg_off,
+                                 const int32_t* n_unique, int64_t max_unique,
+                                 const int32_t* perm, const int32_t* sorted_slot, const int32_t* pair_slot, const void* scores,
+                                 int64_t n_tok, int32_t n_heads, int32_t top_k, int32_t d_latent, int32_t d_hidden,
+                                 int32_t d_model, int32_t dtype, int32_t order, const void* workspace, size_t workspace_bytes,
+                                 const void* h_out, const void* out) {
+    if (!dtype_ok(dtype)) return fail(ETHOS_EDTYPE, "%s: unknown dtype %d", name, dtype);
+    if (order != 0 && order != 1) return fail(ETHOS_ESIZE, "%s: order must be 0 or 1, got %d", name, order);
+    if (n_tok < 0 || n_heads <= 0 || top_k <= 0 || n_experts <= 0 || max_unique < 0 || d_latent <= 0 ||
+        d_hidden <= 0 || d_model <= 0)
+        return fail(ETHOS_ESIZE, "%s: bad sizes", name);
+    if (n_tok * n_heads * top_k > INT32_MAX || n_tok > INT32_MAX)
+        return fail(ETHOS_ESIZE, "%s: too many pairs", name);
+    const int kq = dtype == ETHOS_BF16 ? 16 : 2;
+    const int vec = dtype == ETHOS_BF16 ? 8 : 4;
+    if (d_latent % kq || d_hidden % 32 || d_model % 32 || d_model > 4096 ||
+        ethos::apply_chunks(d_model, dtype) > 8 || ethos::apply_chunks(d_hidden, dtype) > 8 ||
+        ethos::generate_smem_bytes(d_latent, d_hidden, dtype) > 160 * 1024 || d_model % vec || d_hidden % vec)
+        return fail(ETHOS_EUNSUPPORTED,
+                    "%s: needs d_latent %% %d == 0, d_hidden and d_model multiples of 32 with "
+                    "d_model <= 4096 and d_hidden <= %d (got %d, %d, %d)", name, kq, 8 * 64 * vec, d_latent, d_hidden,
+                    d_model);
+    if (n_tok == 0) return 0;
+    if (max_unique < 1) return fail(ETHOS_ESIZE, "%s: max_unique must be >= 1 for a nonempty batch", name);
+    if (!x || !latents || !w1 || !w2 || !uniq_ids || !seg_off || !n_unique || !perm || !sorted_slot || !pair_slot ||
+        !scores || !workspace || !h_out || !out)
+        return fail(ETHOS_ENULL, "%s: null pointer", name);
+    const size_t need = ethos::expert_forward_workspace_bytes(n_tok, n_heads, top_k, max_unique, d_model, d_hidden,
+                                                              dtype, order);
+    if (workspace_bytes < need)
+        return fail(ETHOS_EWORKSPACE, "%s: workspace of %zu bytes, %zu needed", name, workspace_bytes, need);
+    if (!aligned16(x) || !aligned16(w1) || !aligned16(w2) || (wut && !aligned16(wut)) || (xp && !aligned16(xp)) ||
+        !aligned16(workspace) || !aligned16(h_out) || !aligned16(out))
+        return fail(ETHOS_EALIGN, "%s: x, w1, w2, wut, xp, workspace, h_out and out must be 16-byte aligned", name);
+    return 0;
+}
+
 int ethos_expert_forward(const void* x, const void* latents, int64_t n_experts, const void* w1, const void* w2,
                          const void* wut, const void* xp, const int32_t* uniq_ids, const int32_t* seg_off,
                          const int32_t* n_unique, int64_t max_unique,
@@ -492,36 +558,11 @@ int ethos_expert_forward(const void* x, const void* latents, int64_t n_experts, 
                          int32_t d_model, int32_t dtype, int32_t order, void* workspace, size_t workspace_bytes,
                          void* h_out, void* out, void* stream) {
     g_err[0] = 0;
-    if (!dtype_ok(dtype)) return fail(ETHOS_EDTYPE, "ethos_expert_forward: unknown dtype %d", dtype);
-    if (order != 0 && order != 1) return fail(ETHOS_ESIZE, "ethos_expert_forward: order must be 0 or 1, got %d", order);
-    if (n_tok < 0 || n_heads <= 0 || top_k <= 0 || n_experts <= 0 || max_unique < 0 || d_latent <= 0 ||
-        d_hidden <= 0 || d_model <= 0)
-        return fail(ETHOS_ESIZE, "ethos_expert_forward: bad sizes");
-    if (n_tok * n_heads * top_k > INT32_MAX || n_tok > INT32_MAX)
-        return fail(ETHOS_ESIZE, "ethos_expert_forward: too many pairs");
-    const int kq = dtype == ETHOS_BF16 ? 16 : 2;
-    const int vec = dtype == ETHOS_BF16 ? 8 : 4;
-    if (d_latent % kq || d_hidden % 32 || d_model % 32 || d_model > 4096 ||
-        ethos::apply_chunks(d_model, dtype) > 8 || ethos::apply_chunks(d_hidden, dtype) > 8 ||
-        ethos::generate_smem_bytes(d_latent, d_hidden, dtype) > 160 * 1024 || d_model % vec || d_hidden % vec)
-        return fail(ETHOS_EUNSUPPORTED,
-                    "ethos_expert_forward: needs d_latent %% %d == 0, d_hidden and d_model multiples of 32 with "
-                    "d_model <= 4096 and d_hidden <= %d (got %d, %d, %d)", kq, 8 * 64 * vec, d_latent, d_hidden,
-                    d_model);
+    if (const int rc = expert_forward_checks("ethos_expert_forward", x, latents, n_experts, w1, w2, wut, xp, uniq_ids, seg_off, n_unique,
+                                             max_unique, perm, sorted_slot, pair_slot, scores, n_tok, n_heads, top_k, d_latent,
+                                             d_hidden, d_model, dtype, order, workspace, workspace_bytes, h_out, out))
+        return rc;
     if (n_tok == 0) return 0;
-    if (max_unique < 1) return fail(ETHOS_ESIZE, "ethos_expert_forward: max_unique must be >= 1 for a nonempty batch");
-    if (!x || !latents || !w1 || !w2 || !uniq_ids || !seg_off || !n_unique || !perm || !sorted_slot || !pair_slot ||
-        !scores || !workspace || !h_out || !out)
-        return fail(ETHOS_ENULL, "ethos_expert_forward: null pointer");
-    const size_t need = ethos::expert_forward_workspace_bytes(n_tok, n_heads, top_k, max_unique, d_model, d_hidden,
-                                                              dtype, order);
-    if (workspace_bytes < need)
-        return fail(ETHOS_EWORKSPACE, "ethos_expert_forward: workspace of %zu bytes, %zu needed", workspace_bytes,
-                    need);
-    if (!aligned16(x) || !aligned16(w1) || !aligned16(w2) || (wut && !aligned16(wut)) || (xp && !aligned16(xp)) ||
-        !aligned16(workspace) || !aligned16(h_out) || !aligned16(out))
-        return fail(ETHOS_EALIGN, "ethos_expert_forward: x, w1, w2, wut, xp, workspace, h_out and out must be "
-                                  "16-byte aligned");
     const int rc = ethos::launch_expert_forward(x, latents, n_experts, w1, w2, dtype == ETHOS_BF16 ? wut : nullptr,
                                                 xp, uniq_ids, seg_off, n_unique, max_unique, perm, sorted_slot,
                                                 pair_slot, scores,
@@ -839,18 +880,36 @@ int ethos_layer_forward(const void* x, const void* wq, const void* wq_prepared, 
     int32_t *ids = (int32_t*)(w + l.ids), *perm = (int32_t*)(w + l.perm), *uniq = (int32_t*)(w + l.uniq);
     int32_t *seg_off = (int32_t*)(w + l.seg_off), *pair_slot = (int32_t*)(w + l.pair_slot);
     int32_t *sorted_slot = (int32_t*)(w + l.sorted_slot), *n_unique = (int32_t*)(w + l.n_unique);
-    int rc = wq_prepared ? ethos_query_proj_prepared(x, wq, wq_prepared, wq_prepared_bytes, bq, bn_alpha, bn_beta, n_tok, d_model,
-                                                     n_heads, d_query, dtype, w + l.qws, l.qws_bytes, q, stream)
-                         : ethos_query_proj(x, wq, bq, bn_alpha, bn_beta, n_tok, d_model, n_heads, d_query, dtype, w + l.qws,
-                                            l.qws_bytes, q, stream);
-    if (rc) return rc;
     const int64_t rows = n_tok * n_heads;
+    // every stage's checks before the first launch: after an error nothing is enqueued.  (The sort has
+    // none that the sizes and the workspace above leave open.)
+    const char* name = "ethos_layer_forward";
+    int rc = 0;
+    if (n_experts > INT32_MAX || (int64_t)n_sub_keys * n_sub_keys > n_experts)
+        return fail(ETHOS_ESIZE, "%s: %d sub-keys give ids past the %lld experts", name, n_sub_keys, (long long)n_experts);
+    if (wq_prepared && (rc = query_prepared_checks(name, wq_prepared, wq_prepared_bytes, n_tok, d_model, n_heads, d_query, dtype)))
+        return rc;
+    if ((rc = query_proj_checks(name, x, wq, wq_prepared, bq, bn_alpha, bn_beta, n_tok, d_model, n_heads, d_query, dtype, w + l.qws,
+                                l.qws_bytes, q)))
+        return rc;
+    if ((rc = route_checks(name, rows, d_query, n_sub_keys, top_k, k_cand, dtype))) return rc;
+    if (keys_prepared && (rc = route_prepared_checks(name, keys_prepared, keys_prepared_bytes, d_query, n_sub_keys, dtype))) return rc;
+    if ((rc = route_pointer_checks(name, q, sub_keys_1, sub_keys_2, gates, ids))) return rc;
+    if ((rc = expert_forward_checks(name, x, latents, n_experts, w1, w2, wut, xp, uniq, seg_off, n_unique, l.max_u, perm, sorted_slot,
+                                    pair_slot, gates, n_tok, n_heads, top_k, d_latent, d_hidden, d_model, dtype, order, w + l.ews,
+                                    l.ews_bytes, w + l.h, out)))
+        return rc;
+    rc = wq_prepared ? ethos_query_proj_prepared(x, wq, wq_prepared, wq_prepared_bytes, bq, bn_alpha, bn_beta, n_tok, d_model,
+                                                 n_heads, d_query, dtype, w + l.qws, l.qws_bytes, q, stream)
+                     : ethos_query_proj(x, wq, bq, bn_alpha, bn_beta, n_tok, d_model, n_heads, d_query, dtype, w + l.qws,
+                                        l.qws_bytes, q, stream);
+    if (rc) return rc;
     rc = keys_prepared ? ethos_route_topk_prepared(q, sub_keys_1, sub_keys_2, key_norms, keys_prepared, keys_prepared_bytes, rows,
                                                    d_query, n_sub_keys, top_k, k_cand, dtype, gates, ids, stream)
                        : ethos_route_topk(q, sub_keys_1, sub_keys_2, key_norms, rows, d_query, n_sub_keys, top_k, k_cand, dtype,
                                           gates, ids, stream);
     if (rc) return rc;
-    if (dtype == ETHOS_BF16 && l.n_pairs <= ETHOS_SMALL_SORT_PAIRS) {  // with the token projection in the sort's launch
+    if (dtype == ETHOS_BF16 && wut && l.n_pairs <= ETHOS_SMALL_SORT_PAIRS) {  // with the token projection in the sort's launch
         xp = w + l.xp;
         rc = ethos_sort_segment_token_proj(ids, l.n_pairs, n_experts, w + l.shared, l.sort_bytes, perm, uniq, seg_off, pair_slot,
                                            sorted_slot, n_unique, x, w2, wut, n_tok, d_model, d_hidden, dtype, xp, stream);

@@ -479,8 +479,9 @@ int ethos_mla_attention(const void* q, const void* kv, const void* k_rot, int64_
  * The eval-mode layer (model.py:288-343) in one call: ethos_query_proj(_prepared),
  * ethos_route_topk(_prepared), ethos_sort_segment (with the token projection in its launch for
  * bf16 batches of at most ETHOS_SMALL_SORT_PAIRS pairs) and ethos_expert_forward, with every
- * intermediate in the workspace.  The arguments are those calls', with the same limits; an error
- * is the failing call's.  wq_prepared, key_norms, keys_prepared and wut may be NULL.
+ * intermediate in the workspace.  The arguments are those calls', with the same limits, and
+ * n_sub_keys^2 <= n_experts; all are checked before the first stage is enqueued.  wq_prepared,
+ * key_norms, keys_prepared and wut may be NULL.
  *   out        [n_tok, d_model] T
  *   workspace  >= ethos_layer_forward_workspace_bytes(...) bytes, 16-byte aligned (scratch)
  */

@@ -228,10 +228,11 @@ def test_layer_forward_argument_errors_are_codes():
     need = L.ethos_layer_forward_workspace_bytes(4, 2, 4, 64, 32, 256, 32, 1, 0)
     assert need > 0
 
-    def rc(ws=16, ws_bytes=need, dtype=1, order=0, n=4, x=16):
-        s = sizes
-        return L.ethos_layer_forward(x, 16, None, 0, 16, 16, 16, 16, 16, None, None, 0, 16, 16, 16, None, n, s["d"], s["H"], s["dq"],
-                                     s["K"], s["k"], 2 * s["k"], s["E"], s["dl"], s["dh"], dtype, order, ws, ws_bytes, 16, None)
+    def rc(ws=16, ws_bytes=need, dtype=1, order=0, n=4, x=16, kc=8, out=16, lat=16, w1=16, k2=16, kp=None, kpb=0, wut=None, wp=None,
+           **kw):
+        s = dict(sizes, **kw)
+        return L.ethos_layer_forward(x, 16, wp, 0, 16, 16, 16, 16, k2, None, kp, kpb, lat, w1, 16, wut, n, s["d"], s["H"], s["dq"],
+                                     s["K"], s["k"], kc, s["E"], s["dl"], s["dh"], dtype, order, ws, ws_bytes, out, None)
 
     assert rc(dtype=7) == -1
     assert rc(order=2) == -2 and rc(n=-1) == -2
@@ -239,6 +240,15 @@ def test_layer_forward_argument_errors_are_codes():
     assert rc(ws=None) == -3 and rc(x=None) == -3
     assert rc(ws=8) == -4
     assert rc(ws_bytes=need - 1) == -5
+    # errors of the later stages come before the first launch (which has no device here): null and
+    # misaligned pointers, prepared forms too small, candidates, sizes, ids past the experts
+    big = dict(ws_bytes=1 << 40)
+    assert rc(out=None) == -3 and rc(lat=None) == -3 and rc(w1=None) == -3 and rc(k2=None) == -3
+    assert rc(out=8) == -4 and rc(w1=24) == -4 and rc(wut=8) == -4 and rc(k2=8) == -4
+    assert rc(kp=16, kpb=1) == -2 and rc(wp=16) == -5
+    assert rc(kc=17) == -2 and rc(K=64, E=4096, kc=40, **big) == -6 and rc(dh=40, **big) == -6 and rc(dl=10) == -6
+    assert rc(K=17, kc=8) == -2 and b"past" in L.ethos_last_error()
+    assert rc(dl=0) == -2 and rc(dq=30, **big) == -6
 
 
 def test_training_entry_points_argument_errors_are_codes():

@@ -297,6 +297,23 @@ def test_one_call_forward_matches_stages(name, n, hidden):
     assert seen and torch.equal(a, b)
 
 
+@pytest.mark.parametrize("n", [5, 64, 200])
+def test_one_call_forward_without_prepared_forms(n):
+    """The one-call layer with NULL for every prepared form (the library transposes and prepares by
+    itself) gives the bits of the prepared one, on either side of the small sort's limit."""
+    sh = SHAPES["cfg3"]
+    x, sd = make_inputs(sh.with_tokens(n), signal=True)
+    m = ethos_amd.EthosExpertLayer(sh.config()).to(sh.torch_dtype)
+    m.load_state_dict(sd)
+    m, x = m.cuda().eval(), x.cuda()
+    with torch.no_grad():
+        want = m.forward_flat(x)
+        r = m.router
+        gen = m._generator_params(x.dtype, x.device)
+        got = hip.layer_forward(x, r._packed(x.dtype, x.device), r._key_norms, None, None, (*gen[:3], None), m.num_experts, m.top_k, False)
+    assert torch.equal(got, want)
+
+
 def _two_layers(name):
     sh = SHAPES[name]
     x, sd = make_inputs(sh, signal=True)
