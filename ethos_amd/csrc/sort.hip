@@ -34,6 +34,8 @@
 // writes an expert -> slot table at the heads instead (one store per unique expert) and a
 // gather over the ids in pair order writes pair_slot with coalesced stores.
 
+#include <type_traits>
+
 #include "ethos_common.hpp"
 #include "ethos_launch.hpp"
 #include "ethos_tp.hpp"
@@ -729,13 +731,24 @@ constexpr int kSmallPer = kSmallChunks / kSmallWaves;        // chunks per wave 
 // Most batches need no radix passes: the words differ, so any order-preserving spread over
 // buckets (the key's top 11 bits; places within a bucket in the order the LDS counters give
 // them) followed by ranking each word among its bucket's words ends in the one sorted order.
-// When some bucket holds more than kSmallBucketMax words (few distinct experts) the ranking
-// would cost more than the passes, which then run (they cost 0.5 to 1.5 us more than without
-// the attempt).  us, routed pairs of 262,144 experts, passes | buckets: 128 pairs 7.7 | 5.6,
-// 4,096 14.7 | 10.0, 8,192 23.3 | 15.8, 16,384 40.0 | 28.9.
+// Ranking takes time with the sum of the buckets' squared counts, S, and with the largest, M:
+// about S / 38,000 + M / 75 us; the passes take 1.5 us and 0.95 per 1,024 pairs more than the
+// buckets without it.  So the words are ranked where S + 500 M is below that line in n
+// (small_line), decided twice: before the counting, from the coincidences among 256 spread words
+// in waves of 64, so that a batch of few experts does not pay for the counting, and after it, with
+// the counting's time added to the line, from the counts themselves.  Up to 128 pairs the words are
+// always ranked.  us, passes always | counted always, then ranked up to 96 a bucket | as here, of
+// 262,144 experts: all of them in use, 128 pairs 7.4 | 5.0 | 4.3, 1,024 8.2 | 5.9 | 5.8, 4,096 15.0 |
+// 9.9 | 9.6, 16,384 43.0 | 29.4 | 29.4; 32 of them, 1,024 8.2 | 6.6 | 6.5, 4,096 14.5 | 17.2 | 14.5,
+// 16,384 39.7 | 44.5 | 40.6; 3% of the pairs with one, 4,096 15.0 | 17.4 | 11.7, 16,384 43.0 | 47.0 |
+// 38.2.  So a batch of few experts pays up to 0.8 us, at 16,384 pairs, and none up to 4,096.
 constexpr int kSmallBucketBits = 11, kSmallBuckets = 1 << kSmallBucketBits;
-constexpr uint32_t kSmallBucketMax = 96, kSmallCrowded = 24;
-constexpr int kSmallSample = 256;
+constexpr int kSmallSure = 128;
+constexpr int kSmallSample = 4;  // waves that look at 64 words each, one a SIMD
+constexpr float kSmallLargest = 500.0f;
+__device__ __forceinline__ float small_line(int n, bool counted) {
+    return counted ? 71000.0f + 45.0f * (float)n : 56000.0f + 36.0f * (float)n;
+}
 static_assert(kSmallBuckets == 2 * kSmallWaves * 64, "two buckets a thread");
 
 // LDS of the small sort: the words twice, per-wave digit counts (then bases, < 2^14), head
@@ -743,6 +756,19 @@ static_assert(kSmallBuckets == 2 * kSmallWaves * 64, "two buckets a thread");
 constexpr size_t kSmallBufB = 2 * (size_t)kSmallMax * 4, kSmallCntB = (size_t)kSmallWaves * kRadix * 2;
 constexpr size_t kSmallLds = kSmallBufB + kSmallCntB + (size_t)kSmallChunks * 8 + (size_t)kSmallChunks * 4 +
                              (size_t)kSmallWaves * 4;
+
+// f(j) for the thread's pairs tid + j * 1,024 of n, the index known to the compiler, so that what f
+// keeps for each stays in registers of its own: a loop that ends early it may leave rolled, with its
+// loads waited for one by one.
+template <int J = 0, typename F>
+__device__ __forceinline__ void small_chunks(int n, F&& f) {
+    if constexpr (J < kSmallPer) {
+        if (J * kSmallWaves * 64 < n) {
+            f(std::integral_constant<int, J>{});
+            small_chunks<J + 1>(n, f);
+        }
+    }
+}
 
 __device__ __forceinline__ void sort_small_body(unsigned char* lds, const int32_t* __restrict__ ids, int n,
                                                 int key_bits_, int vb, int passes, int32_t* __restrict__ perm,
@@ -759,45 +785,71 @@ __device__ __forceinline__ void sort_small_body(unsigned char* lds, const int32_
     const int n_chunks = (n + 63) / 64;
     const int cpw = (n_chunks + kSmallWaves - 1) / kSmallWaves;  // chunks per wave (<= kSmallPer)
     const int c0 = wave * cpw;
-    constexpr int kIn = kSmallMax / (kSmallWaves * 64), kStep = kSmallWaves * 64;
+    constexpr int kStep = kSmallWaves * 64;
     uint32_t* hist = reinterpret_cast<uint32_t*>(lds + kSmallBufB);  // then each bucket's first position
     const int bsh = vb + (key_bits_ > kSmallBucketBits ? key_bits_ - kSmallBucketBits : 0);  // word -> bucket
-    bool bucketed;
+    uint32_t first;     // this thread's first word, pair tid
+    bool clear = true;  // the digit counts' storage holds zeros
     {
-        // all of the thread's ids in flight at once (one workgroup: latency, not bandwidth)
-        uint32_t word[kIn], off[kIn];
-#pragma unroll
-        for (int j = 0; j < kIn; ++j) {
+        uint32_t word[kSmallPer], rank[kSmallPer];  // pair tid + j * 1,024
+        // all of the thread's ids in flight at once (one workgroup: latency, not bandwidth), and in
+        // the last waves one of the sample: the waves' 64 are spread over the batch, at uneven distances
+        const bool sure = n <= kSmallSure, sample = !sure && wave >= kSmallWaves - kSmallSample;
+        // (loaded in every wave: a branch around the load would end in a wait for it)
+        const uint32_t place = (uint32_t)(lane * kSmallSample + (wave & (kSmallSample - 1)));
+        uint32_t mine = (uint32_t)ids[(((place << 7) | (place * 2654435761u >> 25)) * (uint32_t)n) >> 15];
+        small_chunks(n, [&](auto j) {
             const int i = tid + j * kStep;
-            word[j] = i < n ? (uint32_t)ids[i] : 0u;
-        }
-        for (int e = tid; e < kSmallBuckets; e += kStep) hist[e] = 0;
-        __syncthreads();
+            word[j] = (uint32_t)ids[i < n ? i : n - 1];
+        });
+        for (int e = tid; e < (int)(kSmallCntB / 16); e += kStep) reinterpret_cast<uint4*>(hist)[e] = make_uint4(0, 0, 0, 0);
+        if (sample) {
+            mine = mine > kmax ? kmax : mine;
+            const uint32_t b = key_bits_ > kSmallBucketBits ? mine >> (key_bits_ - kSmallBucketBits) : mine;
+            uint64_t peers = ~0ull;
 #pragma unroll
-        for (int j = 0; j < kIn; ++j) {
-            if (j * kStep >= n) break;
-            const uint32_t kk = word[j] > kmax ? kmax : word[j];  // ids outside [0, 2^key_bits) (a caller error) stay in range
-            word[j] = (kk << vb) | (uint32_t)(tid + j * kStep);
-        }
-        // one bucket's counter takes its words one after the other: the first 256 words tell a
-        // crowded one before the rest are counted
-        off[0] = tid < kSmallSample && tid < n ? atomicAdd(&hist[word[0] >> bsh], 1u) : 0u;
-        const bool crowded = __syncthreads_or(off[0] >= (n <= kSmallSample ? kSmallBucketMax : kSmallCrowded));
-        if (!crowded) {
-            if (tid >= kSmallSample && tid < n) off[0] = atomicAdd(&hist[word[0] >> bsh], 1u);
-#pragma unroll
-            for (int j = 1; j < kIn; ++j) {
-                if (j * kStep >= n) break;
-                off[j] = tid + j * kStep < n ? atomicAdd(&hist[word[j] >> bsh], 1u) : 0u;
+            for (int i = 0; i < kSmallBucketBits; ++i) {
+                const uint64_t m = __ballot((b >> i) & 1u);
+                peers &= (b >> i) & 1u ? m : ~m;
             }
+            const float others = (float)(__popcll(peers) - 1);
+            const float pairs = wave_sum(others), triples = wave_sum(others * (others - 1.0f));
+            if (lane == 0) reinterpret_cast<float2*>(cbase)[wave - (kSmallWaves - kSmallSample)] = make_float2(pairs, triples);
         }
-        uint32_t top = 0;
-        if (!crowded) {
+        small_chunks(n, [&](auto j) {
+            const uint32_t kk = word[j] > kmax ? kmax : word[j];  // ids outside [0, 2^key_bits) (a caller error) stay in range
+            const int i = tid + j * kStep;
+            word[j] = (kk << vb) | (uint32_t)i;
+            if (cpw > 1 && i < n) buf[0][i] = word[j];
+        });
+        first = word[0];
+        __syncthreads();
+        bool ranked = true;
+        if (!sure) {
+            float pairs = 0.0f, triples = 0.0f;
+#pragma unroll
+            for (int w = 0; w < kSmallSample; ++w) {
+                const float2 v = reinterpret_cast<const float2*>(cbase)[w];
+                pairs += v.x;
+                triples += v.y;
+            }
+            // words of one bucket among a wave's 64: two of them with the sum of the buckets' squared
+            // shares, three with that of their cubes, which over the former is a crowded one's share
+            const float fn = (float)n;
+            const float squares = fn + fn * fn * pairs * (1.0f / (kSmallSample * 64.0f * 63.0f));
+            const float largest = pairs > 0.0f ? fn * triples * __builtin_amdgcn_rcpf(62.0f * pairs) : 0.0f;
+            ranked = squares + kSmallLargest * largest <= small_line(n, false);
+        }
+        if (ranked) {
+            clear = false;
+            small_chunks(n, [&](auto j) {
+                rank[j] = tid + j * kStep < n ? atomicAdd(&hist[word[j] >> bsh], 1u) : 0u;
+            });
             __syncthreads();
-            // two buckets a thread: their first positions, and the largest count
+            // two buckets a thread: their first positions, the largest count and the squares
             const uint32_t n0 = hist[2 * tid], n1 = hist[2 * tid + 1];
-            uint32_t inc = n0 + n1;
-            top = n0 > n1 ? n0 : n1;
+            uint32_t inc = n0 + n1, top = n0 > n1 ? n0 : n1;
+            const float squares = wave_sum((float)(n0 * n0 + n1 * n1));
 #pragma unroll
             for (int o = 1; o < 64; o <<= 1) {
                 const uint32_t u = __shfl_up(inc, o, 64), v = __shfl_xor(top, o, 64);
@@ -807,59 +859,62 @@ __device__ __forceinline__ void sort_small_body(unsigned char* lds, const int32_
             if (lane == 63) {
                 wsum[wave] = inc;
                 cbase[wave] = top;
+                cbase[kSmallWaves + wave] = __float_as_uint(squares);
             }
             __syncthreads();
             uint32_t run = inc - n0 - n1;
             top = 0;
+            float sq = 0.0f;
 #pragma unroll
             for (int w = 0; w < kSmallWaves; ++w) {
                 run += w < wave ? wsum[w] : 0u;
                 top = top > cbase[w] ? top : cbase[w];
+                sq += __uint_as_float(cbase[kSmallWaves + w]);
             }
             hist[2 * tid] = run;
             hist[2 * tid + 1] = run + n0;
             if (tid == kStep - 1) hist[kSmallBuckets] = run + n0 + n1;
+            ranked = sure || sq + kSmallLargest * (float)top <= small_line(n, true);
             __syncthreads();
         }
-        bucketed = !crowded && top <= kSmallBucketMax;
-#pragma unroll
-        for (int j = 0; j < kIn; ++j) {
-            if (j * kStep >= n) break;
-            const int i = tid + j * kStep;
-            if (i < n) buf[0][bucketed ? hist[word[j] >> bsh] + off[j] : (uint32_t)i] = word[j];
+        if (ranked) {
+            small_chunks(n, [&](auto j) {
+                if (tid + j * kStep < n) buf[1][hist[word[j] >> bsh] + rank[j]] = word[j];
+            });
+            __syncthreads();
+            // each word's place in its bucket: the words below it there (all words differ)
+            for (int i = tid; i < n; i += kStep) {
+                const uint32_t wd = buf[1][i];
+                const uint32_t b0 = hist[wd >> bsh], b1 = hist[(wd >> bsh) + 1];
+                uint32_t r = b0;
+                uint32_t q = b0;
+                for (; q + 4 <= b1; q += 4) {
+                    const uint32_t x0 = buf[1][q], x1 = buf[1][q + 1], x2 = buf[1][q + 2], x3 = buf[1][q + 3];
+                    r += (x0 < wd ? 1u : 0u) + (x1 < wd ? 1u : 0u) + (x2 < wd ? 1u : 0u) + (x3 < wd ? 1u : 0u);
+                }
+                for (; q < b1; ++q) r += buf[1][q] < wd ? 1u : 0u;
+                buf[0][r] = wd;
+            }
+            passes = 0;
+            __syncthreads();
         }
-        __syncthreads();
     }
     int cur = 0;
-    if (bucketed) {
-        // each word's place in its bucket: the words below it there (all words differ)
-        for (int i = tid; i < n; i += kStep) {
-            const uint32_t wd = buf[0][i];
-            const uint32_t b0 = hist[wd >> bsh], b1 = hist[(wd >> bsh) + 1];
-            uint32_t r = b0;
-            uint32_t q = b0;
-            for (; q + 4 <= b1; q += 4) {
-                const uint32_t x0 = buf[0][q], x1 = buf[0][q + 1], x2 = buf[0][q + 2], x3 = buf[0][q + 3];
-                r += (x0 < wd ? 1u : 0u) + (x1 < wd ? 1u : 0u) + (x2 < wd ? 1u : 0u) + (x3 < wd ? 1u : 0u);
-            }
-            for (; q < b1; ++q) r += buf[0][q] < wd ? 1u : 0u;
-            buf[1][r] = wd;
-        }
-        cur = 1;
-        passes = 0;
-        __syncthreads();
-    }
     for (int p = 0; p < passes; ++p) {
         const int shift = vb + kRadixBits * p;
-        for (int e = tid; e < kSmallWaves * kRadix; e += kSmallWaves * 64) cnt[e / kRadix][e % kRadix] = 0;
-        __syncthreads();
+        if (!clear) {
+            for (int e = tid; e < (int)(kSmallCntB / 16); e += kStep) reinterpret_cast<uint4*>(hist)[e] = make_uint4(0, 0, 0, 0);
+            __syncthreads();
+        }
+        clear = false;
         uint32_t word[kSmallPer], rank[kSmallPer];
 #pragma unroll
         for (int j = 0; j < kSmallPer; ++j) {
             if (j >= cpw) break;  // wave-uniform: the wave's chunks end here
             const int idx = (c0 + j) * 64 + lane;
             const bool v = idx < n;
-            word[j] = v ? buf[cur][idx] : 0u;
+            // (a wave's one chunk of the first pass is still in its registers)
+            word[j] = p == 0 && cpw == 1 ? first : v ? buf[cur][idx] : 0u;
             const uint32_t dg = (word[j] >> shift) & (kRadix - 1);
             const uint64_t peers = peer_mask(dg, __ballot(v));
             const uint32_t below = (uint32_t)__popcll(peers & lanemask_lt(lane));
@@ -899,7 +954,7 @@ __device__ __forceinline__ void sort_small_body(unsigned char* lds, const int32_
         __syncthreads();
 #pragma unroll
         for (int j = 0; j < kSmallPer; ++j) {
-            if (j >= cpw) break;
+            if (j >= cpw) break;  // wave-uniform: the wave's chunks end here
             const int idx = (c0 + j) * 64 + lane;
             if (idx < n) buf[cur ^ 1][cnt[wave][(word[j] >> shift) & (kRadix - 1)] + rank[j]] = word[j];
         }

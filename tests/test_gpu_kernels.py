@@ -710,6 +710,44 @@ def test_sort_segment_token_proj_matches_separate_calls(n_tok, H, k, d, dh, E, d
     assert torch.equal(xp, xp_ref)
 
 
+def _small_sort_sample(n):
+    """The positions that the small sort looks at before it chooses."""
+    place = np.arange(256, dtype=np.uint64)
+    frac = ((place * 2654435761) & 0xffffffff) >> 25
+    return np.unique((((place << 7) | frac) * n) >> 15).astype(np.int64)
+
+
+@pytest.mark.parametrize("E", [40, 2048, 65536, 262144])
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 128, 129, 257, 1000, 1024, 2049, 8191, 16384])
+def test_small_sort_choices_agree(n, E):
+    """The small sort's two ways (ranking in buckets, radix passes) and its two looks at the batch
+    give the one stable order: spread and few experts, one hot expert, and batches whose sampled
+    words are all one expert's, or none of the hot one's (chosen late)."""
+    rng = np.random.default_rng(n + E)
+    at = _small_sort_sample(n)
+    for kind in ("spread", "1", "8", "64", "hot0.1", "hot0.5", "sampled", "hidden"):
+        ids = rng.integers(0, E, n)
+        if kind.isdigit():
+            ids = rng.integers(0, E, int(kind))[rng.integers(0, int(kind), n)]
+        elif kind.startswith("hot"):
+            ids[rng.random(n) < float(kind[3:])] = E // 3
+        elif kind == "sampled":
+            ids[at] = E // 3
+        elif kind == "hidden":
+            keep = ids[at]
+            ids[:] = E // 3
+            ids[at] = keep
+        ids = ids.astype(np.int32)
+        seg = {k: v.cpu().numpy() for k, v in hip.sort_segment(torch.from_numpy(ids).cuda(), E).items() if torch.is_tensor(v)}
+        perm = np.argsort(ids, kind="stable")
+        uniq, first, inv = np.unique(ids, return_index=True, return_inverse=True)
+        U = len(uniq)
+        assert int(seg["n_unique"][0]) == U and np.array_equal(seg["perm"], perm), kind
+        assert np.array_equal(seg["uniq"][:U], uniq) and np.array_equal(seg["pair_slot"], inv), kind
+        assert np.array_equal(seg["sorted_slot"], inv[perm]), kind
+        assert np.array_equal(seg["seg_off"][:U + 1], np.append(np.searchsorted(ids[perm], uniq), n)), kind
+
+
 @pytest.mark.parametrize("n,d,cols", [(1, 4, 4), (33, 36, 68), (64, 100, 64), (130, 256, 192)])
 def test_chain_tiles_agree(n, d, cols):
     """The float32 projections' float64 chains do not depend on the tile edge: a batch tiled by 64
