@@ -67,25 +67,33 @@ def _packing():
 
 class _Made:
     """The key of tensors that are made once and read by later calls on any stream: another stream's
-    first call waits for their making and holds their memory from then on.  What a graph capture
-    makes exists only after a replay, so it serves no call outside (`once`: the key is that of a
-    single pass, which may go on using it).  A copied or unpickled module makes its own."""
+    first call waits for their making and holds their memory from then on.  `once`: the key is that
+    of a single pass, which goes on using them on its stream.  What a graph capture makes exists
+    only after a replay, so it serves no call outside.  A copied or unpickled module makes its own."""
 
-    def __init__(self, key=None, tensors=(), once: bool = False):
-        self.key, self.event = key, None
-        self.tensors = [t for t in tensors if t is not None and t.is_cuda]
-        if not self.tensors:
+    def __init__(self):
+        self.key, self.event, self.tensors, self.streams = None, None, (), None
+
+    def clear(self) -> None:
+        self.key = None
+
+    def set(self, key, tensors, once: bool = False) -> None:
+        self.key, self.tensors, self.streams = key, (), None
+        on = [t for t in tensors if t is not None and t.is_cuda]
+        if not on or once:
             return
         if torch.cuda.is_current_stream_capturing():
-            self.key = key if once else None
-        else:
-            self.event, self.streams = torch.cuda.Event(), {hip._stream()}
-            self.event.record()
+            self.key = None
+            return
+        if self.event is None:
+            self.event = torch.cuda.Event()
+        self.event.record()
+        self.tensors, self.streams = on, {hip._stream()}
 
     def fits(self, key) -> bool:
         if key != self.key:
             return False
-        if self.event is not None:
+        if self.streams is not None:
             s = hip._stream()
             # (a capture starts after the work before it: torch.cuda.graph waits for the device)
             if s not in self.streams and not torch.cuda.is_current_stream_capturing():
@@ -351,7 +359,7 @@ class ProductKeyRouter(nn.Module):
                 # until a parameter changes
                 self._wq_prepared = hip.query_proj_prepare(wq) if wq.is_cuda else None
             self._cache = (wq, bq, k1, k2)
-            self._cache_made = _Made(key, (*self._cache, self._key_norms, self._keys_prepared, self._wq_prepared), mode > 0)
+            self._cache_made.set(key, (*self._cache, self._key_norms, self._keys_prepared, self._wq_prepared), mode > 0)
         return self._cache
 
     def _bn_coefficients(self, device: torch.device):
@@ -371,7 +379,7 @@ class ProductKeyRouter(nn.Module):
                 else:
                     ab = [_bn_eval_coefficients(m, self.d_query) for m in norms]
                     self._bn = tuple(torch.from_numpy(np.stack(c)).contiguous().to(device) for c in zip(*ab))
-            self._bn_made = _Made(key, self._bn)
+            self._bn_made.set(key, self._bn)
         return self._bn
 
     def _packed(self, dtype: torch.dtype, device: torch.device):
@@ -415,7 +423,7 @@ class ProductKeyRouter(nn.Module):
             with _packing():
                 ones = torch.ones((self.num_heads, self.d_query), dtype=torch.float32, device=x_flat.device)
                 self._identity = (ones, torch.zeros_like(ones))
-            self._identity_made = _Made(x_flat.device, self._identity)
+            self._identity_made.set(x_flat.device, self._identity)
         q_lin = hip.query_proj(x_flat, wq, bq, *self._identity, prepared=self._wq_prepared)
         if self._bn_one_call(x_flat):
             m0 = self.query_norms[0]
@@ -442,7 +450,7 @@ class ProductKeyRouter(nn.Module):
                                      m0.momentum if m0.momentum is not None else 0.1, m0.eps, batch=batch)
             if track:
                 torch._foreach_add_([m.num_batches_tracked for m in self.query_norms], 1)
-                self._bn_made = _Made()  # the running statistics' version counters do not move
+                self._bn_made.clear()  # the running statistics' version counters do not move
             return out
         outs = []
         for h, m in enumerate(self.query_norms):
@@ -455,7 +463,7 @@ class ProductKeyRouter(nn.Module):
         # batch_norm updated the running statistics in place without bumping their version
         # counters, so the cached eval-mode coefficients are stale
         if any(m.training and m.track_running_stats for m in self.query_norms):
-            self._bn_made = _Made()
+            self._bn_made.clear()
         return torch.stack(outs, dim=1).contiguous()
 
     def route(self, x_flat: torch.Tensor, mark=None):
@@ -574,7 +582,7 @@ class EthosExpertLayer(nn.Module):
                     gen = tuple(p.detach().to(device=device, dtype=dtype).contiguous() for p in ps)
                 wut = gen[2][: self.d_model].t().contiguous() if dtype == torch.bfloat16 else None
             self._gen = gen + (wut,)
-            self._gen_made = _Made(key, (t for t in self._gen if all(t is None or t.data_ptr() != p.data_ptr() for p in ps)), mode > 0)
+            self._gen_made.set(key, [t for t in self._gen if all(t is None or t.data_ptr() != p.data_ptr() for p in ps)], mode > 0)
         return self._gen
 
     def _expert_stages(self, x_flat: torch.Tensor, gates: torch.Tensor, seg: dict, xp: torch.Tensor | None = None):
