@@ -30,6 +30,7 @@ from __future__ import annotations
 
 import contextlib
 import math
+from typing import NamedTuple
 
 import numpy as np
 import torch
@@ -65,47 +66,65 @@ def _packing():
         yield
 
 
-class _Made:
-    """The key of tensors that are made once and read by later calls on any stream: another stream's
-    first call waits for their making and holds their memory from then on.  `once`: the key is that
-    of a single pass, which goes on using them on its stream.  What a graph capture makes exists
-    only after a replay, so it serves no call outside.  A copied or unpickled module makes its own."""
+class _Kept:
+    """A value with tensors that is made once and read by later calls of any thread, on any stream:
+    another stream's first call waits for the making and holds the memory from then on.  `once`: the
+    key is that of a single pass, which goes on using the value on its stream.  What a graph capture
+    makes exists only after a replay, so it is not kept for calls outside.  A copied or unpickled
+    module makes its own."""
 
     def __init__(self):
-        self.key, self.event, self.tensors, self.streams = None, None, (), None
+        self.entry = None  # (key, value, event, the raw streams that are past it, tensors), replaced whole
 
-    def clear(self) -> None:
-        self.key = None
-
-    def set(self, key, tensors, once: bool = False) -> None:
-        self.key, self.tensors, self.streams = key, (), None
-        on = [t for t in tensors if t is not None and t.is_cuda]
-        if not on or once:
-            return
-        if torch.cuda.is_current_stream_capturing():
-            self.key = None
-            return
-        if self.event is None:
-            self.event = torch.cuda.Event()
-        self.event.record()
-        self.tensors, self.streams = on, {hip._stream()}
-
-    def fits(self, key) -> bool:
-        if key != self.key:
-            return False
-        if self.streams is not None:
+    def get(self, key):
+        entry = self.entry
+        if entry is None or entry[0] != key:
+            return None
+        _, value, event, streams, tensors = entry
+        if event is not None:
             s = hip._stream()
             # (a capture starts after the work before it: torch.cuda.graph waits for the device)
-            if s not in self.streams and not torch.cuda.is_current_stream_capturing():
+            if s not in streams and not torch.cuda.is_current_stream_capturing():
                 stream = torch.cuda.current_stream()
-                stream.wait_event(self.event)
-                for t in self.tensors:
+                stream.wait_event(event)
+                for t in tensors:
                     t.record_stream(stream)
-                self.streams.add(s)
-        return True
+                streams.add(s)
+        return value
+
+    def put(self, key, value, tensors, once: bool = False):
+        on = [t for t in tensors if t is not None and t.is_cuda]
+        event = None
+        if on and not once:
+            if torch.cuda.is_current_stream_capturing():
+                return value
+            event = torch.cuda.Event()
+            event.record()
+        self.entry = (key, value, event, {hip._stream()} if event is not None else None, on)
+        return value
+
+    def clear(self) -> None:
+        self.entry = None
+
+    @property
+    def value(self):
+        entry = self.entry
+        return None if entry is None else entry[1]
 
     def __reduce__(self):
-        return _Made, ()
+        return _Kept, ()
+
+
+class _Weights(NamedTuple):
+    """The routing's packed parameters in one dtype on one device."""
+
+    wq: torch.Tensor
+    bq: torch.Tensor
+    k1: torch.Tensor
+    k2: torch.Tensor
+    key_norms: torch.Tensor
+    keys_prepared: torch.Tensor | None  # the sub-keys in the scoring MFMAs' fragment order
+    wq_prepared: torch.Tensor | None    # bf16: the projection weights' digit planes
 
 
 def _gelu_grad(x: torch.Tensor) -> torch.Tensor:
@@ -302,16 +321,8 @@ class ProductKeyRouter(nn.Module):
         self.query_norms = nn.ModuleList([nn.BatchNorm1d(self.d_query) for _ in range(self.num_heads)])
         self.sub_keys_1 = nn.Embedding(self.num_sub_keys, self.d_query // 2)
         self.sub_keys_2 = nn.Embedding(self.num_sub_keys, self.d_query // 2)
-        self._cache_made = _Made()
-        self._cache = None
         self._train_pass = 0
-        self._bn_made = _Made()
-        self._bn = None
-        self._identity_made = _Made()
-        self._identity = None
-        self._key_norms = None
-        self._keys_prepared = None
-        self._wq_prepared = None
+        self._kept_weights, self._kept_bn, self._kept_identity = _Kept(), _Kept(), _Kept()
 
     # -- parameter packing (cached until a parameter changes; made anew by every training pass) ---
     def _weight_sources(self) -> list:
@@ -343,30 +354,33 @@ class ProductKeyRouter(nn.Module):
         evaluation after them."""
         return self._train_pass if any(m.training for m in self._modules["query_norms"]._modules.values()) else 0
 
-    def _packed_weights(self, dtype: torch.dtype, device: torch.device, mode: int | None = None):
+    def _packed_weights(self, dtype: torch.dtype, device: torch.device, mode: int | None = None) -> _Weights:
         mode = self._pack_mode() if mode is None else mode
         key = (dtype, device, mode, tuple((t.data_ptr(), t._version) for t in self._weight_sources() if t is not None))
-        if not self._cache_made.fits(key):
+        w = self._kept_weights.get(key)
+        if w is None:
             with _packing():
                 wq = torch.stack([m.weight.detach() for m in self.query_projs]).to(device=device, dtype=dtype).contiguous()
                 bq = torch.stack([m.bias.detach() for m in self.query_projs]).to(device=device, dtype=dtype).contiguous()
                 k1 = self.sub_keys_1.weight.detach().to(device=device, dtype=dtype).contiguous()
                 k2 = self.sub_keys_2.weight.detach().to(device=device, dtype=dtype).contiguous()
-                self._key_norms = hip.key_norm_bounds(k1, k2)
-                # the sub-keys in the scoring MFMAs' fragment order
-                self._keys_prepared = hip.route_prepare_keys(k1, k2) if k1.is_cuda else None
-                # the projection weights' prepared form (bf16: digit planes), reused by every call
-                # until a parameter changes
-                self._wq_prepared = hip.query_proj_prepare(wq) if wq.is_cuda else None
-            self._cache = (wq, bq, k1, k2)
-            self._cache_made.set(key, (*self._cache, self._key_norms, self._keys_prepared, self._wq_prepared), mode > 0)
-        return self._cache
+                w = _Weights(wq, bq, k1, k2, hip.key_norm_bounds(k1, k2), hip.route_prepare_keys(k1, k2) if k1.is_cuda else None,
+                             hip.query_proj_prepare(wq) if wq.is_cuda else None)
+            self._kept_weights.put(key, w, w, mode > 0)
+        return w
+
+    # the last packed weights' prepared forms, and the identity affine of the training-mode projection
+    _key_norms = property(lambda self: self._kept_weights.value.key_norms)
+    _keys_prepared = property(lambda self: self._kept_weights.value.keys_prepared)
+    _wq_prepared = property(lambda self: self._kept_weights.value.wq_prepared)
+    _identity = property(lambda self: self._kept_identity.value)
 
     def _bn_coefficients(self, device: torch.device):
         """(alpha, beta) of the eval-mode BatchNorms, float32 [H, d_query] on the device."""
         ts = self._bn_sources()
         key = (device, tuple((t.data_ptr(), t._version) for t in ts if t is not None))
-        if not self._bn_made.fits(key):
+        bn = self._kept_bn.get(key)
+        if bn is None:
             with _packing():
                 norms, H = list(self.query_norms), self.num_heads
                 one = ts[0].dtype if ts[0] is not None else None
@@ -374,17 +388,17 @@ class ProductKeyRouter(nn.Module):
                         and all(m.affine and m.track_running_stats for m in norms) and one in (torch.float32, torch.bfloat16)
                         and all(t is not None and t.dtype == one and t.device == device and t.is_contiguous() for t in ts)):
                     # on the device: the host evaluation below waits for four tensors of every head
-                    self._bn = hip.bn_coefficients(*([m.detach() for m in ts[i::4]] for i in range(4)), norms[0].eps, self.d_query,
-                                                   one, device)
+                    bn = hip.bn_coefficients(*([m.detach() for m in ts[i::4]] for i in range(4)), norms[0].eps, self.d_query,
+                                             one, device)
                 else:
                     ab = [_bn_eval_coefficients(m, self.d_query) for m in norms]
-                    self._bn = tuple(torch.from_numpy(np.stack(c)).contiguous().to(device) for c in zip(*ab))
-            self._bn_made.set(key, self._bn)
-        return self._bn
+                    bn = tuple(torch.from_numpy(np.stack(c)).contiguous().to(device) for c in zip(*ab))
+            self._kept_bn.put(key, bn, bn)
+        return bn
 
     def _packed(self, dtype: torch.dtype, device: torch.device):
         """What an evaluation reads: the packed weights and the BatchNorm coefficients."""
-        return self._packed_weights(dtype, device, 0) + tuple(self._bn_coefficients(device))
+        return self._packed_weights(dtype, device, 0)[:4] + tuple(self._bn_coefficients(device))
 
     def _bn_uses_batch_stats(self) -> bool:
         return any(m.training or not m.track_running_stats for m in self._modules["query_norms"]._modules.values())
@@ -410,21 +424,32 @@ class ProductKeyRouter(nn.Module):
     def queries(self, x_flat: torch.Tensor, packed=None) -> torch.Tensor:
         """Per-head queries after BatchNorm, [n, H, d_query] (model.py:215-216).  `packed`:
         the result of _packed for x_flat's dtype and device, if the caller has it."""
-        if not self._bn_uses_batch_stats():
-            wq, bq, _, _, alpha, beta = packed if packed is not None else self._packed(x_flat.dtype, x_flat.device)
-            return hip.query_proj(x_flat, wq, bq, alpha, beta, prepared=self._wq_prepared)
+        batch = self._bn_uses_batch_stats()
+        if packed is not None:
+            w = _Weights(*packed[:4], None, None, None)
+            return self._batch_queries(x_flat, w) if batch else hip.query_proj(x_flat, w.wq, w.bq, *packed[4:])
+        w = self._pass_weights(x_flat, batch)
+        return self._batch_queries(x_flat, w) if batch else self._eval_queries(x_flat, w)
+
+    def _pass_weights(self, x_flat: torch.Tensor, batch: bool) -> _Weights:
+        """The packed weights of a pass that starts here."""
+        if batch:
+            self._train_pass += 1
+        return self._packed_weights(x_flat.dtype, x_flat.device, None if batch else 0)
+
+    def _eval_queries(self, x_flat: torch.Tensor, w: _Weights) -> torch.Tensor:
+        return hip.query_proj(x_flat, w.wq, w.bq, *self._bn_coefficients(x_flat.device), prepared=w.wq_prepared)
+
+    def _batch_queries(self, x_flat: torch.Tensor, w: _Weights) -> torch.Tensor:
         # Training-mode BatchNorm normalises with batch statistics and updates the
         # running stats: project with an identity affine, then normalise the projected queries.
-        if packed is None:
-            self._train_pass += 1
-            packed = self._packed_weights(x_flat.dtype, x_flat.device)
-        wq, bq = packed[:2]
-        if not self._identity_made.fits(x_flat.device):
+        one = self._kept_identity.get(x_flat.device)
+        if one is None:
             with _packing():
                 ones = torch.ones((self.num_heads, self.d_query), dtype=torch.float32, device=x_flat.device)
-                self._identity = (ones, torch.zeros_like(ones))
-            self._identity_made.set(x_flat.device, self._identity)
-        q_lin = hip.query_proj(x_flat, wq, bq, *self._identity, prepared=self._wq_prepared)
+                one = (ones, torch.zeros_like(ones))
+            self._kept_identity.put(x_flat.device, one, one)
+        q_lin = hip.query_proj(x_flat, w.wq, w.bq, *one, prepared=w.wq_prepared)
         if self._bn_one_call(x_flat):
             m0 = self.query_norms[0]
             ts, track = self._bn_sources(), m0.track_running_stats
@@ -450,7 +475,7 @@ class ProductKeyRouter(nn.Module):
                                      m0.momentum if m0.momentum is not None else 0.1, m0.eps, batch=batch)
             if track:
                 torch._foreach_add_([m.num_batches_tracked for m in self.query_norms], 1)
-                self._bn_made.clear()  # the running statistics' version counters do not move
+                self._kept_bn.clear()  # the running statistics' version counters do not move
             return out
         outs = []
         for h, m in enumerate(self.query_norms):
@@ -463,22 +488,18 @@ class ProductKeyRouter(nn.Module):
         # batch_norm updated the running statistics in place without bumping their version
         # counters, so the cached eval-mode coefficients are stale
         if any(m.training and m.track_running_stats for m in self.query_norms):
-            self._bn_made.clear()
+            self._kept_bn.clear()
         return torch.stack(outs, dim=1).contiguous()
 
     def route(self, x_flat: torch.Tensor, mark=None):
         """(gates [n, H, k] x.dtype, expert ids [n, H, k] int32).  `mark(stage)`, if given,
         is called after each stage is enqueued (used to place timing events)."""
-        if self._bn_uses_batch_stats():
-            self._train_pass += 1
-            packed = self._packed_weights(x_flat.dtype, x_flat.device)
-        else:
-            packed = self._packed(x_flat.dtype, x_flat.device)
-        k1, k2 = packed[2:4]
-        q = self.queries(x_flat, packed)
+        batch = self._bn_uses_batch_stats()
+        w = self._pass_weights(x_flat, batch)
+        q = self._batch_queries(x_flat, w) if batch else self._eval_queries(x_flat, w)
         if mark is not None:
             mark("query_proj")
-        out = hip.route_topk(q, k1, k2, self.top_k, key_norms=self._key_norms, prepared_keys=self._keys_prepared)
+        out = hip.route_topk(q, w.k1, w.k2, self.top_k, key_norms=w.key_norms, prepared_keys=w.keys_prepared)
         if mark is not None:
             mark("route")
         return out
@@ -550,8 +571,7 @@ class EthosExpertLayer(nn.Module):
         self.generation_network = ExpertGenerationNetwork(config.d_latent, config.d_model,
                                                           config.d_intermediate_hypernet)
         self.router = ProductKeyRouter(config)
-        self._gen_made = _Made()
-        self._gen = None
+        self._kept_gen = _Kept()
 
     def _param_sources(self) -> list:
         """Every tensor a forward reads (router parameters and BatchNorm buffers, latents and
@@ -565,7 +585,7 @@ class EthosExpertLayer(nn.Module):
     def packed_tensors(self) -> list:
         """The packed forms that the last evaluation read."""
         r = self.router
-        return [t for t in (*r._cache, *r._bn, r._key_norms, r._keys_prepared, r._wq_prepared, *self._gen) if t is not None]
+        return [t for kept in (r._kept_weights, r._kept_bn, self._kept_gen) for t in kept.value or () if t is not None]
 
     def _generator_params(self, dtype, device, mode: int | None = None):
         """(latents, W1, W2, W_u^T): the generator weights in the layer dtype on the device,
@@ -574,16 +594,17 @@ class EthosExpertLayer(nn.Module):
         ps = (self.expert_latents.weight, self.generation_network.net[0].weight, self.generation_network.net[2].weight)
         mode = self._modules["router"]._pack_mode() if mode is None else mode
         key = (dtype, device, mode, tuple((p.data_ptr(), p._version) for p in ps))
-        if not self._gen_made.fits(key):
+        gen = self._kept_gen.get(key)
+        if gen is None:
             with _packing():
                 if all(p.dtype == dtype and p.device == device and p.is_contiguous() for p in ps):
                     gen = tuple(p.detach() for p in ps)
                 else:
                     gen = tuple(p.detach().to(device=device, dtype=dtype).contiguous() for p in ps)
                 wut = gen[2][: self.d_model].t().contiguous() if dtype == torch.bfloat16 else None
-            self._gen = gen + (wut,)
-            self._gen_made.set(key, [t for t in self._gen if all(t is None or t.data_ptr() != p.data_ptr() for p in ps)], mode > 0)
-        return self._gen
+            own = [t for t in gen if all(t.data_ptr() != p.data_ptr() for p in ps)]
+            gen = self._kept_gen.put(key, gen + (wut,), own + [wut], mode > 0)
+        return gen
 
     def _expert_stages(self, x_flat: torch.Tensor, gates: torch.Tensor, seg: dict, xp: torch.Tensor | None = None):
         """(out, h): generation over the unique experts, activations and scatter-back in the
@@ -621,9 +642,10 @@ class EthosExpertLayer(nn.Module):
         router = self._modules["router"]
         if mark is None and side_stream is None and x_flat.shape[0] > 0 and not router._bn_uses_batch_stats():
             with torch.no_grad():
-                packed = router._packed(x_flat.dtype, x_flat.device)
+                w = router._packed_weights(x_flat.dtype, x_flat.device, 0)
+                packed = w[:4] + tuple(router._bn_coefficients(x_flat.device))
                 gen = self._generator_params(x_flat.dtype, x_flat.device, 0)
-                return hip.layer_forward(x_flat, packed, router._key_norms, router._keys_prepared, router._wq_prepared, gen,
+                return hip.layer_forward(x_flat, packed, w.key_norms, w.keys_prepared, w.wq_prepared, gen,
                                          self.num_experts, self.top_k, self.hidden_space)
         with torch.no_grad():
             xp = None

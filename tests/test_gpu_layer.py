@@ -372,3 +372,29 @@ def test_packing_inside_a_capture_serves_only_the_graph():
             assert torch.equal(out, want)
             assert torch.equal(m.forward_flat(x), want)
         assert torch.equal(copy.deepcopy(m)(x[None])[0], want)
+
+
+def test_first_calls_of_several_threads():
+    """Threads that call a layer for the first time at once, each on a stream of its own: every one
+    reads packed parameters that it made or waited for, whichever set is kept in the end."""
+    import threading
+    x, (_, ref) = _two_layers("cfg3")
+    with torch.no_grad():
+        want = ref.forward_flat(x)
+    for _ in range(5):
+        _, (m, _) = _two_layers("cfg3")
+        torch.cuda.synchronize()
+        start, got = threading.Barrier(4), [None] * 4
+
+        def call(i):
+            with torch.no_grad(), torch.cuda.stream(torch.cuda.Stream()):
+                start.wait()
+                got[i] = m.forward_flat(x)
+                torch.cuda.current_stream().synchronize()
+
+        ts = [threading.Thread(target=call, args=(i,)) for i in range(4)]
+        for t in ts:
+            t.start()
+        for t in ts:
+            t.join()
+        assert all(torch.equal(y, want) for y in got)
