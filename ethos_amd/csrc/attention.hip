@@ -20,6 +20,11 @@
 // library's fused attention on values padded to 128 columns and about 110 us of torch operations
 // that rotated, padded and laid out its operands; the same error against float64 (2.0e-3).
 // 1 x 1,024 tokens (workgroups of 64 queries): 32 us against 54.
+//
+// The running maximum's scaled form is a product rounded by itself, also where it is subtracted:
+// fused multiply-adds are written out.
+#pragma clang fp contract(off)
+
 #include "ethos_common.hpp"
 #include "ethos_launch.hpp"
 #include "ethos_mfma.hpp"
@@ -151,7 +156,9 @@ __global__ __launch_bounds__(WAVES * 64, 2) void mla_attention_kernel(const uint
     };
 
     f32x16_t o[2] = {f32x16_zero(), f32x16_zero()};
-    float m = -INFINITY, l = 0.0f;
+    // the running maximum (from a finite start: scores that have overflowed to -inf weigh nothing,
+    // rather than NaN) and its scaled, rounded form, which every exponential is relative to
+    float m = -0x1p126f, shift = m * scale2, l = 0.0f;
     const int q_last = q0 + 32 * WAVES - 1 < n ? q0 + 32 * WAVES - 1 : n - 1;
     load(0);
     for (int key0 = 0; key0 <= q_last; key0 += kKeys) {
@@ -182,10 +189,9 @@ __global__ __launch_bounds__(WAVES * 64, 2) void mla_attention_kernel(const uint
 #pragma unroll
                 for (int i = 0; i < 16; ++i) top = fmaxf(top, s[k][i]);
             top = fmaxf(top, __shfl_xor(top, 32, 64));
-            const float m1 = fmaxf(m, top);
-            const float shift = m1 * scale2;
-            const float r = __builtin_amdgcn_exp2f(__builtin_fmaf(m, scale2, -shift));
-            m = m1;
+            m = fmaxf(m, top);
+            const float r = __builtin_amdgcn_exp2f(shift - m * scale2);
+            shift = m * scale2;
             l *= r;
 #pragma unroll
             for (int k = 0; k < 2; ++k)

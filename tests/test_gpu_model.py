@@ -187,6 +187,49 @@ def test_mla_attention_against_float64(b, n, H):
     assert err < 4e-3, err
 
 
+def test_mla_attention_large_scores():
+    """Scores near 10^8, whole multiples of 2^7 (so that float32 sums hold them exactly): the weights
+    of earlier keys stay as they are while the maximum does, however large its rounding."""
+    from ethos_amd import hip
+    n, H = 500, 1
+    g = torch.Generator(device="cuda").manual_seed(2)
+    q, kv, k_rot = (torch.zeros(1, n, w, device="cuda").bfloat16() for w in (128, 128, 64))
+    q[..., 0], q[..., 1] = 2.0 ** 14, 128.0
+    kv[..., 0] = 8191.0 // 64 * 64
+    kv[..., 1] = torch.randint(0, 2, (1, n), generator=g, device="cuda").bfloat16()
+    kv[..., 64:] = torch.randn(1, n, 64, generator=g, device="cuda").bfloat16()
+    rates = torch.ones(32, device="cuda")
+    pos, scale = torch.arange(n, device="cuda"), 0.0313
+    o = hip.mla_attention(q, kv, k_rot, pos, rates, H, 64, 64, 64, scale)
+    s = (kv[0, :, 1].double() * 128 * scale).expand(n, n).masked_fill(torch.ones(n, n, dtype=torch.bool, device="cuda").triu(1), float("-inf"))
+    ref = torch.softmax(s, -1) @ kv[0, :, 64:].double()
+    # every exponential is relative to one rounded maximum, which cancels: the bound of the other sizes
+    err = float((o[0].double() - ref).norm() / ref.norm())
+    assert err < 4e-3, err
+
+
+def test_mla_attention_scores_that_overflow():
+    """Scores of the first 64 keys overflow to -inf (products of finite values): queries that also
+    see later keys weigh those alone, as a softmax over all scores does; the others have no finite
+    score and are NaN."""
+    import math
+
+    from ethos_amd import hip
+    g = torch.Generator(device="cuda").manual_seed(1)
+    n, H = 200, 2
+    q, kv, k_rot = (torch.randn(1, n, w, generator=g, device="cuda").bfloat16() for w in (H * 128, H * 128, 64))
+    q.view(1, n, H, 128)[..., 0] = 3e38
+    kv.view(1, n, H, 128)[..., 0] = 0.0
+    kv.view(1, n, H, 128)[:, :64, :, 0] = -3e38
+    rates = 1.0 / 10000.0 ** (torch.arange(0, 64, 2, device="cuda", dtype=torch.float32) / 64)
+    pos, scale = torch.arange(n, device="cuda"), 1.0 / math.sqrt(128)
+    o = hip.mla_attention(q, kv, k_rot, pos, rates, H, 64, 64, 64, scale)
+    ref = _attention_double(q, kv, k_rot, pos, rates, H, scale)
+    assert torch.isnan(o[:, :64]).all()
+    err = float((o[:, 64:].double() - ref[:, 64:]).norm() / ref[:, 64:].norm())
+    assert err < 4e-3, err
+
+
 @pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("rows,d,ld", [(1, 8, 8), (5, 72, 80), (33, 768, 1088), (4, 1000, 1000), (3, 2048, 2056)])
 def test_rms_norm_against_float64(dt, rows, d, ld):
