@@ -6,8 +6,12 @@
 // nine.  The sums are float32, as in a float32 GEMM; the bf16 MFMAs run at 16 times the float32
 // MFMAs' rate, so three of them cost a fifth of one float32 product and nine a little over half.
 // Six of the nine (down to 2^-16 of the result) leave out up to 2^-22 of a product that a float32
-// multiply-add keeps; all nine cost the float32 layer of 256 tokens 114.9 us against 113.3, and
-// a training step of 500 tokens nothing that shows.  A sum with an infinity in it comes out as NaN
+// multiply-add keeps; all nine cost the float32 layer of 256 tokens 116 us against 113, and a
+// training step of 500 tokens nothing that shows.  Tiles of 64 sum the products of the upper planes
+// by themselves and add the others at the end: one rounding of the whole sum per 16 terms instead
+// of nine (or three), which halves the error against float64 (float32 layer 2.3e-7 -> 1.3e-7, its
+// gradients about 1.3e-6 -> 0.55e-6, library float32 products 2.5e-7 and 1.5e-6) at the same time;
+// in tiles of 128 the second sums would halve the workgroups a CU holds.  A sum with an infinity in it comes out as NaN
 // and is taken again as a float32 chain (the step of 4,096 tokens with one infinite output gradient,
 // whose gradients are then NaN nearly everywhere: 2.3 -> 3.3 ms).
 //
@@ -260,7 +264,9 @@ __global__ __launch_bounds__(kGemmThreads, (BM > 64 ? (sizeof(TB) == 4 ? 3 : 4) 
     const GemmRange range = gemm_range(p, part_id);
     const int64_t m = range.m, kb = range.kb, ke = range.ke;
     if (group >= gg.groups || m0 >= m) return;
-    f32x16_t acc[MI][NI];
+    // sums of the products of upper planes, and (kApart) of the others, added at the end
+    constexpr bool kApart = PA + PB > 2 && MI * NI == 1;
+    f32x16_t acc[MI][NI], low = f32x16_zero();
 #pragma unroll
     for (int i = 0; i < MI; ++i)
 #pragma unroll
@@ -310,8 +316,10 @@ __global__ __launch_bounds__(kGemmThreads, (BM > 64 ? (sizeof(TB) == 4 ? 3 : 4) 
 #pragma unroll
                         for (int i = 0; i < MI; ++i)
 #pragma unroll
-                            for (int j = 0; j < NI; ++j)
-                                acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[i][qa], fb[j][qb], acc[i][j], 0, 0, 0);
+                            for (int j = 0; j < NI; ++j) {
+                                f32x16_t& to = kApart && q > 0 ? low : acc[i][j];
+                                to = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[i][qa], fb[j][qb], to, 0, 0, 0);
+                            }
                     }
                 }
             }
@@ -319,6 +327,7 @@ __global__ __launch_bounds__(kGemmThreads, (BM > 64 ? (sizeof(TB) == 4 ? 3 : 4) 
         }
     }
 
+    if constexpr (kApart) acc[0][0] += low;
     float* part = p.split > 1 ? p.part + (size_t)part_id * (size_t)p.m * (size_t)p.n : nullptr;
     auto emit = [&](int64_t mm, int n, float v, float bias, float aux) {
         if (part) {
